@@ -2620,10 +2620,10 @@ int mg_build_static(lsamd_fd_system* s, Mg* m, hipStream_t st) {
       break;
     const lsamd_grid gc = mg_coarse_grid(gprev);
     lsamd_fd_reg rc_reg = s->reg;
-    const double sc = ldexp(1.0, -l);
-    for (double* f : {&rc_reg.w2_xx, &rc_reg.w2_yy, &rc_reg.w2_zz, &rc_reg.w2_xy, &rc_reg.w2_xz,
-                      &rc_reg.w2_yz, &rc_reg.w2_bx, &rc_reg.w2_by, &rc_reg.w2_bz, &rc_reg.ridge2})
-      *f *= sc;
+    // weights of the re-discretised regulariser: interior rows as on the fine
+    // level, border rows quartered per level (see the note in mg.hpp)
+    for (double* f : {&rc_reg.w2_bx, &rc_reg.w2_by, &rc_reg.w2_bz}) *f *= ldexp(1.0, -2 * l);
+    rc_reg.ridge2 *= ldexp(1.0, -l);
     lsamd_fd_system* cs = nullptr;
     if (int rc = lsamd_fd_system_create(&gc, &rc_reg, nullptr, &cs)) return rc;
     MgLevel L;
