@@ -3829,11 +3829,7 @@ void mr_apply(lsamd_fd_system* s, MrWork* w, int l, const float* x, float* y, hi
     }
     return;
   }
-  if (L.n >= kMrNodeThreads)
-    hipLaunchKernelGGL(k_mr_apply_coarse_all<R>, dim3((unsigned)ceil_div(L.n, 256)), b256, 0, st,
-                       mg_dev(L), x, y, ad);
-  else
-    hipLaunchKernelGGL(k_mr_apply_coarse, nb, b256, 0, st, mg_dev(L), x, y, R, ad);
+  hipLaunchKernelGGL(k_mr_apply_coarse, nb, b256, 0, st, mg_dev(L), x, y, ad);
 }
 
 // lanes per thread of the covered-node smoothing step (LSAMD_MR_COV_LANES:
@@ -4103,16 +4099,18 @@ int mr_solve_group(lsamd_fd_system* s, MrWork* w, const lsamd_solve_opts* o, int
 }  // namespace
 
 // Several right-hand sides of the system's normal equations; multigrid with
-// all lanes per launch when every level has a class table, else one
-// multigrid solve per right-hand side.
+// all lanes per launch when the fine level has a class table, else one
+// multigrid solve per right-hand side.  (Until the coarse levels were freed
+// of that condition, 24 lanes on 38 x 56 x 43 nodes took 1.49 s, one solve
+// after the other.)
 int mr_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, int nrhs, const double* rhs,
              double* c, lsamd_solve_info* infos, hipStream_t st) {
   if (s->op != 0) return fail(LSAMD_ERR_ARG, "multi-rhs multigrid: FD systems only");
   if (int rc = mg_ensure(s, st)) return rc;
   if (int rc = mr_sell_ensure(s, st)) return rc;
-  const Mg* m = s->mg;
-  bool lanes = s->regular && s->tab32 && s->tab64;
-  for (size_t l = 1; l + 1 < m->lv.size(); ++l) lanes = lanes && m->lv[l].sys->regular;
+  // coarse levels without a class table (an axis under 7 nodes, as most ragged
+  // grids reach before the coarsest) apply their regulariser node by node
+  const bool lanes = s->regular && s->tab32 && s->tab64;
   const int64_t n = s->n;
   if (!lanes) {
     for (int r = 0; r < nrhs; ++r)

@@ -16,8 +16,8 @@
 
 namespace lsamd {
 
-// levels with at least this many nodes apply their coarse operator one
-// thread per node for all lanes (fewer, per-lane threads below)
+// levels with at least this many nodes stream their transfers along z (the
+// smaller ones lack the work items and keep one thread per node)
 constexpr int64_t kMrNodeThreads = 1 << 17;
 
 // per right-hand side
@@ -39,36 +39,6 @@ __global__ void k_mr_pack(const double* __restrict__ in, int nr, int R, int64_t 
 // Every kernel of the V-cycle runs one thread per (lane, node), the lane in
 // blockIdx.y: the loads of one lane are coalesced and the small levels still
 // get R times the threads of a single solve.
-
-// y = R x (class-table regulariser, ridge included)
-template <typename T>
-__global__ __launch_bounds__(256) void k_mr_stencil(const T* __restrict__ x, T* __restrict__ y,
-                                                    GridDev g, const T* __restrict__ tab, int R,
-                                                    const int* __restrict__ all_done) {
-  if (*all_done) return;
-  const int64_t n = (int64_t)g.nx * g.ny * g.nz;
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= n) return;
-  const int64_t r = blockIdx.y;
-  const T* xs = x + r * n;
-  const int nx = g.nx, ny = g.ny, nz = g.nz;
-  const int64_t nxy = (int64_t)nx * ny;
-  const int k = (int)(id / nxy);
-  const int64_t rr = id - (int64_t)k * nxy;
-  const int j = (int)(rr / nx);
-  const int i = (int)(rr - (int64_t)j * nx);
-  const T* c = tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
-  T acc = c[0] * xs[id];
-#pragma unroll
-  for (int t = 1; t < kTaps; ++t) {
-    const int dx = kBTap[t][0], dy = kBTap[t][1], dz = kBTap[t][2];
-    const bool ok = (unsigned)(i + dx) < (unsigned)nx && (unsigned)(j + dy) < (unsigned)ny &&
-                    (unsigned)(k + dz) < (unsigned)nz;
-    const T xv = xs[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
-    acc += c[t] * (ok ? xv : (T)0);
-  }
-  y[r * n + id] = acc;
-}
 
 // t[r nrows + row] = w_r^2 (a_r . x_r)
 template <typename T>
@@ -131,57 +101,16 @@ __global__ __launch_bounds__(256) void k_mr_rows_scatter(RowsDev Rw, const T* __
   y[r * n + Rw.dnode[d]] += acc;
 }
 
-// coarse level: y = (class-table regulariser + Gram) x
+// coarse level without a class table (an axis under 7 nodes):
+// y = (regulariser + Gram) x, one thread per node and lane
 __global__ __launch_bounds__(256) void k_mr_apply_coarse(MgDev L, const float* __restrict__ x,
-                                                         float* __restrict__ y, int R,
+                                                         float* __restrict__ y,
                                                          const int* __restrict__ all_done) {
   if (*all_done) return;
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= L.n) return;
   const int64_t r = blockIdx.y;
   y[r * L.n + id] = mg_apply_node(L, x + r * L.n, id);
-}
-
-// coarse level, one thread per node and all lanes (large coarse levels: the
-// class row and the Gram row are read once for the R lanes)
-template <int R>
-__global__ __launch_bounds__(256) void k_mr_apply_coarse_all(MgDev L,
-                                                             const float* __restrict__ x,
-                                                             float* __restrict__ y,
-                                                             const int* __restrict__ all_done) {
-  if (*all_done) return;
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= L.n) return;
-  const int64_t n = L.n;
-  int i, j, k;
-  mg_ijk(id, L.g.nx, L.g.ny, i, j, k);
-  const int nx = L.g.nx, ny = L.g.ny, nz = L.g.nz;
-  const int64_t nxy = (int64_t)nx * ny;
-  const float* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
-  float acc[R];
-  const float c0 = c[0];
-#pragma unroll
-  for (int r = 0; r < R; ++r) acc[r] = c0 * x[r * n + id];
-#pragma unroll
-  for (int t = 1; t < kTaps; ++t) {
-    const int dx = kBTap[t][0], dy = kBTap[t][1], dz = kBTap[t][2];
-    const bool ok = (unsigned)(i + dx) < (unsigned)nx && (unsigned)(j + dy) < (unsigned)ny &&
-                    (unsigned)(k + dz) < (unsigned)nz;
-    if (!ok) continue;
-    const int64_t o = id + dx + (int64_t)nx * dy + nxy * dz;
-    const float ct = c[t];
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] += ct * x[r * n + o];
-  }
-  if (L.gptr)
-    for (int64_t e = L.gptr[id]; e < L.gptr[id + 1]; ++e) {
-      const float a = L.gval[e];
-      const int64_t o = L.gcol[e];
-#pragma unroll
-      for (int r = 0; r < R; ++r) acc[r] += a * x[r * n + o];
-    }
-#pragma unroll
-  for (int r = 0; r < R; ++r) y[r * n + id] = acc[r];
 }
 
 // y += G x for the lanes of a coarse level (G its Gram rows), LG lanes per

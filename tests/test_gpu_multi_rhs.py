@@ -137,3 +137,26 @@ def test_multi_rhs_work_rebuilt_after_a_failed_allocation(monkeypatch):
     for r in range(5):
         c1, _ = s.solve(rtol=1e-12, rhs=rhs[r], multigrid=True, check_every=8)
         assert float(torch.linalg.vector_norm(c[r] - c1) / torch.linalg.vector_norm(c1)) <= 1e-9
+
+
+@pytest.mark.parametrize("nodes,nreal", [((38, 56, 43), 6), ((7, 30, 9), 9), ((33, 8, 20), 4)])
+def test_ragged_grids_match_single_solves(nodes, nreal):
+    """Grids whose coarse levels fall under 7 nodes on an axis (no class
+    table there) still take the lanes."""
+    from loopstructural_amd import _lib, synthetic
+    from loopstructural_amd import fd_system as fs
+
+    g = _lib.make_grid((0, 0, 0), tuple(1.0 / (k - 1) for k in nodes), nodes)
+    n = int(np.prod(nodes))
+    values, normals = synthetic.constraints(150, 40, 5)
+    reals = [synthetic.perturb(values, normals, 300 + r) for r in range(nreal)]
+    s = fs.FdSystem(g, fs.reg_struct(W, nodes, 1e-8))
+    s.set_rows(_rows(fs, _lib, g, n, *reals[0]))
+    rhs = torch.stack([s.rhs_for(_rows(fs, _lib, g, n, v, m).b) for v, m in reals])
+    c, infos = s.solve_multi(rhs, rtol=1e-12)
+    for r in range(nreal):
+        one, _ = s.solve(rtol=1e-12, multigrid=True, rhs=rhs[r])
+        assert infos[r]["converged"]
+        err = float(torch.linalg.vector_norm(c[r] - one) / torch.linalg.vector_norm(one))
+        assert err <= 1e-8, (nodes, r, err)
+    s.close()
