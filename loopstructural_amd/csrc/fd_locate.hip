@@ -15,6 +15,7 @@
 
 #include <math.h>
 
+#include "exact_div.hpp"
 #include "lsamd_common.hpp"
 
 namespace lsamd {
@@ -334,53 +335,160 @@ __global__ void k_build_rows(GridDev g, int kind, double* __restrict__ pts, int6
   emit_row(n + i, id, c2, b1, wscale, l1, cols, coef, b, w, norm);
 }
 
-__global__ void k_evaluate(GridDev g, const double* __restrict__ c, const double* __restrict__ pts,
-                           int64_t n, double* __restrict__ vals, double* __restrict__ grads) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double px = pts[3 * i], py = pts[3 * i + 1], pz = pts[3 * i + 2];
+// values[i] and gradient of one point from its located cell and the cell's
+// corner coefficients, as numpy evaluates them
+__device__ inline void eval_point(const GridDev& g, const double* __restrict__ c, double px,
+                                  double py, double pz, double* val, double* gr) {
   const Located L = locate(g, px, py, pz);
+  *val = isnan(px) || isnan(py) || isnan(pz) ? 0.0 : __builtin_nan("");
+  gr[0] = gr[1] = gr[2] = 0.0;
+  if (!L.inside) return;
   int64_t id[8];
   corner_ids(g, L, id);
-  double cv[8];
-  if (L.inside) {
+  double a[8], T[24];
+  trilinear(L.lx, L.ly, L.lz, a);
+  shape_grad(L.lx, L.ly, L.lz, L.hx, L.hy, L.hz, T);
 #pragma unroll
-    for (int k = 0; k < 8; ++k) cv[k] = c[id[k]];
+  for (int k = 0; k < 8; ++k) {
+    const double cv = c[id[k]];
+    a[k] *= cv;
+    T[k] *= cv;
+    T[8 + k] *= cv;
+    T[16 + k] *= cv;
   }
-  if (vals) {
-    double out;
-    if (isnan(px) || isnan(py) || isnan(pz)) {
-      out = 0.0;
-    } else if (!L.inside) {
-      out = __builtin_nan("");
-    } else {
-      double a[8];
-      trilinear(L.lx, L.ly, L.lz, a);
+  *val = sum8(a);
+  gr[0] = sum8(T);
+  gr[1] = sum8(T + 8);
+  gr[2] = sum8(T + 16);
+}
+
+// What an evaluation on a uniform grid computes once: the bounds of the
+// inside test and the rounded reciprocal of each step.
+struct EvalGrid {
+  double lo[3], hi[3], y[3];
+};
+
+inline EvalGrid to_eval(const lsamd_grid& g) {
+  EvalGrid e;
+  for (int a = 0; a < 3; ++a) {
+    const double o = g.origin[a], mx = o + (double)(g.nnodes[a] - 1) * g.step[a];
+    double ext = fabs(mx - o);
+    ext = ext > 1.0 ? ext : 1.0;
+    e.lo[a] = o - kEps32 * ext;
+    e.hi[a] = mx + kEps32 * ext;
+    e.y[a] = 1.0 / g.step[a];
+  }
+  return e;
+}
+
+typedef double pair_t __attribute__((ext_vector_type(2), aligned(8)));
+
+// eval_point on a uniform grid whose steps are known divisors, bit for bit
+// the same: the steps' reciprocals replace the divisions (div_known), and the
+// 24 gradient weights come from the 12 that differ in more than their sign
+// (1 - y is -(y - 1) exactly, and a product's sign does not change its
+// rounding).  False where a dividend is out of range (the caller takes
+// eval_point); cells past int32 node ids stay with 64-bit offsets.
+__device__ inline bool eval_point_known(const GridDev& g, const EvalGrid& e,
+                                        const double* __restrict__ c, double px, double py,
+                                        double pz, double* val, double* gr) {
+  *val = isnan(px) || isnan(py) || isnan(pz) ? 0.0 : __builtin_nan("");
+  gr[0] = gr[1] = gr[2] = 0.0;
+  if (!(px >= e.lo[0] && px <= e.hi[0] && py >= e.lo[1] && py <= e.hi[1] && pz >= e.lo[2] &&
+        pz <= e.hi[2]))
+    return true;
+  auto cell = [](double d, double h, double y, int nn) {
+    const int k = (int)floor(div_known(d, h, y));
+    return k < 0 ? 0 : (k > nn - 2 ? nn - 2 : k);
+  };
+  const double dx = px - g.ox, dy = py - g.oy, dz = pz - g.oz;
+  bool ok = div_known_dividend(dx) && div_known_dividend(dy) && div_known_dividend(dz);
+  const int cx = cell(dx, g.hx, e.y[0], g.nx);
+  const int cy = cell(dy, g.hy, e.y[1], g.ny);
+  const int cz = cell(dz, g.hz, e.y[2], g.nz);
+  const int64_t nx = g.nx, nxy = nx * g.ny;
+  const double* c0 = c + cx + nx * cy + nxy * cz;
+  const pair_t c01 = *(const pair_t*)c0, c23 = *(const pair_t*)(c0 + nx);
+  const pair_t c45 = *(const pair_t*)(c0 + nxy), c67 = *(const pair_t*)(c0 + nxy + nx);
+  const double ax = px - (g.ox + g.hx * (double)cx), ay = py - (g.oy + g.hy * (double)cy);
+  const double az = pz - (g.oz + g.hz * (double)cz);
+  ok = ok && div_known_dividend(ax) && div_known_dividend(ay) && div_known_dividend(az);
+  const double x = clip01(div_known(ax, g.hx, e.y[0]));
+  const double y = clip01(div_known(ay, g.hy, e.y[1]));
+  const double z = clip01(div_known(az, g.hz, e.y[2]));
+  const double x1 = 1 - x, y1 = 1 - y, z1 = 1 - z;
+  // products of two factors, shared by the weights and the gradients
+  const double yz00 = y1 * z1, yz10 = y * z1, yz01 = y1 * z, yz11 = y * z;
+  const double xz00 = x1 * z1, xz10 = x * z1, xz01 = x1 * z, xz11 = x * z;
+  const double xy00 = x1 * y1, xy10 = x * y1, xy01 = x1 * y, xy11 = x * y;
+  for (const double d : {yz00, yz10, yz01, yz11, xz00, xz10, xz01, xz11, xy00, xy10, xy01, xy11})
+    ok = ok && div_known_dividend(d);
+  if (!ok) return false;
+  const double cv[8] = {c01.x, c01.y, c23.x, c23.y, c45.x, c45.y, c67.x, c67.y};
+  const double w[8] = {xy00 * z1, xy10 * z1, xy01 * z1, xy11 * z1,
+                       xy00 * z,  xy10 * z,  xy01 * z,  xy11 * z};
+  double a[8];
 #pragma unroll
-      for (int k = 0; k < 8; ++k) a[k] *= cv[k];
-      out = sum8(a);
-    }
-    vals[i] = out;
-  }
-  if (grads) {
-    double gx = 0.0, gy = 0.0, gz = 0.0;
-    if (L.inside) {
-      double T[24];
-      shape_grad(L.lx, L.ly, L.lz, L.hx, L.hy, L.hz, T);
+  for (int k = 0; k < 8; ++k) a[k] = w[k] * cv[k];
+  *val = sum8(a);
+  // gradient weights of the corner pairs along each axis
+  const double p0 = div_known(yz00, g.hx, e.y[0]), p1 = div_known(yz10, g.hx, e.y[0]);
+  const double p2 = div_known(yz01, g.hx, e.y[0]), p3 = div_known(yz11, g.hx, e.y[0]);
+  const double tx[8] = {-p0 * cv[0], p0 * cv[1], -p1 * cv[2], p1 * cv[3],
+                        -p2 * cv[4], p2 * cv[5], -p3 * cv[6], p3 * cv[7]};
+  gr[0] = sum8(tx);
+  const double q0 = div_known(xz00, g.hy, e.y[1]), q1 = div_known(xz10, g.hy, e.y[1]);
+  const double q2 = div_known(xz01, g.hy, e.y[1]), q3 = div_known(xz11, g.hy, e.y[1]);
+  const double ty[8] = {-q0 * cv[0], -q1 * cv[1], q0 * cv[2], q1 * cv[3],
+                        -q2 * cv[4], -q3 * cv[5], q2 * cv[6], q3 * cv[7]};
+  gr[1] = sum8(ty);
+  const double r0 = div_known(xy00, g.hz, e.y[2]), r1 = div_known(xy10, g.hz, e.y[2]);
+  const double r2 = div_known(xy01, g.hz, e.y[2]), r3 = div_known(xy11, g.hz, e.y[2]);
+  const double tz[8] = {-r0 * cv[0], -r1 * cv[1], -r2 * cv[2], -r3 * cv[3],
+                        r0 * cv[4],  r1 * cv[5],  r2 * cv[6],  r3 * cv[7]};
+  gr[2] = sum8(tz);
+  return true;
+}
+
+// Values and gradients at n points.  A workgroup's points come in, and its
+// gradients leave, through LDS in whole lines (a thread's own three doubles
+// lie 24 bytes from its neighbour's); they are streamed past the caches, whose
+// room belongs to c.  KNOWN: uniform grid with steps that div_known takes.
+constexpr int kEvalBlock = 256;
+template <bool KNOWN>
+__global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
+                                                         const double* __restrict__ c,
+                                                         const double* __restrict__ pts,
+                                                         int64_t n, double* __restrict__ vals,
+                                                         double* __restrict__ grads) {
+  __shared__ double sh[3 * kEvalBlock];
+  const int t = threadIdx.x;
+  const int64_t b = (int64_t)blockIdx.x * kEvalBlock;
+  const int m = (int)(n - b < kEvalBlock ? n - b : kEvalBlock);
 #pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        T[k] *= cv[k];
-        T[8 + k] *= cv[k];
-        T[16 + k] *= cv[k];
-      }
-      gx = sum8(T);
-      gy = sum8(T + 8);
-      gz = sum8(T + 16);
-    }
-    grads[3 * i] = gx;
-    grads[3 * i + 1] = gy;
-    grads[3 * i + 2] = gz;
+  for (int k = 0; k < 3; ++k)
+    if (t + k * kEvalBlock < 3 * m)
+      sh[t + k * kEvalBlock] = __builtin_nontemporal_load(pts + 3 * b + t + k * kEvalBlock);
+  __syncthreads();
+  double val = 0.0, gr[3] = {0.0, 0.0, 0.0};
+  if (t < m) {
+    const double px = sh[3 * t], py = sh[3 * t + 1], pz = sh[3 * t + 2];
+    if (!KNOWN || !eval_point_known(g, e, c, px, py, pz, &val, gr))
+      eval_point(g, c, px, py, pz, &val, gr);
+    if (vals) __builtin_nontemporal_store(val, vals + b + t);
   }
+  if (!grads) return;
+  // a thread overwrites only the three entries that it alone has read
+  if (t < m) {
+    sh[3 * t] = gr[0];
+    sh[3 * t + 1] = gr[1];
+    sh[3 * t + 2] = gr[2];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (t + k * kEvalBlock < 3 * m)
+      __builtin_nontemporal_store(sh[t + k * kEvalBlock], grads + 3 * b + t + k * kEvalBlock);
 }
 
 // numpy's pairwise summation of a contiguous run of n <= 128 doubles
@@ -512,9 +620,15 @@ extern "C" int lsamd_fd_evaluate(const lsamd_grid* g, const double* c, const dou
   if (n < 0) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate: n < 0");
   if (n == 0) return LSAMD_OK;
   if (!c || !pts) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate: NULL input");
-  const int bs = 256;
-  hipLaunchKernelGGL(k_evaluate, dim3((unsigned)ceil_div(n, bs)), dim3(bs), 0,
-                     (hipStream_t)stream, to_dev(*g), c, pts, n, values, grads);
+  const dim3 nb((unsigned)ceil_div(n, kEvalBlock)), bs(kEvalBlock);
+  const EvalGrid e = to_eval(*g);
+  if (!g->axis_nodes[0] && div_known_divisor(g->step[0]) && div_known_divisor(g->step[1]) &&
+      div_known_divisor(g->step[2]))
+    hipLaunchKernelGGL(k_evaluate<true>, nb, bs, 0, (hipStream_t)stream, to_dev(*g), e, c, pts, n,
+                       values, grads);
+  else
+    hipLaunchKernelGGL(k_evaluate<false>, nb, bs, 0, (hipStream_t)stream, to_dev(*g), e, c, pts,
+                       n, values, grads);
   LSAMD_CHECK_LAUNCH("k_evaluate");
   return LSAMD_OK;
 }

@@ -39,9 +39,67 @@ struct TetLoc {
   double bc[4];
 };
 
+// barycentric coordinates of p in tet t of a cell, by scalar triple products
+// as the reference forms them.
+// KNOWN: the divisions by 6 and by v through their reciprocals (div_known),
+// falling back where a dividend or v leaves its range.
+template <bool KNOWN>
+__device__ inline void p1_barycentric(const P1Mesh& m, const int* cell, int t, const double* p,
+                                      double* bc) {
+  double V[4][3];
+  tet_vertices(m, cell, t, V);
+  double vap[3], vbp[3], vab[3], vac[3], vad[3], vbc[3], vbd[3], cr[3];
+  for (int a = 0; a < 3; ++a) {
+    vap[a] = p[a] - V[0][a];
+    vbp[a] = p[a] - V[1][a];
+    vab[a] = V[1][a] - V[0][a];
+    vac[a] = V[2][a] - V[0][a];
+    vad[a] = V[3][a] - V[0][a];
+    vbc[a] = V[2][a] - V[1][a];
+    vbd[a] = V[3][a] - V[1][a];
+  }
+  double num[4], den;
+  cross3(vbd, vbc, cr);
+  num[0] = dot3(vbp, cr);
+  cross3(vac, vad, cr);
+  num[1] = dot3(vap, cr);
+  den = dot3(vab, cr);
+  cross3(vad, vab, cr);
+  num[2] = dot3(vap, cr);
+  cross3(vab, vac, cr);
+  num[3] = dot3(vap, cr);
+  if constexpr (KNOWN) {
+    const double v = div_known(den, 6.0, 1.0 / 6.0), av = fabs(v);
+    bool ok = div_known_dividend(den) && div_known_divisor(av);
+    double s[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      ok = ok && div_known_dividend(num[k]);
+      s[k] = div_known(num[k], 6.0, 1.0 / 6.0);
+      ok = ok && div_known_dividend(s[k]);
+    }
+    if (ok) {
+      const double y = 1.0 / v;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) bc[k] = div_known(s[k], v, y);
+      return;
+    }
+  }
+  const double v = den / 6.0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) bc[k] = (num[k] / 6.0) / v;
+}
+
 // get_element_for_location for one point: strict box test, cell lookup,
-// barycentric coordinates by scalar triple products in all 5 tets, the last
-// tet with all coordinates >= 0 wins.
+// barycentric coordinates in the tets, the last tet with all coordinates
+// >= 0 wins.
+//
+// Coordinates of all five tets (nine divisions and a hundred other FP64
+// operations each) bound evaluation by arithmetic, not memory, so with
+// m.slack > 0 only the tets are computed that can pass: the cell's local coordinates give
+// every tet's smallest barycentric coordinate up to a rounding error far
+// below m.slack (see p1_slack), and a tet below -m.slack fails the exact test
+// for certain.  Almost every point has one such tet.
 __device__ TetLoc p1_locate(const P1Mesh& m, const double* p) {
   TetLoc L;
   bool ins = true;
@@ -52,46 +110,52 @@ __device__ TetLoc p1_locate(const P1Mesh& m, const double* p) {
   for (int a = 0; a < 3; ++a) {
     L.cell[a] = 0;
     if (ins) {
-      long long c = (long long)floor((p[a] - m.o[a]) / m.h[a]);
+      const double d = p[a] - m.o[a];
+      const double r =
+          m.slack > 0.0 && div_known_dividend(d) ? div_known(d, m.h[a], m.y[a]) : d / m.h[a];
+      long long c = (long long)floor(r);
       if (c < 0) c = 0;
       if (c > m.c[a] - 1) c = m.c[a] - 1;
       L.cell[a] = (int)c;
     }
   }
   L.loc = -1;
+  L.inside = false;
   for (int q = 0; q < 4; ++q) L.bc[q] = __builtin_nan("");
-  for (int t = 0; t < 5; ++t) {
-    double V[4][3];
-    tet_vertices(m, L.cell, t, V);
-    double vap[3], vbp[3], vab[3], vac[3], vad[3], vbc[3], vbd[3], cr[3];
-    for (int a = 0; a < 3; ++a) {
-      vap[a] = p[a] - V[0][a];
-      vbp[a] = p[a] - V[1][a];
-      vab[a] = V[1][a] - V[0][a];
-      vac[a] = V[2][a] - V[0][a];
-      vad[a] = V[3][a] - V[0][a];
-      vbc[a] = V[2][a] - V[1][a];
-      vbd[a] = V[3][a] - V[1][a];
-    }
-    cross3(vbd, vbc, cr);
-    const double va = dot3(vbp, cr) / 6.0;
-    cross3(vac, vad, cr);
-    const double vb = dot3(vap, cr) / 6.0;
-    const double v = dot3(vab, cr) / 6.0;
-    cross3(vad, vab, cr);
-    const double vc = dot3(vap, cr) / 6.0;
-    cross3(vab, vac, cr);
-    const double vd = dot3(vap, cr) / 6.0;
-    const double c0 = va / v, c1 = vb / v, c2 = vc / v, c3 = vd / v;
-    if (c0 >= 0 && c1 >= 0 && c2 >= 0 && c3 >= 0) {
+  if (!ins) return L;
+  unsigned todo = 31u;
+  if (m.slack > 0.0) {
+    // local coordinates, mirrored along x in odd cells, whose split is the
+    // mirror image of the even one
+    const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
+    double u[3];
+    for (int a = 0; a < 3; ++a)
+      u[a] = (p[a] - node_pos(m, a, L.cell[a])) * m.y[a];
+    if (odd) u[0] = 1.0 - u[0];
+    // barycentric coordinate of the apex in the corner tets 1..4 (the apexes of
+    // an even cell's are 011, 101, 000 and 110; 000 and 110 change places in
+    // an odd cell); the centre tet 0 has minus half of each
+    const double e011 = u[1] + u[2] - u[0] - 1.0, e101 = u[0] + u[2] - u[1] - 1.0;
+    const double e000 = 1.0 - u[0] - u[1] - u[2], e110 = u[0] + u[1] - u[2] - 1.0;
+    const double top = fmax(fmax(e011, e101), fmax(e000, e110));
+    todo = (top < 2.0 * m.slack ? 1u : 0u) | (e011 > -m.slack ? 2u : 0u) |
+           (e101 > -m.slack ? 4u : 0u) | ((odd ? e110 : e000) > -m.slack ? 8u : 0u) |
+           ((odd ? e000 : e110) > -m.slack ? 16u : 0u);
+  }
+  while (todo) {
+    const int t = __ffs(todo) - 1;
+    todo &= todo - 1;
+    double b[4];
+    if (m.slack > 0.0)
+      p1_barycentric<true>(m, L.cell, t, p, b);
+    else
+      p1_barycentric<false>(m, L.cell, t, p, b);
+    if (b[0] >= 0 && b[1] >= 0 && b[2] >= 0 && b[3] >= 0) {
       L.loc = t;
-      L.bc[0] = c0;
-      L.bc[1] = c1;
-      L.bc[2] = c2;
-      L.bc[3] = c3;
+      for (int q = 0; q < 4; ++q) L.bc[q] = b[q];
     }
   }
-  L.inside = ins && L.loc >= 0;
+  L.inside = L.loc >= 0;
   return L;
 }
 
@@ -286,32 +350,78 @@ __global__ void k_p1_build_rows(P1Mesh m, int kind, const double* __restrict__ p
   if (norm) norm[i] = len;
 }
 
-__global__ void k_p1_evaluate(P1Mesh m, const double* __restrict__ c,
-                              const double* __restrict__ pts, int64_t n,
-                              double* __restrict__ values, double* __restrict__ grads) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
-  const TetLoc L = p1_locate(m, p);
-  const double nan = __builtin_nan("");
-  if (!L.inside) {
-    if (values) values[i] = nan;
-    if (grads)
-      for (int d = 0; d < 3; ++d) grads[3 * i + d] = nan;
-    return;
+// gradient of the linear field of a tet from its corner values cv: along each
+// axis the difference over the edge at the apex of a corner tet, half the
+// difference of two corner pairs of the centre tet, over the cell's width
+// (the entries of the element gradient are 0, +-1 and +-1/2 over it).
+__device__ inline void p1_field_gradient(const P1Mesh& m, const int* cell, int loc,
+                                         const double* cv, double* out) {
+  const int odd = (cell[0] + cell[1] + cell[2]) & 1;
+  double d[3];
+  if (loc == 0) {
+    const double s = odd ? -0.5 : 0.5;
+    d[0] = s * ((cv[0] - cv[2]) + (cv[1] - cv[3]));
+    d[1] = s * ((cv[0] - cv[1]) + (cv[2] - cv[3]));
+    d[2] = s * ((cv[0] - cv[1]) + (cv[3] - cv[2]));
+  } else {
+    const int apex = tet_corner(odd, loc, 0);
+    const int v1 = tet_corner(odd, loc, 1) ^ apex, v2 = tet_corner(odd, loc, 2) ^ apex;
+    for (int a = 0; a < 3; ++a) {
+      const double other = v1 == 1 << a ? cv[1] : (v2 == 1 << a ? cv[2] : cv[3]);
+      d[a] = (apex >> a) & 1 ? cv[0] - other : other - cv[0];
+    }
   }
-  int64_t nd[4];
-  tet_nodes(m, loc_tet(m, L), nd);
-  const double cv[4] = {c[nd[0]], c[nd[1]], c[nd[2]], c[nd[3]]};
-  if (values)
-    values[i] = ((L.bc[0] * cv[0] + L.bc[1] * cv[1]) + L.bc[2] * cv[2]) + L.bc[3] * cv[3];
-  if (grads) {
-    double V[4][3], G[3][4];
-    tet_vertices(m, L.cell, L.loc, V);
-    grad_from_vertices(V, G);
-    for (int d = 0; d < 3; ++d)
-      grads[3 * i + d] = ((G[d][0] * cv[0] + G[d][1] * cv[1]) + G[d][2] * cv[2]) + G[d][3] * cv[3];
+  for (int a = 0; a < 3; ++a)
+    out[a] = d[a] / (node_pos(m, a, cell[a] + 1) - node_pos(m, a, cell[a]));
+}
+
+// Values and gradients at n points; points and gradients pass through LDS in
+// whole lines, as in the grid evaluation.
+constexpr int kP1EvalBlock = 256;
+__global__ __launch_bounds__(kP1EvalBlock) void k_p1_evaluate(P1Mesh m,
+                                                              const double* __restrict__ c,
+                                                              const double* __restrict__ pts,
+                                                              int64_t n,
+                                                              double* __restrict__ values,
+                                                              double* __restrict__ grads) {
+  __shared__ double sh[3 * kP1EvalBlock];
+  const int t = threadIdx.x;
+  const int64_t b = (int64_t)blockIdx.x * kP1EvalBlock;
+  const int nb = (int)(n - b < kP1EvalBlock ? n - b : kP1EvalBlock);
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (t + k * kP1EvalBlock < 3 * nb)
+      sh[t + k * kP1EvalBlock] = __builtin_nontemporal_load(pts + 3 * b + t + k * kP1EvalBlock);
+  __syncthreads();
+  if (t < nb) {
+    const double p[3] = {sh[3 * t], sh[3 * t + 1], sh[3 * t + 2]};
+    const TetLoc L = p1_locate(m, p);
+    double val = __builtin_nan(""), gr[3] = {val, val, val};
+    if (L.inside) {
+      const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
+      const int64_t nx = m.n[0], nxy = nx * m.n[1];
+      const double* q = c + L.cell[0] + nx * L.cell[1] + nxy * L.cell[2];
+      double cv[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int cr = tet_corner(odd, L.loc, k);
+        cv[k] = q[(cr & 1) + ((cr & 2) ? nx : 0) + ((cr & 4) ? nxy : 0)];
+      }
+      val = ((L.bc[0] * cv[0] + L.bc[1] * cv[1]) + L.bc[2] * cv[2]) + L.bc[3] * cv[3];
+      if (grads) p1_field_gradient(m, L.cell, L.loc, cv, gr);
+    }
+    if (values) __builtin_nontemporal_store(val, values + b + t);
+    // a thread overwrites only the three entries that it alone has read
+    sh[3 * t] = gr[0];
+    sh[3 * t + 1] = gr[1];
+    sh[3 * t + 2] = gr[2];
   }
+  if (!grads) return;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (t + k * kP1EvalBlock < 3 * nb)
+      __builtin_nontemporal_store(sh[t + k * kP1EvalBlock], grads + 3 * b + t + k * kP1EvalBlock);
 }
 
 int check_mesh(const lsamd_grid* g, const char* fn) {
@@ -488,7 +598,8 @@ extern "C" int lsamd_p1_evaluate(const lsamd_grid* g, const double* c, const dou
   if (n < 0) return fail(LSAMD_ERR_ARG, "lsamd_p1_evaluate: n < 0");
   if (n == 0) return LSAMD_OK;
   if (!c || !pts) return fail(LSAMD_ERR_ARG, "lsamd_p1_evaluate: NULL input");
-  hipLaunchKernelGGL(k_p1_evaluate, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0,
+  hipLaunchKernelGGL(k_p1_evaluate, dim3((unsigned)ceil_div(n, kP1EvalBlock)),
+                     dim3(kP1EvalBlock), 0,
                      (hipStream_t)stream, to_p1(*g), c, pts, n, values, grads);
   LSAMD_CHECK_LAUNCH("k_p1_evaluate");
   return LSAMD_OK;

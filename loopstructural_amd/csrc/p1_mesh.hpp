@@ -9,6 +9,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "exact_div.hpp"
 #include "lsamd_common.hpp"
 
 #define LSAMD_HD __host__ __device__ inline
@@ -19,7 +20,26 @@ struct P1Mesh {
   double o[3], h[3];
   int n[3];  // nodes per axis
   int c[3];  // cells per axis
+  double y[3];   // 1 / h, rounded
+  double slack;  // see p1_slack; 0: location computes every tet, plain divisions
 };
+
+// How far below zero a barycentric coordinate formed from the cell's local
+// coordinates proves that the reference's formula is negative too.  Both
+// carry a few tens of roundings of the node positions relative to the cell
+// width, eps M / h; 1e4 of them leaves a wide margin.  0 where that is no
+// longer a small number, or the steps are no divisors of div_known.
+inline double p1_slack(const P1Mesh& m) {
+  double worst = 0.0;
+  for (int a = 0; a < 3; ++a) {
+    if (!div_known_divisor(m.h[a])) return 0.0;
+    const double e = fmax(fabs(m.o[a]), fabs(m.o[a] + m.h[a] * (double)m.c[a])) / m.h[a];
+    if (!(e < 1e15)) return 0.0;
+    worst = fmax(worst, e);
+  }
+  const double s = 1e-9 + 1e4 * 2.220446049250313e-16 * worst;
+  return s < 0.05 ? s : 0.0;
+}
 
 inline P1Mesh to_p1(const lsamd_grid& g) {
   P1Mesh m;
@@ -28,7 +48,9 @@ inline P1Mesh to_p1(const lsamd_grid& g) {
     m.h[a] = g.step[a];
     m.n[a] = (int)g.nnodes[a];
     m.c[a] = (int)g.nnodes[a] - 1;
+    m.y[a] = 1.0 / g.step[a];
   }
+  m.slack = p1_slack(m);
   return m;
 }
 
