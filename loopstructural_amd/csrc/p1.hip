@@ -39,13 +39,11 @@ struct TetLoc {
   double bc[4];
 };
 
-// barycentric coordinates of p in tet t of a cell, by scalar triple products
-// as the reference forms them.
-// KNOWN: the divisions by 6 and by v through their reciprocals (div_known),
-// falling back where a dividend or v leaves its range.
-template <bool KNOWN>
-__device__ inline void p1_barycentric(const P1Mesh& m, const int* cell, int t, const double* p,
-                                      double* bc) {
+// The six times signed volumes whose ratios are the barycentric coordinates
+// of p in tet t of a cell, by scalar triple products as the reference forms
+// them: num[0..3] and the tet's own den.
+__device__ inline void p1_volumes(const P1Mesh& m, const int* cell, int t, const double* p,
+                                  double* num, double* den) {
   double V[4][3];
   tet_vertices(m, cell, t, V);
   double vap[3], vbp[3], vab[3], vac[3], vad[3], vbc[3], vbd[3], cr[3];
@@ -58,105 +56,116 @@ __device__ inline void p1_barycentric(const P1Mesh& m, const int* cell, int t, c
     vbc[a] = V[2][a] - V[1][a];
     vbd[a] = V[3][a] - V[1][a];
   }
-  double num[4], den;
   cross3(vbd, vbc, cr);
   num[0] = dot3(vbp, cr);
   cross3(vac, vad, cr);
   num[1] = dot3(vap, cr);
-  den = dot3(vab, cr);
+  *den = dot3(vab, cr);
   cross3(vad, vab, cr);
   num[2] = dot3(vap, cr);
   cross3(vab, vac, cr);
   num[3] = dot3(vap, cr);
-  if constexpr (KNOWN) {
-    const double v = div_known(den, 6.0, 1.0 / 6.0), av = fabs(v);
-    bool ok = div_known_dividend(den) && div_known_divisor(av);
-    double s[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      ok = ok && div_known_dividend(num[k]);
-      s[k] = div_known(num[k], 6.0, 1.0 / 6.0);
-      ok = ok && div_known_dividend(s[k]);
-    }
-    if (ok) {
-      const double y = 1.0 / v;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) bc[k] = div_known(s[k], v, y);
-      return;
-    }
-  }
-  const double v = den / 6.0;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) bc[k] = (num[k] / 6.0) / v;
+}
+
+__device__ inline bool p1_inside(const P1Mesh& m, const double* p) {
+  bool ins = true;
+  for (int a = 0; a < 3; ++a)
+    ins = ins && (p[a] > m.o[a]) && (p[a] < m.o[a] + m.h[a] * (double)m.c[a]);
+  return ins;
 }
 
 // get_element_for_location for one point: strict box test, cell lookup,
-// barycentric coordinates in the tets, the last tet with all coordinates
+// barycentric coordinates in all 5 tets, the last tet with all coordinates
 // >= 0 wins.
-//
-// Coordinates of all five tets (nine divisions and a hundred other FP64
-// operations each) bound evaluation by arithmetic, not memory, so with
-// m.slack > 0 only the tets are computed that can pass: the cell's local coordinates give
-// every tet's smallest barycentric coordinate up to a rounding error far
-// below m.slack (see p1_slack), and a tet below -m.slack fails the exact test
-// for certain.  Almost every point has one such tet.
 __device__ TetLoc p1_locate(const P1Mesh& m, const double* p) {
   TetLoc L;
-  bool ins = true;
-  for (int a = 0; a < 3; ++a) {
-    ins = ins && (p[a] > m.o[a]);
-    ins = ins && (p[a] < m.o[a] + m.h[a] * (double)m.c[a]);
-  }
+  const bool ins = p1_inside(m, p);
   for (int a = 0; a < 3; ++a) {
     L.cell[a] = 0;
     if (ins) {
-      const double d = p[a] - m.o[a];
-      const double r =
-          m.slack > 0.0 && div_known_dividend(d) ? div_known(d, m.h[a], m.y[a]) : d / m.h[a];
-      long long c = (long long)floor(r);
+      long long c = (long long)floor((p[a] - m.o[a]) / m.h[a]);
       if (c < 0) c = 0;
       if (c > m.c[a] - 1) c = m.c[a] - 1;
       L.cell[a] = (int)c;
     }
   }
   L.loc = -1;
-  L.inside = false;
   for (int q = 0; q < 4; ++q) L.bc[q] = __builtin_nan("");
-  if (!ins) return L;
-  unsigned todo = 31u;
-  if (m.slack > 0.0) {
-    // local coordinates, mirrored along x in odd cells, whose split is the
-    // mirror image of the even one
-    const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
-    double u[3];
-    for (int a = 0; a < 3; ++a)
-      u[a] = (p[a] - node_pos(m, a, L.cell[a])) * m.y[a];
-    if (odd) u[0] = 1.0 - u[0];
-    // barycentric coordinate of the apex in the corner tets 1..4 (the apexes of
-    // an even cell's are 011, 101, 000 and 110; 000 and 110 change places in
-    // an odd cell); the centre tet 0 has minus half of each
-    const double e011 = u[1] + u[2] - u[0] - 1.0, e101 = u[0] + u[2] - u[1] - 1.0;
-    const double e000 = 1.0 - u[0] - u[1] - u[2], e110 = u[0] + u[1] - u[2] - 1.0;
-    const double top = fmax(fmax(e011, e101), fmax(e000, e110));
-    todo = (top < 2.0 * m.slack ? 1u : 0u) | (e011 > -m.slack ? 2u : 0u) |
-           (e101 > -m.slack ? 4u : 0u) | ((odd ? e110 : e000) > -m.slack ? 8u : 0u) |
-           ((odd ? e000 : e110) > -m.slack ? 16u : 0u);
+  for (int t = 0; t < 5; ++t) {
+    double num[4], den;
+    p1_volumes(m, L.cell, t, p, num, &den);
+    const double v = den / 6.0;
+    const double c0 = (num[0] / 6.0) / v, c1 = (num[1] / 6.0) / v, c2 = (num[2] / 6.0) / v,
+                 c3 = (num[3] / 6.0) / v;
+    if (c0 >= 0 && c1 >= 0 && c2 >= 0 && c3 >= 0) {
+      L.loc = t;
+      L.bc[0] = c0;
+      L.bc[1] = c1;
+      L.bc[2] = c2;
+      L.bc[3] = c3;
+    }
   }
+  L.inside = ins && L.loc >= 0;
+  return L;
+}
+
+// p1_locate of a point inside the box, bit for bit the same, for meshes with
+// m.slack > 0.  Coordinates of all five tets (nine divisions and a hundred
+// other FP64 operations each) bound evaluation by arithmetic, so only the
+// tets are computed that can pass: the cell's local coordinates give every
+// tet's smallest barycentric coordinate up to a rounding error far below
+// m.slack (see p1_slack), and a tet below -m.slack fails the exact test for
+// certain; almost every point has one such tet.  The divisions go through
+// their divisors' reciprocals (div_known).  False where a dividend leaves
+// their range.  One straight line of code: in small calls every jump waits
+// for its instructions (with a fall-back at each division 5e4 points took 16
+// us against 8).
+__device__ inline bool p1_locate_known(const P1Mesh& m, const double* p, TetLoc& L) {
+  bool ok = true;
+  double u[3];
+  for (int a = 0; a < 3; ++a) {
+    const double d = p[a] - m.o[a];
+    ok = ok & div_known_dividend(d);
+    int c = (int)floor(div_known(d, m.h[a], m.y[a]));
+    c = c < 0 ? 0 : c;
+    L.cell[a] = c > m.c[a] - 1 ? m.c[a] - 1 : c;
+    u[a] = (p[a] - node_pos(m, a, L.cell[a])) * m.y[a];
+  }
+  // local coordinates, mirrored along x in odd cells, whose split is the
+  // mirror image of the even one
+  const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
+  u[0] = odd ? 1.0 - u[0] : u[0];
+  // barycentric coordinate of the apex in the corner tets 1..4 (the apexes of
+  // an even cell's are 011, 101, 000 and 110; 000 and 110 change places in
+  // an odd cell); the centre tet 0 has minus half of each
+  const double e011 = u[1] + u[2] - u[0] - 1.0, e101 = u[0] + u[2] - u[1] - 1.0;
+  const double e000 = 1.0 - u[0] - u[1] - u[2], e110 = u[0] + u[1] - u[2] - 1.0;
+  const double top = fmax(fmax(e011, e101), fmax(e000, e110));
+  unsigned todo = (top < 2.0 * m.slack ? 1u : 0u) | (e011 > -m.slack ? 2u : 0u) |
+                  (e101 > -m.slack ? 4u : 0u) | ((odd ? e110 : e000) > -m.slack ? 8u : 0u) |
+                  ((odd ? e000 : e110) > -m.slack ? 16u : 0u);
+  L.loc = -1;
   while (todo) {
     const int t = __ffs(todo) - 1;
     todo &= todo - 1;
-    double b[4];
-    if (m.slack > 0.0)
-      p1_barycentric<true>(m, L.cell, t, p, b);
-    else
-      p1_barycentric<false>(m, L.cell, t, p, b);
-    if (b[0] >= 0 && b[1] >= 0 && b[2] >= 0 && b[3] >= 0) {
-      L.loc = t;
-      for (int q = 0; q < 4; ++q) L.bc[q] = b[q];
+    double num[4], den;
+    p1_volumes(m, L.cell, t, p, num, &den);
+    const double v = div_known(den, 6.0, 1.0 / 6.0), y = 1.0 / v;
+    ok = ok & div_known_dividend(den) & div_known_divisor(fabs(v));
+    bool in = true;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double s = div_known(num[k], 6.0, 1.0 / 6.0);
+      ok = ok & div_known_dividend(num[k]) & div_known_dividend(s);
+      num[k] = div_known(s, v, y);
+      in = in & (num[k] >= 0);
     }
+    L.loc = in ? t : L.loc;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) L.bc[k] = in ? num[k] : L.bc[k];
   }
   L.inside = L.loc >= 0;
-  return L;
+  return ok;
 }
 
 __device__ inline int64_t loc_tet(const P1Mesh& m, const TetLoc& L) {
@@ -350,34 +359,42 @@ __global__ void k_p1_build_rows(P1Mesh m, int kind, const double* __restrict__ p
   if (norm) norm[i] = len;
 }
 
-// gradient of the linear field of a tet from its corner values cv: along each
-// axis the difference over the edge at the apex of a corner tet, half the
-// difference of two corner pairs of the centre tet, over the cell's width
-// (the entries of the element gradient are 0, +-1 and +-1/2 over it).
-__device__ inline void p1_field_gradient(const P1Mesh& m, const int* cell, int loc,
-                                         const double* cv, double* out) {
-  const int odd = (cell[0] + cell[1] + cell[2]) & 1;
-  double d[3];
-  if (loc == 0) {
-    const double s = odd ? -0.5 : 0.5;
-    d[0] = s * ((cv[0] - cv[2]) + (cv[1] - cv[3]));
-    d[1] = s * ((cv[0] - cv[1]) + (cv[2] - cv[3]));
-    d[2] = s * ((cv[0] - cv[1]) + (cv[3] - cv[2]));
-  } else {
-    const int apex = tet_corner(odd, loc, 0);
-    const int v1 = tet_corner(odd, loc, 1) ^ apex, v2 = tet_corner(odd, loc, 2) ^ apex;
-    for (int a = 0; a < 3; ++a) {
-      const double other = v1 == 1 << a ? cv[1] : (v2 == 1 << a ? cv[2] : cv[3]);
-      d[a] = (apex >> a) & 1 ? cv[0] - other : other - cv[0];
-    }
+// value and gradient at p of the linear field of its tet, from the corner
+// values cv.  Along each axis the gradient is the difference over the edge at
+// the apex of a corner tet, half the difference of two corner pairs of the
+// centre tet, over the cell's width (the entries of the element gradient are
+// 0, +-1 and +-1/2 over it).
+__device__ inline void p1_field(const P1Mesh& m, const TetLoc& L, const double* __restrict__ c,
+                                double* val, double* gr) {
+  const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
+  const int64_t nx = m.n[0], nxy = nx * m.n[1];
+  const double* q = c + L.cell[0] + nx * L.cell[1] + nxy * L.cell[2];
+  int cr[4];
+  double cv[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    cr[k] = tet_corner(odd, L.loc, k);
+    cv[k] = q[(cr[k] & 1) + ((cr[k] & 2) ? nx : 0) + ((cr[k] & 4) ? nxy : 0)];
   }
-  for (int a = 0; a < 3; ++a)
-    out[a] = d[a] / (node_pos(m, a, cell[a] + 1) - node_pos(m, a, cell[a]));
+  *val = ((L.bc[0] * cv[0] + L.bc[1] * cv[1]) + L.bc[2] * cv[2]) + L.bc[3] * cv[3];
+  const double s = odd ? -0.5 : 0.5;
+  const double mid[3] = {s * ((cv[0] - cv[2]) + (cv[1] - cv[3])),
+                         s * ((cv[0] - cv[1]) + (cv[2] - cv[3])),
+                         s * ((cv[0] - cv[1]) + (cv[3] - cv[2]))};
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int nb = cr[0] ^ (1 << a);  // the apex's neighbour along the axis
+    const double other = cr[1] == nb ? cv[1] : (cr[2] == nb ? cv[2] : cv[3]);
+    const double edge = (cr[0] >> a) & 1 ? cv[0] - other : other - cv[0];
+    gr[a] = (L.loc == 0 ? mid[a] : edge) /
+            (node_pos(m, a, L.cell[a] + 1) - node_pos(m, a, L.cell[a]));
+  }
 }
 
 // Values and gradients at n points; points and gradients pass through LDS in
 // whole lines, as in the grid evaluation.
 constexpr int kP1EvalBlock = 256;
+template <bool KNOWN>
 __global__ __launch_bounds__(kP1EvalBlock) void k_p1_evaluate(P1Mesh m,
                                                               const double* __restrict__ c,
                                                               const double* __restrict__ pts,
@@ -395,21 +412,15 @@ __global__ __launch_bounds__(kP1EvalBlock) void k_p1_evaluate(P1Mesh m,
   __syncthreads();
   if (t < nb) {
     const double p[3] = {sh[3 * t], sh[3 * t + 1], sh[3 * t + 2]};
-    const TetLoc L = p1_locate(m, p);
     double val = __builtin_nan(""), gr[3] = {val, val, val};
-    if (L.inside) {
-      const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
-      const int64_t nx = m.n[0], nxy = nx * m.n[1];
-      const double* q = c + L.cell[0] + nx * L.cell[1] + nxy * L.cell[2];
-      double cv[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) {
-        const int cr = tet_corner(odd, L.loc, k);
-        cv[k] = q[(cr & 1) + ((cr & 2) ? nx : 0) + ((cr & 4) ? nxy : 0)];
-      }
-      val = ((L.bc[0] * cv[0] + L.bc[1] * cv[1]) + L.bc[2] * cv[2]) + L.bc[3] * cv[3];
-      if (grads) p1_field_gradient(m, L.cell, L.loc, cv, gr);
+    TetLoc L;
+    L.inside = false;
+    if (KNOWN) {
+      if (p1_inside(m, p) && !p1_locate_known(m, p, L)) L = p1_locate(m, p);
+    } else {
+      L = p1_locate(m, p);
     }
+    if (L.inside) p1_field(m, L, c, &val, gr);
     if (values) __builtin_nontemporal_store(val, values + b + t);
     // a thread overwrites only the three entries that it alone has read
     sh[3 * t] = gr[0];
@@ -598,9 +609,14 @@ extern "C" int lsamd_p1_evaluate(const lsamd_grid* g, const double* c, const dou
   if (n < 0) return fail(LSAMD_ERR_ARG, "lsamd_p1_evaluate: n < 0");
   if (n == 0) return LSAMD_OK;
   if (!c || !pts) return fail(LSAMD_ERR_ARG, "lsamd_p1_evaluate: NULL input");
-  hipLaunchKernelGGL(k_p1_evaluate, dim3((unsigned)ceil_div(n, kP1EvalBlock)),
-                     dim3(kP1EvalBlock), 0,
-                     (hipStream_t)stream, to_p1(*g), c, pts, n, values, grads);
+  const P1Mesh m = to_p1(*g);
+  const dim3 nb((unsigned)ceil_div(n, kP1EvalBlock)), bs(kP1EvalBlock);
+  if (m.slack > 0.0)
+    hipLaunchKernelGGL(k_p1_evaluate<true>, nb, bs, 0, (hipStream_t)stream, m, c, pts, n, values,
+                       grads);
+  else
+    hipLaunchKernelGGL(k_p1_evaluate<false>, nb, bs, 0, (hipStream_t)stream, m, c, pts, n, values,
+                       grads);
   LSAMD_CHECK_LAUNCH("k_p1_evaluate");
   return LSAMD_OK;
 }
