@@ -72,6 +72,10 @@ int check_uniform_grid(const lsamd_grid* g, const char* fn) {
 struct CgCtl {
   double rho, rho_prev, pq_st, pq_rows, thr, bnorm, acc, alpha, res2;
   int iter, done, maxiter, converged;
+  // two-launch iteration (pcg.hpp): rho and the count of iterations begun,
+  // written alternately by even and odd iterations
+  double rs[2];
+  int its[2];
 };
 
 // ------------------------------------------------------------- stencil ----
@@ -993,56 +997,8 @@ __global__ __launch_bounds__(VB) void k_cg_init_fin(const double* __restrict__ p
     ctl->maxiter = maxiter;
     ctl->converged = (sqrt(tot) < thr) || bn == 0.0;
     ctl->done = ctl->converged;
-  }
-}
-
-// p = minv r + beta p  (beta = rho/rho_prev, p = minv r on the first step)
-template <typename T>
-__global__ __launch_bounds__(VB) void k_cg_dir(const T* __restrict__ r, const T* __restrict__ minv,
-                                               T* __restrict__ p, int64_t n, CgCtl* ctl) {
-  if (ctl->done) return;
-  const int first = ctl->iter == 0;
-  const T beta = first ? (T)0 : (T)(ctl->rho / ctl->rho_prev);
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    const T z = minv[i] * r[i];
-    p[i] = first ? z : z + beta * p[i];
-  }
-}
-
-// x += alpha p ; r -= alpha q ; partials of r.(minv r)
-template <typename T>
-__global__ __launch_bounds__(VB) void k_cg_upd(T* __restrict__ x, T* __restrict__ r,
-                                               const T* __restrict__ p, const T* __restrict__ q,
-                                               const T* __restrict__ minv, int64_t n,
-                                               double* part, CgCtl* ctl) {
-  if (ctl->done) return;
-  __shared__ double sh[VB / 64];
-  const T alpha = (T)ctl->alpha;
-  double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * VB + threadIdx.x; i < n; i += (int64_t)gridDim.x * VB) {
-    x[i] += alpha * p[i];
-    const T rv = r[i] - alpha * q[i];
-    r[i] = rv;
-    acc += (double)rv * (double)(minv[i] * rv);
-  }
-  const double bs = block_sum(acc, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = bs;
-}
-
-// one block: rho_prev = rho ; rho = sum(part) ; iter++ ; stopping test
-__global__ __launch_bounds__(VB) void k_cg_upd_fin(const double* __restrict__ part, int np,
-                                                   CgCtl* ctl) {
-  if (ctl->done) return;
-  __shared__ double sh[VB / 64];
-  const double tot = reduce_partials(part, np, sh);
-  if (threadIdx.x == 0) {
-    ctl->rho_prev = ctl->rho;
-    ctl->rho = tot;
-    const int it = ctl->iter + 1;
-    ctl->iter = it;
-    const int conv = sqrt(tot) < ctl->thr;
-    ctl->converged = conv;
-    ctl->done = conv || it >= ctl->maxiter;
+    ctl->rs[0] = ctl->rs[1] = 1.0;
+    ctl->its[0] = ctl->its[1] = 0;
   }
 }
 
@@ -1133,6 +1089,7 @@ __global__ void k_check_cols(const int32_t* __restrict__ cols, int64_t nnz, int6
 }
 
 #include "batch_kernels.hpp"
+#include "pcg.hpp"
 #include "lsmr.hpp"
 #include "mg.hpp"
 #include "mrhs.hpp"
@@ -1236,6 +1193,17 @@ struct lsamd_fd_system {
   double* minv64 = nullptr;
   float* minv32 = nullptr;
   // work
+  // Jacobi PCG (pcg.hpp): the data term by node (gram_state: 0 not built for
+  // these rows, 1 built, 2 its rows are too long), the direction's second
+  // buffer per precision, the partials of r.z and of the data term
+  int gram_state = 0, gram_width = 0;
+  int32_t *gram_col = nullptr, *gram_base = nullptr;
+  double* gram_v64 = nullptr;
+  float* gram_v32 = nullptr;
+  uint64_t* gram_mask = nullptr;
+  void* gram_q = nullptr;
+  double *pcg_b64 = nullptr, *pcg_pr = nullptr, *pcg_pg = nullptr;
+  float* pcg_b32 = nullptr;
   double *x64 = nullptr, *r64 = nullptr, *p64 = nullptr, *q64 = nullptr, *t64 = nullptr;
   float *x32 = nullptr, *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *t32 = nullptr;
   double* part = nullptr;
@@ -1305,7 +1273,8 @@ void dfree(lsamd_fd_system* s, void* p) {
 enum RowSlot {
   kRsRowPtr, kRsCols, kRsCoef64, kRsCoef32, kRsB, kRsW, kRsW2_64, kRsW2_32, kRsT64, kRsT32,
   kRsPartRows, kRsURows, kRsBad, kRsErow, kRsKeys, kRsVals, kRsSegEntry, kRsSegRow, kRsUniq,
-  kRsCounts, kRsNrun, kRsTmp, kRsOff32, kRsSegPtr, kRsDnode, kRsAdjoint, kRsSlots
+  kRsCounts, kRsNrun, kRsTmp, kRsOff32, kRsSegPtr, kRsDnode, kRsAdjoint, kRsGramCol,
+  kRsGramV64, kRsGramV32, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart, kRsGramOver, kRsSlots
 };
 
 template <typename P>
@@ -1417,7 +1386,7 @@ int64_t stencil_partials(const lsamd_fd_system* s, int zc) {
     return p1_blocks(s, (zc >= 1 && zc <= kP1NCfg) ? zc - 1 : kP1Default - 1);
   }
   if (!s->regular) return ceil_div(s->n, 256);
-  return s->nstile[zc_index(zc)];
+  return s->nstile[zc_index(zc ? zc : kTile32 + 8)];
 }
 
 // the regular single-system stencil: one launch over the system's work items
@@ -1567,12 +1536,13 @@ int64_t launch_stencil(lsamd_fd_system* s, const T* x, T* y, const CgCtl* ctl, h
     return ceil_div(s->n, 256);
   }
   switch (zc) {
+    case 0:  // not timed: a grid small enough for k_pcg_tile
+    case kTile32 + 8: launch_bulk<T, 8, false, 32>(s, x, y, ctl, st); break;
     case 8: launch_bulk<T, 8>(s, x, y, ctl, st); break;
     case 16: launch_bulk<T, 16>(s, x, y, ctl, st); break;
     case kDmaZc + 8: launch_bulk<T, 8, true>(s, x, y, ctl, st); break;
     case kDmaZc + 16: launch_bulk<T, 16, true>(s, x, y, ctl, st); break;
     case kDmaZc + 32: launch_bulk<T, 32, true>(s, x, y, ctl, st); break;
-    case kTile32 + 8: launch_bulk<T, 8, false, 32>(s, x, y, ctl, st); break;
     case kTile32 + 16: launch_bulk<T, 16, false, 32>(s, x, y, ctl, st); break;
     case kTile32 + 32: launch_bulk<T, 32, false, 32>(s, x, y, ctl, st); break;
     default: launch_bulk<T, 32>(s, x, y, ctl, st); break;
@@ -1694,14 +1664,136 @@ int launch_apply(lsamd_fd_system* s, const T* x, T* y, T* t, CgCtl* ctl, hipStre
   return LSAMD_OK;
 }
 
+// Data term by node of the current rows, built on the first Jacobi solve
+// after they changed (gram_state).  Rows that couple a node with more than
+// kGramCap others, or more than kGramNodesMax data nodes, keep the row form.
+
+int pcg_gram_ensure(lsamd_fd_system* s, hipStream_t st) {
+  if (s->gram_state || s->nrows == 0) return LSAMD_OK;
+  s->gram_state = 2;
+  const int64_t nd = s->ndn, nw = ceil_div(s->n, 64);
+  if (nd > kGramNodesMax) return LSAMD_OK;
+  int* over = nullptr;
+  double* gq = nullptr;
+  if (int rc = rbuf(s, kRsGramCol, &s->gram_col, nd * kGramCap)) return rc;
+  if (int rc = rbuf(s, kRsGramV64, &s->gram_v64, nd * kGramCap)) return rc;
+  if (int rc = rbuf(s, kRsGramV32, &s->gram_v32, nd * kGramCap)) return rc;
+  if (int rc = rbuf(s, kRsGramMask, &s->gram_mask, nw)) return rc;
+  if (int rc = rbuf(s, kRsGramBase, &s->gram_base, nw)) return rc;
+  if (int rc = rbuf(s, kRsGramQ, &gq, nd)) return rc;
+  if (int rc = rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB))) return rc;
+  if (int rc = rbuf(s, kRsGramOver, &over, 2)) return rc;
+  s->gram_q = gq;
+  // rows of half the width first where one row set's columns suggest it
+  // (four-node rows); a longer one costs a second pass
+  int width = s->nnz <= 5 * s->nrows ? kGramCap / 2 : kGramCap;
+  for (;;) {
+    LSAMD_HIP(hipMemsetAsync(over, 0, 2 * sizeof(int), st));
+    hipLaunchKernelGGL(k_pcg_gram_build, dim3((unsigned)ceil_div(nd, 64)), dim3(64), 0, st,
+                       rows_dev(s, false), (const double*)s->coef64, (const double*)s->w2_64,
+                       width, s->gram_col, s->gram_v64, s->gram_v32, over);
+    hipLaunchKernelGGL(k_pcg_gram_mask, dim3((unsigned)ceil_div(nw, 256)), dim3(256), 0, st,
+                       (const int32_t*)s->dnode, nd, nw, s->gram_mask, s->gram_base);
+    LSAMD_CHECK_LAUNCH("data term by node");
+    int ho[2] = {0, 0};
+    LSAMD_HIP(hipMemcpyAsync(ho, over, sizeof(ho), hipMemcpyDeviceToHost, st));
+    LSAMD_HIP(hipStreamSynchronize(st));
+    if (ho[0]) return LSAMD_OK;
+    if (!ho[1] || width == kGramCap) break;
+    width = kGramCap;
+  }
+  s->gram_width = width;
+  s->gram_state = 1;
+  return LSAMD_OK;
+}
+
+GramDev gram_dev(const lsamd_fd_system* s, bool f32) {
+  GramDev G;
+  memset(&G, 0, sizeof(G));
+  if (s->gram_state != 1) return G;
+  G.ndn = s->ndn;
+  G.node = s->dnode;
+  G.col = s->gram_col;
+  G.val = f32 ? (const void*)s->gram_v32 : (const void*)s->gram_v64;
+  G.mask = s->gram_mask;
+  G.base = s->gram_base;
+  return G;
+}
+
+// Workgroups of the one-launch direction and regulariser (k_pcg_tile); 0 where
+// a direction launch and the plane-streaming stencil are faster.  The tile
+// saves a launch and its loads' latency but reads three vectors over its halo
+// (3.75 times per node).  us per iteration, tile against streaming, FP64 and
+// FP32: 11^3 nodes (6 tiles) 9.5 against 16.1, 9.4 against 15.1; 46^3 (216)
+// 11.5, 19.0 and 10.4, 16.8; 64^3 (512) 18.6, 22.7 and 14.5, 19.1; 93 x 77 x 61
+// (960) 28.2, 26.8 and 21.1, 21.0; 96^3 (1728) 42.0, 36.3 and 28.6, 25.7; so up
+// to three tiles per CU.
+constexpr int kPcgTilesMax = 768;
+int pcg_tiles(const lsamd_fd_system* s) {
+  if (s->op != 0 || !s->regular) return 0;
+  const int64_t nb = ceil_div(s->gd.nx, kTlX) * ceil_div(s->gd.ny, kTlY) * ceil_div(s->gd.nz, kTlZ);
+  return nb <= kPcgTilesMax ? (int)nb : 0;
+}
+
+// One Jacobi PCG iteration (see pcg.hpp); `par` is its parity.  The operator's
+// partials go to s->part, those of r.z to s->pcg_pr.
 template <typename T>
-int launch_iteration(lsamd_fd_system* s, T* x, T* r, T* p, T* q, T* t, const T* minv, CgCtl* ctl,
-                     hipStream_t st) {
-  const int vb = vec_blocks(s->n);
-  hipLaunchKernelGGL(k_cg_dir<T>, dim3(vb), dim3(VB), 0, st, r, minv, p, s->n, ctl);
-  if (int rc = launch_apply<T>(s, p, q, t, ctl, st)) return rc;
-  hipLaunchKernelGGL(k_cg_upd<T>, dim3(vb), dim3(VB), 0, st, x, r, p, q, minv, s->n, s->part, ctl);
-  hipLaunchKernelGGL(k_cg_upd_fin, dim3(1), dim3(VB), 0, st, (const double*)s->part, vb, ctl);
+int launch_iteration(lsamd_fd_system* s, int par, T* x, T* r, T* pa, T* pb, T* q, T* t,
+                     const T* minv, CgCtl* ctl, hipStream_t st) {
+  const bool f32 = sizeof(T) == 4;
+  const int vb = pcg_blocks(s->n, sizeof(T));
+  const GramDev G = gram_dev(s, f32);
+  T* gq = (T*)s->gram_q;
+  const bool half = s->gram_width == kGramCap / 2;
+  const T* po = par ? pb : pa;
+  T* pn = par ? pa : pb;
+  const int nt = pcg_tiles(s);
+  int64_t nq = 0;
+  int nrow = 0;
+  if (nt > 0) {
+    const int ng = (int)ceil_div(G.ndn * kGramLanes, kTlN);
+    nq = nt + ng;
+    const T* tab = f32 ? (const T*)s->tab32 : (const T*)s->tab64;
+    if (half)
+      hipLaunchKernelGGL((k_pcg_tile<T, kGramCap / 2>), dim3((unsigned)nq), dim3(kTlN), 0, st,
+                         (const T*)r, minv, po, pn, q, s->gd, tab, G, ng, gq,
+                         (const double*)s->pcg_pr, vb, s->part, ctl, par);
+    else
+      hipLaunchKernelGGL((k_pcg_tile<T, kGramCap>), dim3((unsigned)nq), dim3(kTlN), 0, st,
+                         (const T*)r, minv, po, pn, q, s->gd, tab, G, ng, gq,
+                         (const double*)s->pcg_pr, vb, s->part, ctl, par);
+  } else {
+    const int ng = (int)ceil_div(G.ndn * kGramLanes, VB);
+    const dim3 nb((unsigned)(vb + ng));
+    if (half)
+      hipLaunchKernelGGL((k_pcg_dir<T, kGramCap / 2>), nb, dim3(VB), 0, st, (const T*)r, minv, po,
+                         pn, s->n, G, ng, gq, (const double*)s->pcg_pr, vb, s->pcg_pg, ctl, par);
+    else
+      hipLaunchKernelGGL((k_pcg_dir<T, kGramCap>), nb, dim3(VB), 0, st, (const T*)r, minv, po, pn,
+                         s->n, G, ng, gq, (const double*)s->pcg_pr, vb, s->pcg_pg, ctl, par);
+    nq = launch_stencil<T>(s, (const T*)pn, q, ctl, st, s->zc[f32 ? 1 : 0]);
+    nrow = ng;
+  }
+  const double* part_g = s->pcg_pg;
+  if (s->nrows > 0 && s->gram_state != 1) {
+    const RowsDev R = rows_dev(s, f32);
+    nrow = (int)ceil_div(s->nrows, 256);
+    part_g = s->part_rows;
+    hipLaunchKernelGGL(k_rows_t<T>, dim3((unsigned)nrow), dim3(256), 0, st, (const T*)pn, R, t,
+                       s->part_rows, ctl);
+    hipLaunchKernelGGL((k_rows_scatter<T, T>),
+                       dim3((unsigned)std::max<int64_t>(1, ceil_div(s->ndn, 256))), dim3(256), 0,
+                       st, R, (const T*)t, q, 1, ctl, 0, (const double*)nullptr, 0,
+                       (const double*)nullptr, 0);
+  }
+  if (nq + nrow > kPcgPartMax) {
+    hipLaunchKernelGGL(k_pcg_alpha, dim3(1), dim3(VB), 0, st, (const double*)s->part, (int)nq,
+                       part_g, nrow, ctl, par);
+    nq = -1;
+  }
+  hipLaunchKernelGGL(k_pcg_upd<T>, dim3((unsigned)vb), dim3(VB), 0, st, x, r, (const T*)pn,
+                     (const T*)q, minv, s->n, G, (const T*)gq, (const double*)s->part, (int)nq,
+                     part_g, nrow, s->pcg_pr, (const CgCtl*)ctl, par);
   LSAMD_CHECK_LAUNCH("cg iteration");
   return LSAMD_OK;
 }
@@ -1709,9 +1801,10 @@ int launch_iteration(lsamd_fd_system* s, T* x, T* r, T* p, T* q, T* t, const T* 
 template <typename T>
 int launch_init(lsamd_fd_system* s, const double* b, const T* minv, T* x, T* r, double rtol,
                 double atol, int maxiter, hipStream_t st) {
-  const int vb = vec_blocks(s->n);
-  hipLaunchKernelGGL(k_cg_init<T>, dim3(vb), dim3(VB), 0, st, b, minv, x, r, s->n, s->part);
-  hipLaunchKernelGGL(k_cg_init_fin, dim3(1), dim3(VB), 0, st, (const double*)s->part, vb, rtol,
+  // the partials stay for the first iteration's rho
+  const int vb = pcg_blocks(s->n, sizeof(T));
+  hipLaunchKernelGGL(k_cg_init<T>, dim3(vb), dim3(VB), 0, st, b, minv, x, r, s->n, s->pcg_pr);
+  hipLaunchKernelGGL(k_cg_init_fin, dim3(1), dim3(VB), 0, st, (const double*)s->pcg_pr, vb, rtol,
                      atol, maxiter, s->ctl);
   LSAMD_CHECK_LAUNCH("cg init");
   return LSAMD_OK;
@@ -1736,12 +1829,23 @@ int ensure_work(lsamd_fd_system* s, bool f32) {
   return LSAMD_OK;
 }
 
+// second buffer of the PCG direction (zeroed: the first iteration reads and
+// discards it)
+template <typename T>
+int pcg_buffer(lsamd_fd_system* s, T** p) {
+  if (*p) return LSAMD_OK;
+  if (int rc = dalloc(s, p, s->n)) return rc;
+  LSAMD_HIP(legacy_memset(*p, 0, s->n * sizeof(T)));
+  return LSAMD_OK;
+}
+
 // Run chunks of `chunk` PCG iterations (captured once into a graph) until
 // the device control block reports done.
 template <typename T>
-int run_pcg(lsamd_fd_system* s, int chunk, T* x, T* r, T* p, T* q, T* t, const T* minv,
+int run_pcg(lsamd_fd_system* s, int chunk, T* x, T* r, T* p, T* pb, T* q, T* t, const T* minv,
             hipStream_t st) {
   const int gi = sizeof(T) == 4 ? 1 : 0;
+  chunk += chunk & 1;  // whole pairs: an iteration's parity is fixed at capture
   if (s->graph[gi] && s->graph_chunk[gi] != chunk) {
     hipGraphExecDestroy(s->graph[gi]);
     s->graph[gi] = nullptr;
@@ -1754,7 +1858,9 @@ int run_pcg(lsamd_fd_system* s, int chunk, T* x, T* r, T* p, T* q, T* t, const T
     LSAMD_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
     int rc = LSAMD_OK;
     for (int i = 0; i < chunk && rc == LSAMD_OK; ++i)
-      rc = launch_iteration<T>(s, x, r, p, q, t, minv, s->ctl, cs);
+      rc = launch_iteration<T>(s, i & 1, x, r, p, pb, q, t, minv, s->ctl, cs);
+    hipLaunchKernelGGL(k_pcg_check, dim3(1), dim3(VB), 0, cs, (const double*)s->pcg_pr,
+                       pcg_blocks(s->n, sizeof(T)), s->ctl);
     hipError_t e = hipStreamEndCapture(cs, &graph);
     hipStreamDestroy(cs);
     if (rc) return rc;
@@ -1781,8 +1887,11 @@ int init_common(lsamd_fd_system* s) {
     pm = std::max(pm, p1_max_partials(s));
   else
     for (int c = 0; c < kNStCand; ++c) pm = std::max(pm, stencil_partials(s, kStCand[c]));
+  // room for the partials of k_pcg_tile and its data-term workgroups
+  pm += kPcgTilesMax + ceil_div(kGramNodesMax * kGramLanes, kTlN);
   s->part_n = pm;
   if (int rc = dalloc(s, &s->part, s->part_n)) return rc;
+  if (int rc = dalloc(s, &s->pcg_pr, kPcgBlocks)) return rc;
   if (int rc = dalloc(s, &s->ctl, 1)) return rc;
   if (int rc = dalloc(s, &s->ctl_apply, 1)) return rc;
   LSAMD_HIP(legacy_memset(s->ctl, 0, sizeof(CgCtl)));
@@ -4635,6 +4744,7 @@ int lsamd_fd_system_set_rows(lsamd_fd_system* s, int64_t nrows, int64_t nnz,
   s->t64 = nullptr;
   s->t32 = nullptr;
   s->part_rows = nullptr;
+  s->gram_state = 0;
   LSAMD_HIP(hipMemsetAsync(s->ctl, 0, sizeof(CgCtl), st));
   LSAMD_HIP(hipMemsetAsync(s->ctl_apply, 0, sizeof(CgCtl), st));
   s->nrows = nrows;
@@ -4835,12 +4945,19 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
   const int vb = vec_blocks(n);
   lsamd_solve_info inf;
   memset(&inf, 0, sizeof(inf));
+  // the tile form takes no timed stencil (the FP64 residuals of the mixed
+  // solve, a handful, take the form of a small grid)
+  const bool timed = pcg_tiles(s) == 0;
   if (o->precision == LSAMD_FP64) {
     if (int rc = ensure_work(s, false)) return rc;
-    if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
+    if (timed)
+      if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
     if (int rc = launch_init<double>(s, b, minv64, s->x64, s->r64, o->rtol, o->atol, maxiter, st))
       return rc;
-    if (int rc = run_pcg<double>(s, chunk, s->x64, s->r64, s->p64, s->q64, s->t64, minv64, st))
+    if (int rc = pcg_gram_ensure(s, st)) return rc;
+    if (int rc = pcg_buffer(s, &s->pcg_b64)) return rc;
+    if (int rc = run_pcg<double>(s, chunk, s->x64, s->r64, s->p64, s->pcg_b64, s->q64, s->t64,
+                                 minv64, st))
       return rc;
     hipLaunchKernelGGL(k_copy_d, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, s->x64, c, n);
     LSAMD_HIP(hipStreamSynchronize(st));
@@ -4852,8 +4969,12 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
     // FP64 outer refinement around FP32 inner PCG solves of N d = r.
     if (int rc = ensure_work(s, false)) return rc;
     if (int rc = ensure_work(s, true)) return rc;
-    if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
-    if (int rc = ensure_tuned<float>(s, s->p32, s->q32, st)) return rc;
+    if (timed) {
+      if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
+      if (int rc = ensure_tuned<float>(s, s->p32, s->q32, st)) return rc;
+    }
+    if (int rc = pcg_gram_ensure(s, st)) return rc;
+    if (int rc = pcg_buffer(s, &s->pcg_b32)) return rc;
     const double inner = o->inner_rtol > 0 ? o->inner_rtol : 1e-4;
     const int64_t max_outer = o->max_outer > 0 ? o->max_outer : 50;
     hipLaunchKernelGGL(k_zero_d, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, c, n);
@@ -4872,7 +4993,8 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
       const double irtol = inner;
       if (int rc = launch_init<float>(s, s->r64, minv32, s->x32, s->r32, irtol, 0.0, left, st))
         return rc;
-      if (int rc = run_pcg<float>(s, chunk, s->x32, s->r32, s->p32, s->q32, s->t32, minv32, st))
+      if (int rc = run_pcg<float>(s, chunk, s->x32, s->r32, s->p32, s->pcg_b32, s->q32, s->t32,
+                                  minv32, st))
         return rc;
       total += s->ctl_host->iter;
       ++outer;
@@ -5296,6 +5418,8 @@ int lsamd_batch_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const doubl
       inf[i].threshold = s->bctl_host[i].thr;
     }
   } else if (o->precision == LSAMD_FP32) {
+    if (int rc = pcg_gram_ensure(s, st)) return rc;
+    if (int rc = pcg_buffer(s, &s->pcg_b32)) return rc;
     const double inner = o->inner_rtol > 0 ? o->inner_rtol : 1e-4;
     const int64_t max_outer = o->max_outer > 0 ? o->max_outer : 50;
     hipLaunchKernelGGL(k_zero_d, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, c, n);
