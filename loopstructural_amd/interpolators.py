@@ -61,10 +61,12 @@ class InterpolatorType(Enum):
 
 
 class _Lazy:
-    """A ``constraints`` entry computed when it is first read."""
+    """A ``constraints`` entry computed when it is read; ``keep``: once, and
+    then the stored array.  ``uniform``: (value, count) of an entry that holds
+    one value, for readers that need no array."""
 
-    def __init__(self, fn):
-        self.fn = fn
+    def __init__(self, fn, keep=False, uniform=None):
+        self.fn, self.keep, self.uniform = fn, keep, uniform
 
 
 class _Constraint(dict):
@@ -82,7 +84,9 @@ class _Constraint(dict):
                 m = self._csc = v.to_scipy().tocsc()
             return m
         if isinstance(v, _Lazy):
-            v = v.fn()
+            lazy, v = v, v.fn()
+            if lazy.keep:
+                self[key] = v
         if isinstance(v, torch.Tensor):
             return v.detach().cpu().numpy()
         return v
@@ -93,6 +97,21 @@ class _Constraint(dict):
 
     def get(self, key, default=None):
         return self[key] if key in self else default
+
+
+def _weight_statistics(parts):
+    """Mean, least and largest weight of a family's parts: weight arrays, or
+    (value, count) where one value holds for all rows (the regulariser's
+    rows, several per node, whose arrays took a third of a P1 setup)."""
+    arrays = [p for p in parts if isinstance(p, np.ndarray)]
+    if len(arrays) == len(parts):
+        w = np.concatenate(arrays)
+        return float(np.mean(w)), float(np.min(w)), float(np.max(w))
+    same = [p for p in parts if not isinstance(p, np.ndarray)]
+    total = sum(float(np.sum(a)) for a in arrays) + sum(v * c for v, c in same)
+    count = sum(a.size for a in arrays) + sum(c for _, c in same)
+    values = [f(a) for a in arrays for f in (np.min, np.max)] + [v for v, _ in same]
+    return total / count, float(min(values)), float(max(values))
 
 
 class StencilFamily:
@@ -1107,6 +1126,11 @@ class DiscreteInterpolator(GeologicalInterpolator):
             fam = self._family_of(name)
             m = dict.__getitem__(con, "matrix")
             rows[fam] += int(m.shape[0])
+            w = dict.__getitem__(con, "w")
+            if isinstance(w, _Lazy) and w.uniform is not None:
+                if w.uniform[1]:
+                    wts[fam].append(w.uniform)
+                continue
             w = con["w"]
             if w is not None:
                 w = np.atleast_1d(np.asarray(w, dtype=float))
@@ -1124,8 +1148,7 @@ class DiscreteInterpolator(GeologicalInterpolator):
             elif fam == "gradient":
                 dropped = max(src * 2 - rc, 0)
             if wts.get(fam):
-                allw = np.concatenate(wts[fam])
-                mw, lo, hi = float(np.mean(allw)), float(np.min(allw)), float(np.max(allw))
+                mw, lo, hi = _weight_statistics(wts[fam])
             else:
                 mw = lo = hi = None
             fams[fam] = ConstraintFamilyDiagnostics(fam, rc > 0, rc, dropped, mw, lo, hi, src,
@@ -1458,8 +1481,9 @@ class FiniteDifferenceInterpolator(DiscreteInterpolator):
                 w = self.regularisation_scale[fam.centres()] * fam.weight
             return w
 
+        uniform = None if self.use_regularisation_weight_scale else (fam.weight, fam.nrows)
         self.constraints[fam.name] = _Constraint(matrix=fam, b=np.zeros(fam.nrows),
-                                                 w=_Lazy(weights))
+                                                 w=_Lazy(weights, uniform=uniform))
 
     def _reg_struct(self):
         r = _lib.FdReg()
@@ -1630,7 +1654,10 @@ class P1Interpolator(DiscreteInterpolator):
             name = self._unique_name(name)
             fam = EdgeJumpFamily(name, float(w), P, self.dof, grid)
             self._edge_families[name] = fam
-            self.constraints[name] = _Constraint(matrix=fam, b=np.zeros(P), w=np.full(P, float(w)))
+            # the solver needs the weight alone: 2e7 copies of it (128^3 cells)
+            # took 30 ms of a 160 ms solve
+            self.constraints[name] = _Constraint(matrix=fam, b=np.zeros(P), w=_Lazy(
+                lambda: np.full(P, float(w)), keep=True, uniform=(float(w), P)))
         self.up_to_date = False
 
     def get_regularisation_sample_points(self):
