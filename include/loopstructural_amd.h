@@ -102,10 +102,10 @@ typedef struct lsamd_solve_opts {
                            and max_outer unused; check_every capped at 8.
                            Environment: LSAMD_MG_SMOOTHER=jacobi for point
                            Jacobi, LSAMD_MG_DEGREE=1..8 for the Chebyshev
-                           degree of the coarse levels (4),
+                           degree of the coarse levels (3),
                            LSAMD_MG_DEGREE0 for the fine level's (2, at most
                            the coarse one), LSAMD_MR_DEGREE=1..8 for the
-                           coarse levels of the multi-rhs V-cycle (6),
+                           coarse levels of the multi-rhs V-cycle (4),
                            LSAMD_MG_TIMING=1 prints set-up
                            times, LSAMD_MR_COV_LANES=1|2|4|8 sets the
                            right-hand sides per thread of the multi-rhs

@@ -2065,14 +2065,20 @@ struct MgLevel {
 
 struct Mg {
   std::vector<MgLevel> lv;
-  int deg = 4;            // Chebyshev degree of the coarse levels
-  int deg0 = 2;           // Chebyshev degree of the fine level (<= deg)
+  // Chebyshev degrees of the coarse levels and of the fine one (<= deg).  A
+  // coarse step costs launches, a fine one traffic; ms per solve (iterations)
+  // at 2, 3 and 4 coarse steps, 2 fine: 128^3 nodes 41.5 (89), 38.2 (72), 40.3
+  // (63); 97 x 89 x 81 29.8 (84), 29.8 (67), 35.1 (65); 64^3 19.5 (83), 19.2
+  // (70), 22.1 (68); 38 x 56 x 43 16.2 (70), 17.6 (60), 18.4 (55).  One or
+  // three fine steps: 128^3 52.9 (113 with 3 coarse) and 49.9 (65 with 4).
+  int deg = 3;
+  int deg0 = 2;
   // coarse-level degree of the multi-rhs V-cycle: its fine level is HBM-bound
-  // over R lanes, so coarse steps are cheap against the iterations they save
-  // (at 128^3, 32 lanes: degree 4 101 iterations 757 ms per batch, 5 88 and
-  // 713, 6 80 and 708, 7 75 and 726); the single-system and batched solves,
-  // launch-bound, are fastest at 4
-  int deg_mr = 6;
+  // over R lanes, so a coarse step more is cheap against the iterations it
+  // saves.  ms per batch (iterations) at 3, 4, 5 and 6: 128^3 nodes, 64 lanes
+  // 930 (73), 906 (65), 914 (61), 948 (58); 16 lanes 266, 265, 271, 287; 65 x
+  // 61 x 57, 64 lanes 187 (76), 194 (71), 211 (69), 232 (69).
+  int deg_mr = 4;
   bool schwarz = true;    // Schwarz blocks in the smoother (else point Jacobi)
   bool stale = true;      // data rows changed: row-dependent parts to rebuild
   float* cinv = nullptr;  // dense inverse of the coarsest operator
@@ -2238,16 +2244,63 @@ MgSm mg_sm(const MgLevel& L) {
   return S;
 }
 
-// y = N x of a level in FP32: level 0 with its data rows, coarse levels in
-// one fused launch (regulariser stencil + Gram row per node)
+// y += the data term of x by node, one launch (level 0; gram_state == 1);
+// partials of x.Gx to part where given
+template <typename T>
+void launch_gram_add(const lsamd_fd_system* s, const T* x, T* y, double* part, const CgCtl* ctl,
+                     hipStream_t st) {
+  const GramDev G = gram_dev(s, sizeof(T) == 4);
+  const dim3 nb((unsigned)ceil_div(G.ndn * kGramLanes, 256));
+  if (s->gram_width == kGramCap / 2)
+    hipLaunchKernelGGL((k_gram_add<T, kGramCap / 2>), nb, dim3(256), 0, st, G, x, y, part, ctl);
+  else
+    hipLaunchKernelGGL((k_gram_add<T, kGramCap>), nb, dim3(256), 0, st, G, x, y, part, ctl);
+}
+
+// q = N x of a level that keeps q: level 0 (stencil, then its data term by
+// node or by rows) and large coarse levels (stencil and Gram row per node)
 void mg_level_apply(const MgLevel& L, const float* x, float* y, const CgCtl* ctl,
                     hipStream_t st) {
-  if (!L.owned) {
+  if (L.owned) {
+    hipLaunchKernelGGL(k_mg_apply, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st,
+                       mg_dev(L), x, y, ctl);
+  } else if (L.sys->gram_state == 1) {
+    launch_stencil<float>(L.sys, x, y, ctl, st, L.sys->zc[1]);
+    launch_gram_add<float>(L.sys, x, y, nullptr, ctl, st);
+  } else {
     mg_apply<float>(L.sys, x, y, ctl, st);
+  }
+}
+
+// Threads per node of a level's kernels (k_mg_resid, k_mg_smooth): as many as
+// leave the chip a few wavefronts per SIMD.  us per launch of the operator and
+// a smoothing step, one thread against these: 33^3 nodes 9.7 and 7.0 to 5.6
+// and 4.5 (8 threads), 17^3 10.0 and 7.3 to 4.2 and 3.7 (16), 9^3 8.9 and 7.1
+// to 3.7 and 3.0 (16); at 65^3 one thread is the fastest (a 128^3 solve takes
+// 39.5 ms, with two 40.5, with four 40.3).
+template <typename F>
+void mg_lanes(int64_t n, F&& launch) {
+  if (n >= 131072)
+    launch(std::integral_constant<int, 1>());
+  else if (n >= 16384)
+    launch(std::integral_constant<int, 8>());
+  else
+    launch(std::integral_constant<int, 16>());
+}
+
+// r = b - N x of a coarse level
+void mg_level_resid(const MgLevel& L, const CgCtl* ctl, hipStream_t st) {
+  const MgDev A = mg_dev(L);
+  if (!A.tab) {
+    hipLaunchKernelGGL(k_mg_resid_node, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st, A,
+                       (const float*)L.b, (const float*)L.x, L.q, ctl);
     return;
   }
-  hipLaunchKernelGGL(k_mg_apply, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st, mg_dev(L),
-                     x, y, ctl);
+  mg_lanes(L.n, [&](auto g) {
+    constexpr int G = decltype(g)::value;
+    hipLaunchKernelGGL(k_mg_resid<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0, st, A,
+                       (const float*)L.b, (const float*)L.x, L.q, ctl);
+  });
 }
 
 // FP64 level apply (setup: power iteration and the dense coarsest operator)
@@ -2708,9 +2761,6 @@ int mg_build_static(lsamd_fd_system* s, Mg* m, hipStream_t st) {
   if (int rc = mg_alloc(m, &m->scal, 2)) return rc;
   const char* sm_env = getenv("LSAMD_MG_SMOOTHER");
   m->schwarz = !(sm_env && strcmp(sm_env, "jacobi") == 0);
-  // degree 4 on the coarse levels, 2 on the fine one: at 128^3 96 outer
-  // iterations against 145 with degree 2 everywhere, and the coarse steps are
-  // cheap; fine-level steps cost HBM traffic
   if (const char* dg = getenv("LSAMD_MG_DEGREE")) m->deg = std::max(1, std::min(kMgDegMax, atoi(dg)));
   if (const char* dg = getenv("LSAMD_MG_DEGREE0")) m->deg0 = std::max(1, atoi(dg));
   m->deg0 = std::min(m->deg0, m->deg);
@@ -2972,59 +3022,85 @@ void mg_vcycle(Mg* m, int l, const CgCtl* ctl, hipStream_t st) {
                        (const float*)m->cinv, (const float*)L.b, L.x, m->nc, ctl);
     return;
   }
-  const dim3 nb((unsigned)ceil_div(L.n, 256));
   const MgSm S = mg_sm(L);
-  const int split = L.cov && L.n >= kSplitMin ? 1 : 0;
-  const dim3 ncb((unsigned)std::max<int64_t>(1, ceil_div(L.ncov, 256)));
-  auto smooth = [&](int from_zero) {
-    hipLaunchKernelGGL(k_mg_cheb_first, nb, dim3(256), 0, st, (const float*)L.b,
-                       (const float*)L.q, S, L.x, L.d, L.n, L.c0, from_zero, split, ctl);
-    const int deg = l == 0 ? m->deg0 : m->deg;
-    if (split && L.ncov > 0)
-      hipLaunchKernelGGL(k_mg_cheb_cov, ncb, dim3(256), 0, st, (const int32_t*)L.cov, L.ncov,
-                         (const float*)L.b, (const float*)L.q, S, L.x, L.d, from_zero ? 0 : 1,
-                         L.c0, 0.f, 0.f, 0, ctl);
-    for (int k = 1; k < deg; ++k) {
-      const int last = k == deg - 1;
+  // coarse levels hold the residual in L.q; level 0 (and a coarse level of
+  // its size) the product N x
+  const bool resid = l > 0 && L.n < kSplitMin;
+  const int split = !resid && L.cov && L.ncov > 0 ? 1 : 0;
+  const int ncb = split ? (int)ceil_div(L.ncov * kCovLanes, 256) : 0;
+  auto apply = [&]() {
+    if (resid)
+      mg_level_resid(L, ctl, st);
+    else
       mg_level_apply(L, L.x, L.q, ctl, st);
-      hipLaunchKernelGGL(k_mg_cheb_step, nb, dim3(256), 0, st, (const float*)L.b,
-                         (const float*)L.q, S, L.x, L.d, L.n, L.c1[k], L.c2[k], split, last, ctl);
-      if (split && L.ncov > 0)
-        hipLaunchKernelGGL(k_mg_cheb_cov, ncb, dim3(256), 0, st, (const int32_t*)L.cov, L.ncov,
-                           (const float*)L.b, (const float*)L.q, S, L.x, L.d, 2, 0.f, L.c1[k],
-                           L.c2[k], last, ctl);
+  };
+  auto step = [&](int mode, float c1, float c2, int last) {
+    if (resid)
+      mg_lanes(L.n, [&](auto g) {
+        constexpr int G = decltype(g)::value;
+        hipLaunchKernelGGL(k_mg_smooth<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0,
+                           st, (const float*)(mode == 0 ? L.b : L.q), S, L.x, L.d, L.n,
+                           mode == 2 ? c1 : 0.f, mode == 2 ? c2 : L.c0, mode == 0, last, ctl);
+      });
+    else
+      hipLaunchKernelGGL(k_mg_cheb, dim3((unsigned)(ncb + ceil_div(L.n, 256))), dim3(256), 0, st,
+                         (const int32_t*)L.cov, L.ncov, ncb, (const float*)L.b,
+                         (const float*)L.q, S, L.x, L.d, L.n, mode, L.c0, c1, c2, last, ctl);
+  };
+  auto smooth = [&](int from_zero) {
+    const int deg = l == 0 ? m->deg0 : m->deg;
+    step(from_zero ? 0 : 1, 0.f, 0.f, deg == 1);
+    for (int k = 1; k < deg; ++k) {
+      apply();
+      step(2, L.c1[k], L.c2[k], k == deg - 1);
     }
   };
   smooth(1);
-  mg_level_apply(L, L.x, L.q, ctl, st);
+  apply();
   MgLevel& C = m->lv[l + 1];
   hipLaunchKernelGGL(k_mg_restrict, dim3((unsigned)ceil_div(C.n, 256)), dim3(256), 0, st,
-                     (const float*)L.b, (const float*)L.q, L.g, C.b, C.g, ctl);
+                     (const float*)(resid ? L.q : L.b), (const float*)(resid ? nullptr : L.q), L.g,
+                     C.b, C.g, ctl);
   mg_vcycle(m, l + 1, ctl, st);
-  hipLaunchKernelGGL(k_mg_prolong, nb, dim3(256), 0, st, (const float*)C.x, C.g, L.x, L.g, ctl);
-  mg_level_apply(L, L.x, L.q, ctl, st);
+  hipLaunchKernelGGL(k_mg_prolong, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st,
+                     (const float*)C.x, C.g, L.x, L.g, ctl);
+  apply();
   smooth(0);
 }
 
 int launch_fcg_iteration(lsamd_fd_system* s, hipStream_t st) {
   Mg* m = s->mg;
   const int64_t n = s->n;
-  const int vb = vec_blocks(n);
+  const int vb = std::min(vec_blocks(n), kPcgBlocks / 2);
   MgLevel& L0 = m->lv[0];
   // L0.b holds (float) r: written by the previous update (or the set-up)
   mg_vcycle(m, 0, s->ctl, st);
   hipLaunchKernelGGL(k_fcg_dots, dim3(vb), dim3(256), 0, st, (const float*)L0.x,
-                     (const double*)s->r64, (const double*)m->rp64, n, s->part,
+                     (const double*)s->r64, (const double*)m->rp64, n, s->pcg_pr,
                      (const CgCtl*)s->ctl);
-  hipLaunchKernelGGL(k_fcg_dots_fin, dim3(1), dim3(256), 0, st, (const double*)s->part, vb,
-                     s->ctl);
   hipLaunchKernelGGL(k_fcg_dir, dim3(vb), dim3(256), 0, st, (const float*)L0.x, s->p64, n,
-                     (const CgCtl*)s->ctl);
-  if (int rc = launch_apply<double>(s, s->p64, s->q64, s->t64, s->ctl, st)) return rc;
+                     (const double*)s->pcg_pr, vb, s->ctl);
+  int64_t nq = -1;
+  int ng = 0;
+  if (s->gram_state == 1 || s->nrows == 0) {
+    nq = launch_stencil<double>(s, (const double*)s->p64, s->q64, s->ctl, st, s->zc[0]);
+    if (s->gram_state == 1) {
+      launch_gram_add<double>(s, (const double*)s->p64, s->q64, s->pcg_pg, s->ctl, st);
+      ng = (int)ceil_div(s->ndn * kGramLanes, 256);
+    }
+    if (nq + ng > 2 * kPcgPartMax) {
+      hipLaunchKernelGGL(k_fcg_alpha, dim3(1), dim3(256), 0, st, (const double*)s->part, (int)nq,
+                         (const double*)s->pcg_pg, ng, s->ctl);
+      nq = -1;
+    }
+  } else if (int rc = launch_apply<double>(s, s->p64, s->q64, s->t64, s->ctl, st)) {
+    return rc;
+  }
   hipLaunchKernelGGL(k_fcg_upd, dim3(vb), dim3(256), 0, st, s->x64, s->r64, m->rp64,
                      (const double*)s->p64, (const double*)s->q64, (const double*)s->minv64,
-                     L0.b, n, s->part, (const CgCtl*)s->ctl);
-  hipLaunchKernelGGL(k_fcg_upd_fin, dim3(1), dim3(256), 0, st, (const double*)s->part, vb,
+                     L0.b, n, (const double*)s->part, (int)nq, (const double*)s->pcg_pg, ng,
+                     s->pcg_pr, (const CgCtl*)s->ctl);
+  hipLaunchKernelGGL(k_fcg_upd_fin, dim3(1), dim3(256), 0, st, (const double*)s->pcg_pr, vb,
                      s->ctl);
   LSAMD_CHECK_LAUNCH("multigrid PCG iteration");
   return LSAMD_OK;
@@ -3101,6 +3177,7 @@ int mg_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const double* b, dou
              lsamd_solve_info* inf, hipStream_t st) {
   if (s->op != 0) return fail(LSAMD_ERR_ARG, "multigrid is available for FD systems only");
   if (int rc = mg_ensure(s, st)) return rc;
+  if (int rc = pcg_gram_ensure(s, st)) return rc;
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : 10 * n;
   const int maxiter = (int)std::min<int64_t>(maxiter64, 2000000000LL);

@@ -20,7 +20,7 @@
 // against 65, 72 x 69 x 109 with 367 values 85 against 62, 24 x 24 x 36 80
 // against 63, over 48 systems of 32^3..96^3 at most 139 against 101.
 // The coarsest level (<= 5 nodes per axis) is solved with a dense inverse.
-// Smoother: Chebyshev polynomial (degree 2 on the fine level, 4 on the
+// Smoother: Chebyshev polynomial (degree 2 on the fine level, 3 on the
 // coarse ones) in M N on
 // [lambda_max/30, 1.15 lambda_max], lambda_max by power iteration, with M
 // additive Schwarz: the exact inverse of N on each block, summed over
@@ -85,45 +85,60 @@ __device__ inline float mg_precond(int64_t i, const MgSm& S, const float* __rest
   return acc;
 }
 
-// skip_cov: leave the covered nodes to k_mg_cheb_cov (large levels, where
-// their gathers would stall every wavefront that holds one)
-__global__ void k_mg_cheb_first(const float* __restrict__ b, const float* __restrict__ q,
-                                MgSm S, float* __restrict__ x, float* __restrict__ d, int64_t n,
-                                float c0, int from_zero, int skip_cov, const CgCtl* ctl) {
-  if (ctl->done) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (skip_cov && S.sm[i] < 0.f) return;
-  const float dv = c0 * mg_precond(i, S, b, q, from_zero);
-  d[i] = dv;
-  x[i] = from_zero ? dv : x[i] + dv;
-}
-
-// later steps: d = c1 d + c2 M (b - q), x += d; last: the smoothing's final
-// step, whose d is dead and not stored
-__global__ void k_mg_cheb_step(const float* __restrict__ b, const float* __restrict__ q,
-                               MgSm S, float* __restrict__ x, float* __restrict__ d, int64_t n,
-                               float c1, float c2, int skip_cov, int last, const CgCtl* ctl) {
-  if (ctl->done) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  if (skip_cov && S.sm[i] < 0.f) return;
-  const float dv = c1 * d[i] + c2 * mg_precond(i, S, b, q, 0);
-  if (!last) d[i] = dv;
-  x[i] += dv;
-}
-
-// the covered nodes of a level (compact list): mode 0 first step from zero,
-// 1 first step, 2 later step (d = c1 d + c2 M r); last as k_mg_cheb_step
-__global__ void k_mg_cheb_cov(const int32_t* __restrict__ cov, int64_t ncov,
-                              const float* __restrict__ b, const float* __restrict__ q, MgSm S,
-                              float* __restrict__ x, float* __restrict__ d, int mode, float c0,
-                              float c1, float c2, int last, const CgCtl* ctl) {
-  if (ctl->done) return;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ncov) return;
-  const int64_t i = cov[t];
-  const float z = mg_precond(i, S, b, q, mode == 0);
+// Chebyshev step of a level that keeps q = N x: mode 0 first step from zero
+// (d = c0 M b, x = d), 1 first step (d = c0 M (b - q), x += d), 2 later step
+// (d = c1 d + c2 M (b - q), x += d); last: the smoothing's final step, whose
+// d is dead and not stored.
+//
+// Workgroups [0, ncb): the covered nodes (compact list, where the level has
+// one), kCovLanes threads per row of block inverses, whose gathers would
+// otherwise stall every wavefront that holds one; the rest: the other nodes
+// (every node on a level without a list).  One launch for both: at 128^3 the
+// two took 10.4 and 15.4 us one after the other.
+constexpr int kCovLanes = 4;
+__global__ __launch_bounds__(256) void k_mg_cheb(const int32_t* __restrict__ cov, int64_t ncov,
+                                                 int ncb, const float* __restrict__ b,
+                                                 const float* __restrict__ q, MgSm S,
+                                                 float* __restrict__ x, float* __restrict__ d,
+                                                 int64_t n, int mode, float c0, float c1, float c2,
+                                                 int last, const CgCtl* ctl) {
+  const int done = ctl->done;
+  int64_t i;
+  float z;
+  if ((int)blockIdx.x < ncb) {
+    const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (th / kCovLanes >= ncov) return;  // whole groups
+    i = cov[th / kCovLanes];
+    const int64_t e1 = S.sptr[i + 1];
+    z = 0.f;
+    for (int64_t e = S.sptr[i] + th % kCovLanes; e < e1; e += 4 * kCovLanes) {
+      int32_t c[4];
+      float a[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const bool ok = e + k * kCovLanes < e1;
+        const int64_t at = ok ? e + k * kCovLanes : e;
+        c[k] = S.scol[at];
+        a[k] = ok ? S.sval[at] : 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) z += a[k] * mg_r(b, q, c[k], mode == 0);
+    }
+#pragma unroll
+    for (int o = kCovLanes / 2; o > 0; o >>= 1) z += __shfl_xor(z, o, 64);
+    if (th % kCovLanes != 0) return;
+  } else {
+    i = (int64_t)(blockIdx.x - ncb) * 256 + threadIdx.x;
+    if (i >= n) return;
+    if (ncb > 0) {
+      const float t = S.sm[i];
+      if (t < 0.f) return;
+      z = t * mg_r(b, q, i, mode == 0);
+    } else {
+      z = mg_precond(i, S, b, q, mode == 0);
+    }
+  }
+  if (done) return;
   const float dv = mode == 2 ? c1 * d[i] + c2 * z : c0 * z;
   if (!last) d[i] = dv;
   x[i] = mode == 0 ? dv : x[i] + dv;
@@ -137,69 +152,69 @@ __host__ __device__ inline void mg_ijk(int64_t id, int nx, int ny, int& i, int& 
   i = (int)(r - (int64_t)j * nx);
 }
 
-// bc = P^T (bf - qf): per coarse node, the fine nodes 2J-1, 2J, 2J+1 per axis
-// with weights 1/2, 1, 1/2 (those inside the fine grid)
-// P^T (bf - qf) at coarse node id: the fine nodes 2J-1, 2J, 2J+1 per axis
-// with weights 1/2, 1, 1/2 (those inside the fine grid)
+// P^T r at coarse node id, r = bf - qf (qf == nullptr: r = bf): the fine
+// nodes 2J-1, 2J, 2J+1 per axis with weights 1/2, 1, 1/2 (those inside the
+// fine grid).  All 27 loads are issued at once, those outside the grid from
+// the centre with weight 0: a load behind a branch waits for the one before.
 __device__ inline float mg_restrict_node(const float* __restrict__ bf,
                                          const float* __restrict__ qf, const GridDev& gf,
                                          const GridDev& gc, int64_t id) {
   int I, J, K;
   mg_ijk(id, gc.nx, gc.ny, I, J, K);
   const int64_t fnxy = (int64_t)gf.nx * gf.ny;
-  float acc = 0.f;
-  for (int dk = -1; dk <= 1; ++dk) {
-    const int k = 2 * K + dk;
-    if (k < 0 || k >= gf.nz) continue;
-    const float wk = dk == 0 ? 1.f : 0.5f;
-    for (int dj = -1; dj <= 1; ++dj) {
-      const int j = 2 * J + dj;
-      if (j < 0 || j >= gf.ny) continue;
-      const float wj = wk * (dj == 0 ? 1.f : 0.5f);
-      for (int di = -1; di <= 1; ++di) {
-        const int i = 2 * I + di;
-        if (i < 0 || i >= gf.nx) continue;
-        const float w = wj * (di == 0 ? 1.f : 0.5f);
-        const int64_t f = (int64_t)i + (int64_t)j * gf.nx + (int64_t)k * fnxy;
-        acc += w * (bf[f] - qf[f]);
-      }
-    }
+  float v[27];
+#pragma unroll
+  for (int t = 0; t < 27; ++t) {
+    const int di = t % 3 - 1, dj = t / 3 % 3 - 1, dk = t / 9 - 1;
+    const int i = 2 * I + di, j = 2 * J + dj, k = 2 * K + dk;
+    const bool ok = (unsigned)i < (unsigned)gf.nx && (unsigned)j < (unsigned)gf.ny &&
+                    (unsigned)k < (unsigned)gf.nz;
+    const int64_t f = ok ? (int64_t)i + (int64_t)j * gf.nx + (int64_t)k * fnxy : 0;
+    const float r = qf ? bf[f] - qf[f] : bf[f];
+    v[t] = ok ? r : 0.f;
   }
+  float acc = 0.f;
+#pragma unroll
+  for (int t = 0; t < 27; ++t)
+    acc += (t % 3 == 1 ? 1.f : 0.5f) * (t / 3 % 3 == 1 ? 1.f : 0.5f) * (t / 9 == 1 ? 1.f : 0.5f) *
+           v[t];
   return acc;
 }
 
-// (P xc) at fine node id: trilinear, coarse node c = fine node 2c
+// (P xc) at fine node id: trilinear, coarse node c = fine node 2c; eight
+// loads at once, weight 0 where an even index needs one neighbour only
 __device__ inline float mg_prolong_node(const float* __restrict__ xc, const GridDev& gc,
                                         const GridDev& gf, int64_t id) {
   int i, j, k;
   mg_ijk(id, gf.nx, gf.ny, i, j, k);
-  const int i0 = i >> 1, j0 = j >> 1, k0 = k >> 1;
-  const int ni = (i & 1) ? 2 : 1, nj = (j & 1) ? 2 : 1, nk = (k & 1) ? 2 : 1;
-  const float wi = ni == 2 ? 0.5f : 1.f, wj = nj == 2 ? 0.5f : 1.f, wk = nk == 2 ? 0.5f : 1.f;
+  const int oi = i & 1, oj = j & 1, ok = k & 1;
   const int64_t cnxy = (int64_t)gc.nx * gc.ny;
-  float acc = 0.f;
-  for (int c = 0; c < nk; ++c)
-    for (int b = 0; b < nj; ++b)
-      for (int a = 0; a < ni; ++a)
-        acc += xc[(int64_t)(i0 + a) + (int64_t)(j0 + b) * gc.nx + (int64_t)(k0 + c) * cnxy];
-  return wi * wj * wk * acc;
+  const float* c = xc + (i >> 1) + (int64_t)(j >> 1) * gc.nx + (int64_t)(k >> 1) * cnxy;
+  float v[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+    v[t] = c[(t & 1) * oi + (int64_t)((t >> 1) & 1) * oj * gc.nx + (int64_t)(t >> 2) * ok * cnxy];
+  // an even index has both its neighbours at the same node, half each
+  return 0.125f * (((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7])));
 }
 
 __global__ void k_mg_restrict(const float* __restrict__ bf, const float* __restrict__ qf,
                               GridDev gf, float* __restrict__ bc, GridDev gc, const CgCtl* ctl) {
-  if (ctl->done) return;
   const int64_t nc = (int64_t)gc.nx * gc.ny * gc.nz;
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= nc) return;
-  bc[id] = mg_restrict_node(bf, qf, gf, gc, id);
+  const int done = ctl->done;
+  const float v = mg_restrict_node(bf, qf, gf, gc, id);
+  if (!done) bc[id] = v;
 }
 __global__ void k_mg_prolong(const float* __restrict__ xc, GridDev gc, float* __restrict__ xf,
                              GridDev gf, const CgCtl* ctl) {
-  if (ctl->done) return;
   const int64_t nf = (int64_t)gf.nx * gf.ny * gf.nz;
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= nf) return;
-  xf[id] += mg_prolong_node(xc, gc, gf, id);
+  const int done = ctl->done;
+  const float v = xf[id] + mg_prolong_node(xc, gc, gf, id);
+  if (!done) xf[id] = v;
 }
 
 __global__ __launch_bounds__(64) void k_mg_dense(const float* __restrict__ cinv,
@@ -411,7 +426,7 @@ __global__ void k_iota_rows(int64_t* __restrict__ rptr, int64_t n, int64_t wc) {
 }
 
 // ------------------------------------------------------ flexible PCG ----
-// partials of z.r, z.r_prev (z: the FP32 V-cycle output, widened)
+// partials of z.r, then those of z.r_prev (z: the FP32 V-cycle output, widened)
 __global__ __launch_bounds__(256) void k_fcg_dots(const float* __restrict__ z,
                                                   const double* __restrict__ r,
                                                   const double* __restrict__ rp, int64_t n,
@@ -419,72 +434,143 @@ __global__ __launch_bounds__(256) void k_fcg_dots(const float* __restrict__ z,
   if (ctl->done) return;
   __shared__ double sh[4];
   double a = 0.0, b = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    const double zi = (double)z[i];
-    a += zi * r[i];
-    b += zi * rp[i];
+  for (int64_t i = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < n;
+       i += (int64_t)gridDim.x * 512) {
+    float zv[2];
+    double rv[2], pv[2];
+    pcg_ld<float, 2>(z, i, n, zv);
+    pcg_ld<double, 2>(r, i, n, rv);
+    pcg_ld<double, 2>(rp, i, n, pv);
+    a += (double)zv[0] * rv[0] + (double)zv[1] * rv[1];
+    b += (double)zv[0] * pv[0] + (double)zv[1] * pv[1];
   }
   const double sa = block_sum(a, sh);
   const double sb = block_sum(b, sh);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = sa;
-    part[2 * blockIdx.x + 1] = sb;
+    part[blockIdx.x] = sa;
+    part[gridDim.x + blockIdx.x] = sb;
   }
 }
 
-// one block: rho = z.r; beta = (z.r - z.r_prev) / rho_prev (0 on the first step)
-__global__ __launch_bounds__(256) void k_fcg_dots_fin(const double* __restrict__ part, int np,
-                                                      CgCtl* ctl) {
-  if (ctl->done) return;
+// p = z + beta p, beta = (z.r - z.r_prev) / rho_prev (0 on the first step):
+// every workgroup sums the np pairs of partials, workgroup 0 records rho = z.r
+__global__ __launch_bounds__(256) void k_fcg_dir(const float* __restrict__ z,
+                                                 double* __restrict__ p, int64_t n,
+                                                 const double* __restrict__ part, int np,
+                                                 CgCtl* ctl) {
   __shared__ double sh[4];
-  double a = 0.0, b = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) {
-    a += part[2 * i];
-    b += part[2 * i + 1];
-  }
-  const double sa = block_sum(a, sh);
-  const double sb = block_sum(b, sh);
-  if (threadIdx.x == 0) {
-    const double beta = ctl->iter == 0 ? 0.0 : (sa - sb) / ctl->rho_prev;
-    ctl->rho = sa;
-    ctl->acc = beta;
+  const int done = ctl->done, first = ctl->iter == 0;
+  const double prev = ctl->rho_prev;
+  const double zr = pcg_total(part, np, sh);
+  const double zp = pcg_total(part + np, np, sh);
+  if (done) return;
+  const double beta = first ? 0.0 : (zr - zp) / prev;
+  if (blockIdx.x == 0 && threadIdx.x == 0) ctl->rho = zr;
+  for (int64_t i = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < n;
+       i += (int64_t)gridDim.x * 512) {
+    float zv[2];
+    double pv[2];
+    pcg_ld<float, 2>(z, i, n, zv);
+    pcg_ld<double, 2>(p, i, n, pv);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) pv[k] = first ? (double)zv[k] : (double)zv[k] + beta * pv[k];
+    pcg_st<double, 2>(p, i, n, pv);
   }
 }
 
-// p = z + beta p
-__global__ void k_fcg_dir(const float* __restrict__ z, double* __restrict__ p, int64_t n,
-                          const CgCtl* ctl) {
-  if (ctl->done) return;
-  const double beta = ctl->acc;
-  const int first = ctl->iter == 0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
-    p[i] = first ? (double)z[i] : (double)z[i] + beta * p[i];
+// y += the data term of x (rows by node, see pcg.hpp); partials of x.Gx
+// where part is given
+template <typename T, int W>
+__global__ __launch_bounds__(256) void k_gram_add(GramDev G, const T* __restrict__ x,
+                                                  T* __restrict__ y, double* __restrict__ part,
+                                                  const CgCtl* ctl) {
+  __shared__ double sh[4];
+  constexpr int kE = W / kGramLanes;
+  typedef int32_t cols_t __attribute__((ext_vector_type(kE)));
+  const int done = ctl->done;
+  const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t d = th / kGramLanes;
+  double dot = 0.0;
+  if (d < G.ndn) {  // whole groups
+    const int64_t e = d * W + (th % kGramLanes) * kE;
+    const cols_t c = *(const cols_t*)(G.col + e);
+    const T* val = (const T*)G.val + e;
+    const int32_t i = G.node[d];
+    const T xi = x[i], yi = y[i];
+    T acc = 0;
+#pragma unroll
+    for (int k = 0; k < kE; ++k) acc += val[k] * x[c[k]];
+#pragma unroll
+    for (int o = kGramLanes / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    if (th % kGramLanes == 0 && !done) {
+      y[i] = yi + acc;
+      dot = (double)xi * (double)acc;
+    }
+  }
+  if (!part) return;
+  const double bs = block_sum(dot, sh);
+  if (threadIdx.x == 0) part[blockIdx.x] = bs;
 }
 
 // x += alpha p ; r_prev = r ; r -= alpha q ; rf = (float) r, the next
-// V-cycle's input ; partials of r.(minv r)
+// V-cycle's input ; partials of r.(minv r).  alpha = rho / p.q from the
+// operator's partials, or from ctl (nq < 0).
 __global__ __launch_bounds__(256) void k_fcg_upd(double* __restrict__ x, double* __restrict__ r,
                                                  double* __restrict__ rp,
                                                  const double* __restrict__ p,
                                                  const double* __restrict__ q,
                                                  const double* __restrict__ minv,
                                                  float* __restrict__ rf, int64_t n,
+                                                 const double* __restrict__ part_q, int nq,
+                                                 const double* __restrict__ part_g, int ng,
                                                  double* __restrict__ part, const CgCtl* ctl) {
-  if (ctl->done) return;
   __shared__ double sh[4];
-  const double alpha = ctl->alpha;
+  const int done = ctl->done;
+  const double rho = ctl->rho;
+  double alpha;
+  if (nq < 0) {
+    alpha = ctl->alpha;
+  } else {
+    double pq = pcg_total(part_q, nq, sh);
+    if (ng > 0) pq += pcg_total(part_g, ng, sh);
+    alpha = rho / pq;
+  }
+  if (done) return;
   double acc = 0.0;
-  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    x[i] += alpha * p[i];
-    const double rv = r[i];
-    rp[i] = rv;
-    const double rn = rv - alpha * q[i];
-    r[i] = rn;
-    rf[i] = (float)rn;
-    acc += rn * (minv[i] * rn);
+  for (int64_t i = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x); i < n;
+       i += (int64_t)gridDim.x * 512) {
+    double xv[2], rv[2], pv[2], qv[2], mv[2];
+    float fv[2];
+    pcg_ld<double, 2>(x, i, n, xv);
+    pcg_ld<double, 2>(p, i, n, pv);
+    pcg_ld<double, 2>(r, i, n, rv);
+    pcg_ld<double, 2>(q, i, n, qv);
+    pcg_ld<double, 2>(minv, i, n, mv);
+    pcg_st<double, 2>(rp, i, n, rv);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      xv[k] += alpha * pv[k];
+      rv[k] -= alpha * qv[k];
+      fv[k] = (float)rv[k];
+      acc += rv[k] * (mv[k] * rv[k]);
+    }
+    pcg_st<double, 2>(x, i, n, xv);
+    pcg_st<double, 2>(r, i, n, rv);
+    pcg_st<float, 2>(rf, i, n, fv);
   }
   const double bs = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = bs;
+}
+
+// one workgroup: alpha = rho / p.q where its partials are many
+__global__ __launch_bounds__(256) void k_fcg_alpha(const double* __restrict__ part_q, int nq,
+                                                   const double* __restrict__ part_g, int ng,
+                                                   CgCtl* ctl) {
+  if (ctl->done) return;
+  __shared__ double sh[4];
+  double pq = pcg_total(part_q, nq, sh);
+  if (ng > 0) pq += pcg_total(part_g, ng, sh);
+  if (threadIdx.x == 0) ctl->alpha = ctl->rho / pq;
 }
 
 // one block: rho_prev = rho ; iter++ ; stopping test on |S r|
@@ -558,6 +644,121 @@ __global__ __launch_bounds__(256) void k_mg_apply(MgDev L, const float* __restri
   if (ctl->done) return;
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id < L.n) y[id] = mg_apply_node(L, x, id);
+}
+
+// Coarse levels, G neighbouring threads per node.  These levels are bound by
+// the chain of dependent loads (row pointer, columns, gathers) and by a row's
+// length, not by bytes: one thread per row took 8.9 us for the operator and 7
+// us for a smoothing step on 9^3 nodes, hardly less than on 33^3.  With G
+// threads a row's entries are loaded at once and contiguously, the pointer
+// travels beside the stencil's loads, and the solve's state is looked at last.
+// The operator leaves the residual r = b - N x, so that a smoothing step
+// gathers one vector.
+
+// taps 0..24 as kBTap, packed (dx + 2) | (dy + 2) << 4 | (dz + 2) << 8; the
+// rest: no tap
+__constant__ int kTapPack[32] = {
+    0x222, 0x223, 0x221, 0x232, 0x212, 0x224, 0x220, 0x242, 0x202, 0x244, 0x240,
+    0x204, 0x200, 0x122, 0x322, 0x022, 0x024, 0x020, 0x042, 0x002, 0x422, 0x424,
+    0x420, 0x442, 0x402, -1,    -1,    -1,    -1,    -1,    -1,    -1};
+
+// sum of val[e] v[col[e]] over a row's entries, this thread's share
+template <int G>
+__device__ inline float mg_row_share(const int64_t* __restrict__ ptr,
+                                     const int32_t* __restrict__ col,
+                                     const float* __restrict__ val, const float* __restrict__ v,
+                                     int64_t i, int l) {
+  const int64_t e1 = ptr[i + 1];
+  float acc = 0.f;
+  for (int64_t e = ptr[i] + l; e < e1; e += 4 * G) {
+    int32_t c[4];
+    float a[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool ok = e + k * G < e1;
+      const int64_t at = ok ? e + k * G : e;
+      c[k] = col[at];
+      a[k] = ok ? val[at] : 0.f;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) acc += a[k] * v[c[k]];
+  }
+  return acc;
+}
+
+template <int G>
+__device__ inline float mg_lane_sum(float v) {
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// r = b - N x of a level with a class table
+template <int G>
+__global__ __launch_bounds__(256) void k_mg_resid(MgDev L, const float* __restrict__ b,
+                                                  const float* __restrict__ x,
+                                                  float* __restrict__ r, const CgCtl* ctl) {
+  const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t id = th / G;
+  const int l = (int)(th % G);
+  if (id >= L.n) return;  // whole groups
+  const int done = ctl->done;
+  int i, j, k;
+  mg_ijk(id, L.g.nx, L.g.ny, i, j, k);
+  const int nx = L.g.nx, ny = L.g.ny, nz = L.g.nz;
+  const int64_t nxy = (int64_t)nx * ny;
+  const float* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
+  const float bv = b[id];
+  constexpr int kT = (kTaps + G - 1) / G;
+  float cv[kT], xv[kT];
+#pragma unroll
+  for (int q = 0; q < kT; ++q) {
+    const int t = l + q * G;
+    const int p = kTapPack[t < 32 ? t : 31];
+    const int dx = (p & 15) - 2, dy = ((p >> 4) & 15) - 2, dz = ((p >> 8) & 15) - 2;
+    const bool ok = t < kTaps && (unsigned)(i + dx) < (unsigned)nx &&
+                    (unsigned)(j + dy) < (unsigned)ny && (unsigned)(k + dz) < (unsigned)nz;
+    cv[q] = ok ? c[t] : 0.f;
+    xv[q] = x[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
+  }
+  float acc = L.gptr ? mg_row_share<G>(L.gptr, L.gcol, L.gval, x, id, l) : 0.f;
+#pragma unroll
+  for (int q = 0; q < kT; ++q) acc += cv[q] * xv[q];
+  acc = mg_lane_sum<G>(acc);
+  if (l == 0 && !done) r[id] = bv - acc;
+}
+
+// the same where no class table applies, one node per thread
+__global__ __launch_bounds__(256) void k_mg_resid_node(MgDev L, const float* __restrict__ b,
+                                                       const float* __restrict__ x,
+                                                       float* __restrict__ r, const CgCtl* ctl) {
+  if (ctl->done) return;
+  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (id < L.n) r[id] = b[id] - mg_apply_node(L, x, id);
+}
+
+// smoothing step from the residual r: dv = c1 d + c2 M r (c1 = 0: d is not
+// read); x = dv (from_zero) or x += dv; d = dv unless it is dead (last)
+template <int G>
+__global__ __launch_bounds__(256) void k_mg_smooth(const float* __restrict__ r, MgSm S,
+                                                   float* __restrict__ x, float* __restrict__ d,
+                                                   int64_t n, float c1, float c2, int from_zero,
+                                                   int last, const CgCtl* ctl) {
+  const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = th / G;
+  const int l = (int)(th % G);
+  if (i >= n) return;  // whole groups
+  const int done = ctl->done;
+  const float t = S.sm[i], rv = r[i];
+  const float xv = from_zero ? 0.f : x[i], dv0 = c1 != 0.f ? d[i] : 0.f;
+  float z = 0.f;
+  if (S.sptr) z = mg_row_share<G>(S.sptr, S.scol, S.sval, r, i, l);
+  z = mg_lane_sum<G>(z);
+  if (t >= 0.f) z = t * rv;
+  const float dv = c1 * dv0 + c2 * z;
+  if (l != 0 || done) return;
+  if (!last) d[i] = dv;
+  x[i] = xv + dv;
 }
 
 constexpr int64_t kSplitMin = 1 << 20;  // levels this large smooth covered nodes apart
