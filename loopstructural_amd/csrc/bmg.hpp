@@ -33,6 +33,8 @@ struct BmgLevel {
   int nc;
   const int32_t* g0list;  // level 0: the nodes with a nonempty Gram row
   int64_t g0n;
+  const int32_t* cov;  // level 0: the nodes that Schwarz blocks cover
+  int64_t ncov;
 };
 
 // one system's outer iteration (FP64 on level 0)
@@ -83,30 +85,55 @@ __device__ inline double bmg_apply64(const BmgSys& S, const double* __restrict__
   return acc;
 }
 
-// Chebyshev step of the smoother on the blocks of one level.  mode 0: first
-// step from zero (d = c0 M b, x = d); 1: first step (d = c0 M (b - q),
-// x += d); 2: step k (d = c1[k] d + c2[k] M (b - q), x += d; d not stored
-// on the last step).
+// Chebyshev step of the smoother on level 0, which keeps q = N x.  mode 0:
+// first step from zero (d = c0 M b, x = d); 1: first step (d = c0 M (b - q),
+// x += d); 2: step k (d = c1[k] d + c2[k] M (b - q), x += d; d not stored on
+// the last step).  Blocks y < 0: 256 / kCovLanes covered nodes of the
+// system's list (block -1 - y), kCovLanes threads each; y >= 0: 256 nodes, the
+// covered ones skipped where the system has a list (as k_mg_cheb).
 __global__ __launch_bounds__(256) void k_bmg_cheb(const BmgLevel* __restrict__ lv,
                                                   const int2* __restrict__ blk, int mode, int k,
                                                   int last, const CgCtl* __restrict__ ctl) {
   const int2 t = blk[blockIdx.x];
   if (ctl[t.x].done) return;
   const BmgLevel& L = lv[t.x];
-  const int64_t i = (int64_t)t.y * 256 + threadIdx.x;
-  if (i >= L.A.n) return;
-  if (mode == 2) {
-    const float dv = L.c1[k] * L.d[i] + L.c2[k] * mg_precond(i, L.S, L.b, L.q, 0);
-    if (!last) L.d[i] = dv;
-    L.x[i] += dv;
+  int64_t i;
+  float z;
+  if (t.y < 0) {
+    const int64_t th = (int64_t)(-1 - t.y) * 256 + threadIdx.x;
+    if (th / kCovLanes >= L.ncov) return;  // whole groups
+    i = L.cov[th / kCovLanes];
+    const int64_t e1 = L.S.sptr[i + 1];
+    z = 0.f;
+    for (int64_t e = L.S.sptr[i] + th % kCovLanes; e < e1; e += 4 * kCovLanes) {
+      int32_t c[4];
+      float a[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const bool ok = e + q * kCovLanes < e1;
+        const int64_t at = ok ? e + q * kCovLanes : e;
+        c[q] = L.S.scol[at];
+        a[q] = ok ? L.S.sval[at] : 0.f;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) z += a[q] * mg_r(L.b, L.q, c[q], mode == 0);
+    }
+    z = mg_lane_sum<kCovLanes>(z);
+    if (th % kCovLanes != 0) return;
   } else {
-    const float dv = L.c0 * mg_precond(i, L.S, L.b, L.q, mode == 0);
-    L.d[i] = dv;
-    L.x[i] = mode == 0 ? dv : L.x[i] + dv;
+    i = (int64_t)t.y * 256 + threadIdx.x;
+    if (i >= L.A.n) return;
+    const float tag = L.S.sm[i];
+    if (tag < 0.f && L.cov) return;
+    z = tag >= 0.f ? tag * mg_r(L.b, L.q, i, mode == 0)
+                   : mg_precond(i, L.S, L.b, L.q, mode == 0);
   }
+  const float dv = mode == 2 ? L.c1[k] * L.d[i] + L.c2[k] * z : L.c0 * z;
+  if (!last) L.d[i] = dv;
+  L.x[i] = mode == 0 ? dv : L.x[i] + dv;
 }
 
-// q = N x of one level (FP32)
+// q = N x of level 0, node by node (FP32)
 __global__ __launch_bounds__(256) void k_bmg_apply(const BmgLevel* __restrict__ lv,
                                                    const int2* __restrict__ blk,
                                                    const CgCtl* __restrict__ ctl) {
@@ -117,17 +144,54 @@ __global__ __launch_bounds__(256) void k_bmg_apply(const BmgLevel* __restrict__ 
   if (i < L.A.n) L.q[i] = mg_apply_node(L.A, L.x, i);
 }
 
-// coarse b = P^T (b - q) of the fine level (blocks of the coarse level)
+// Coarse levels, G threads per node (blocks of 256 / G nodes), the residual in
+// q, as k_mg_resid and k_mg_smooth; G by the level's nodes over all systems.
+template <int G>
+__global__ __launch_bounds__(256) void k_bmg_resid(const BmgLevel* __restrict__ lv,
+                                                   const int2* __restrict__ blk,
+                                                   const CgCtl* __restrict__ ctl) {
+  const int2 t = blk[blockIdx.x];
+  if (ctl[t.x].done) return;
+  const BmgLevel& L = lv[t.x];
+  const int64_t i = (int64_t)t.y * (256 / G) + threadIdx.x / G;
+  const int l = threadIdx.x % G;
+  if (i >= L.A.n) return;  // whole groups
+  const float bv = L.b[i];
+  const float v = mg_product<G>(L.A, L.x, i, l);
+  if (l == 0) L.q[i] = bv - v;
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void k_bmg_smooth(const BmgLevel* __restrict__ lv,
+                                                    const int2* __restrict__ blk, int mode, int k,
+                                                    int last, const CgCtl* __restrict__ ctl) {
+  const int2 t = blk[blockIdx.x];
+  if (ctl[t.x].done) return;
+  const BmgLevel& L = lv[t.x];
+  const int64_t i = (int64_t)t.y * (256 / G) + threadIdx.x / G;
+  const int l = threadIdx.x % G;
+  if (i >= L.A.n) return;  // whole groups
+  const float xv = mode == 0 ? 0.f : L.x[i], dv0 = mode == 2 ? L.d[i] : 0.f;
+  const float z = mg_smoothed<G>(L.S, mode == 0 ? L.b : L.q, i, l);
+  const float dv = mode == 2 ? L.c1[k] * dv0 + L.c2[k] * z : L.c0 * z;
+  if (l != 0) return;
+  if (!last) L.d[i] = dv;
+  L.x[i] = xv + dv;
+}
+
+// coarse b = P^T r of the fine level (blocks of the coarse level): r = b - q
+// on level 0, q on the others
 __global__ __launch_bounds__(256) void k_bmg_restrict(const BmgLevel* __restrict__ fine,
                                                       const BmgLevel* __restrict__ coarse,
-                                                      const int2* __restrict__ blk,
+                                                      const int2* __restrict__ blk, int level0,
                                                       const CgCtl* __restrict__ ctl) {
   const int2 t = blk[blockIdx.x];
   if (ctl[t.x].done) return;
   const BmgLevel& F = fine[t.x];
   const BmgLevel& C = coarse[t.x];
   const int64_t i = (int64_t)t.y * 256 + threadIdx.x;
-  if (i < C.A.n) C.b[i] = mg_restrict_node(F.b, F.q, F.A.g, C.A.g, i);
+  if (i < C.A.n)
+    C.b[i] = mg_restrict_node(level0 ? F.b : F.q, level0 ? F.q : nullptr, F.A.g, C.A.g, i);
 }
 
 // fine x += P (coarse x) (blocks of the fine level)
@@ -287,23 +351,22 @@ __global__ __launch_bounds__(256) void k_bmg_apply64(const BmgSys* __restrict__ 
   if (threadIdx.x == 0) part[blockIdx.x] = bs;
 }
 
-// per system: alpha = rho / p.q
 // level 0 after the plane-streaming stencil: y += G0 x (the data Gram rows,
-// FP32) over the listed nodes of the smoothed systems (blocks of 256 list
-// entries)
+// FP32) over the listed nodes of the smoothed systems (blocks of 256 /
+// kG0Lanes list entries, kG0Lanes threads each)
+constexpr int kG0Lanes = 8;
 __global__ __launch_bounds__(256) void k_bmg_gram0(const BmgLevel* __restrict__ lv,
                                                    const int2* __restrict__ blk,
                                                    const CgCtl* __restrict__ ctl) {
   const int2 t = blk[blockIdx.x];
   if (ctl[t.x].done) return;
   const BmgLevel& L = lv[t.x];
-  const int64_t k = (int64_t)t.y * 256 + threadIdx.x;
-  if (k >= L.g0n) return;
+  const int64_t k = (int64_t)t.y * (256 / kG0Lanes) + threadIdx.x / kG0Lanes;
+  if (k >= L.g0n) return;  // whole groups
   const int64_t i = L.g0list[k];
-  const int64_t e0 = L.A.gptr[i], e1 = L.A.gptr[i + 1];
-  float acc = 0.f;
-  for (int64_t e = e0; e < e1; ++e) acc += L.A.gval[e] * L.x[L.A.gcol[e]];
-  L.q[i] += acc;
+  const float acc = mg_lane_sum<kG0Lanes>(mg_row_share<kG0Lanes>(
+      L.A.gptr, L.A.gcol, L.A.gval, (const float*)L.x, i, (int)threadIdx.x % kG0Lanes));
+  if (threadIdx.x % kG0Lanes == 0) L.q[i] += acc;
 }
 
 // the same in FP64 for the outer iteration: q += G0 p, per-block partials of
@@ -316,15 +379,16 @@ __global__ __launch_bounds__(256) void k_bmg_gram64(const BmgSys* __restrict__ s
   const int2 t = blk[blockIdx.x];
   if (ctl[t.x].done) return;
   const BmgSys& S = sys[t.x];
-  const int64_t k = (int64_t)t.y * 256 + threadIdx.x;
+  const int64_t k = (int64_t)t.y * (256 / kG0Lanes) + threadIdx.x / kG0Lanes;
   double acc = 0.0;
-  if (k < S.g0n) {
+  if (k < S.g0n) {  // whole groups
     const int64_t i = S.g0list[k];
-    const int64_t e0 = S.gptr[i], e1 = S.gptr[i + 1];
-    double g = 0.0;
-    for (int64_t e = e0; e < e1; ++e) g += S.gval[e] * S.p[S.gcol[e]];
-    S.q[i] += g;
-    acc = S.p[i] * g;
+    const double g = mg_lane_sum<kG0Lanes>(mg_row_share<kG0Lanes>(
+        S.gptr, S.gcol, S.gval, (const double*)S.p, i, (int)threadIdx.x % kG0Lanes));
+    if (threadIdx.x % kG0Lanes == 0) {
+      S.q[i] += g;
+      acc = S.p[i] * g;
+    }
   }
   const double bs = block_sum(acc, sh);
   if (threadIdx.x == 0) part[blockIdx.x] = bs;

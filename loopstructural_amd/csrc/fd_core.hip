@@ -2063,6 +2063,9 @@ struct MgLevel {
   int32_t* cpos = nullptr;
 };
 
+// levels whose covered nodes the multi-rhs kernels smooth apart
+inline bool mr_covered(const MgLevel& L) { return L.cov && L.n >= kCovListMin; }
+
 struct Mg {
   std::vector<MgLevel> lv;
   // Chebyshev degrees of the coarse levels and of the fine one (<= deg).  A
@@ -2222,16 +2225,18 @@ void mg_apply(lsamd_fd_system* s, const T* x, T* y, const CgCtl* ctl, hipStream_
 
 // level apply in FP32: the fine level uses the data rows, coarse levels the
 // assembled Gram matrix of their data term (rows there are many per node)
-MgDev mg_dev(const MgLevel& L) {
-  MgDev d;
+template <typename T = float>
+MgDevT<T> mg_dev(const MgLevel& L) {
+  constexpr bool f32 = sizeof(T) == 4;
+  MgDevT<T> d;
   const lsamd_fd_system* s = L.sys;
   d.g = L.g;
   d.n = L.n;
-  d.tab = s->regular ? s->tab32 : nullptr;
-  d.w = make_regw<float>(s->reg);
+  d.tab = !s->regular ? nullptr : f32 ? (const T*)s->tab32 : (const T*)s->tab64;
+  d.w = make_regw<T>(s->reg);
   d.gptr = L.gptr;
   d.gcol = L.gcol;
-  d.gval = L.gval;
+  d.gval = f32 ? (const T*)L.gval : (const T*)L.gval64;
   return d;
 }
 
@@ -2291,11 +2296,6 @@ void mg_lanes(int64_t n, F&& launch) {
 // r = b - N x of a coarse level
 void mg_level_resid(const MgLevel& L, const CgCtl* ctl, hipStream_t st) {
   const MgDev A = mg_dev(L);
-  if (!A.tab) {
-    hipLaunchKernelGGL(k_mg_resid_node, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st, A,
-                       (const float*)L.b, (const float*)L.x, L.q, ctl);
-    return;
-  }
   mg_lanes(L.n, [&](auto g) {
     constexpr int G = decltype(g)::value;
     hipLaunchKernelGGL(k_mg_resid<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0, st, A,
@@ -2303,15 +2303,21 @@ void mg_level_resid(const MgLevel& L, const CgCtl* ctl, hipStream_t st) {
   });
 }
 
-// FP64 level apply (setup: power iteration and the dense coarsest operator)
+// y = N x of a level in FP64 (power iteration of the set-up)
 int mg_level_apply64(const MgLevel& L, const double* x, double* y, hipStream_t st) {
   lsamd_fd_system* s = L.sys;
-  if (!L.owned) return launch_apply<double>(s, x, y, s->t64, s->ctl_apply, st);
-  launch_stencil<double>(s, x, y, s->ctl_apply, st, s->zc[0]);
-  if (L.gptr)
-    hipLaunchKernelGGL(k_gram_spmv<double>, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st,
-                       (const int64_t*)L.gptr, (const int32_t*)L.gcol, (const double*)L.gval64,
-                       x, y, L.n, (const CgCtl*)s->ctl_apply);
+  if (L.owned) {
+    mg_lanes(L.n, [&](auto g) {
+      constexpr int G = decltype(g)::value;
+      hipLaunchKernelGGL(k_mg_apply64<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0, st,
+                         mg_dev<double>(L), x, y);
+    });
+  } else if (s->gram_state == 1) {
+    launch_stencil<double>(s, x, y, s->ctl_apply, st, s->zc[0]);
+    launch_gram_add<double>(s, x, y, nullptr, s->ctl_apply, st);
+  } else {
+    return launch_apply<double>(s, x, y, s->t64, s->ctl_apply, st);
+  }
   LSAMD_CHECK_LAUNCH("multigrid level apply");
   return LSAMD_OK;
 }
@@ -2326,38 +2332,51 @@ lsamd_grid mg_coarse_grid(const lsamd_grid& f) {
   return c;
 }
 
-int mg_prepare_level(lsamd_fd_system* sys, hipStream_t st) {
+// work vectors of a level; level 0 also times its stencil forms (the coarse
+// levels' operators take none)
+int mg_prepare_level(lsamd_fd_system* sys, bool level0, hipStream_t st) {
   if (int rc = ensure_work(sys, false)) return rc;
+  if (!level0) return LSAMD_OK;
   if (int rc = ensure_work(sys, true)) return rc;
   if (int rc = ensure_tuned<double>(sys, sys->p64, sys->q64, st)) return rc;
   if (int rc = ensure_tuned<float>(sys, sys->p32, sys->q32, st)) return rc;
   return LSAMD_OK;
 }
 
-// lambda_max(D^-1 N) by power iteration (FP64), on the level's work vectors
+// lambda_max(M N) by 20 steps of the power iteration (FP64), on the level's
+// work vectors.  The iterates are not normalised on the way (they grow by
+// lambda, 5 to 20, per step); the last two norms give the estimate.
 int mg_lambda(Mg* m, const MgLevel& L, double* out, hipStream_t st) {
   lsamd_fd_system* sys = L.sys;
   const int64_t n = sys->n;
-  const int vb = vec_blocks(n);
+  const int vb = std::min(vec_blocks(n), kPcgBlocks / 2);
   double *v = sys->p64, *y = sys->q64, *w = sys->r64;
-  const dim3 nb((unsigned)ceil_div(n, 256));
-  hipLaunchKernelGGL(k_mg_start, nb, dim3(256), 0, st, v, n);
+  const float* tag = L.sm ? L.sm : sys->minv32;
+  hipLaunchKernelGGL(k_mg_start, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, v, n);
   for (int it = 0; it < 20; ++it) {
+    if (it > 0) std::swap(v, w);
     if (int rc = mg_level_apply64(L, v, y, st)) return rc;
-    hipLaunchKernelGGL(k_mg_power, dim3(vb), dim3(256), 0, st, (const double*)y,
-                       (const double*)sys->minv64, (const float*)(L.sm ? L.sm : sys->minv32),
-                       (const int64_t*)L.sptr, (const int32_t*)L.scol, (const double*)L.sval64,
-                       (const double*)v, w, n, sys->part);
-    hipLaunchKernelGGL(k_mg_norm_fin, dim3(1), dim3(256), 0, st, (const double*)sys->part, vb,
-                       m->scal);
-    hipLaunchKernelGGL(k_mg_scale, nb, dim3(256), 0, st, (const double*)w, v, n,
-                       (const double*)m->scal);
+    auto power = [&](auto g) {
+      constexpr int G = decltype(g)::value;
+      hipLaunchKernelGGL(k_mg_power<G>, dim3((unsigned)ceil_div(n * G, 256)), dim3(256), 0, st,
+                         (const double*)y, (const double*)sys->minv64, tag,
+                         (const int64_t*)L.sptr, (const int32_t*)L.scol, (const double*)L.sval64,
+                         n, w);
+    };
+    if (n >= 16384)
+      power(std::integral_constant<int, 4>());
+    else
+      power(std::integral_constant<int, 16>());
   }
+  hipLaunchKernelGGL(k_mg_norms, dim3(vb), dim3(256), 0, st, (const double*)v, (const double*)w, n,
+                     sys->pcg_pr);
+  hipLaunchKernelGGL(k_mg_norm_fin, dim3(1), dim3(256), 0, st, (const double*)sys->pcg_pr, vb,
+                     m->scal);
   LSAMD_CHECK_LAUNCH("multigrid power iteration");
-  double sc[2] = {0.0, 0.0};
-  LSAMD_HIP(hipMemcpyAsync(sc, m->scal, 16, hipMemcpyDeviceToHost, st));
+  double lam = 0.0;
+  LSAMD_HIP(hipMemcpyAsync(&lam, m->scal, 8, hipMemcpyDeviceToHost, st));
   LSAMD_HIP(hipStreamSynchronize(st));
-  *out = sc[0];
+  *out = lam;
   return LSAMD_OK;
 }
 
@@ -2613,7 +2632,7 @@ int mg_schwarz(Mg* m, MgLevel& L, const std::vector<int64_t>& cells, const CsrOu
                      (const int64_t*)L.sptr, (const float*)S->minv32, L.sm, L.n);
   cleanup();
   LSAMD_CHECK_LAUNCH("multigrid smoother tags");
-  if (L.n >= kCovListMin) {
+  if (!L.owned || L.n >= kCovListMin) {
     // compact list of the covered nodes (their tags are negative)
     uint8_t* flag = nullptr;
     int32_t *cov = nullptr, *nsel = nullptr;
@@ -2757,7 +2776,7 @@ struct MgTimer {
 // (re-discretised regulariser, tuned stencils, work vectors) and the level
 // vectors.  Built once per system.
 int mg_build_static(lsamd_fd_system* s, Mg* m, hipStream_t st) {
-  if (int rc = mg_prepare_level(s, st)) return rc;
+  if (int rc = mg_prepare_level(s, true, st)) return rc;
   if (int rc = mg_alloc(m, &m->scal, 2)) return rc;
   const char* sm_env = getenv("LSAMD_MG_SMOOTHER");
   m->schwarz = !(sm_env && strcmp(sm_env, "jacobi") == 0);
@@ -2792,7 +2811,7 @@ int mg_build_static(lsamd_fd_system* s, Mg* m, hipStream_t st) {
     L.n = cs->n;
     m->lv.push_back(L);
     if (int rc = mg_level_vectors(m, m->lv.back())) return rc;
-    if (int rc = mg_prepare_level(cs, st)) return rc;
+    if (int rc = mg_prepare_level(cs, false, st)) return rc;
     gprev = gc;
   }
   const int64_t nc = m->lv.back().n;
@@ -3176,8 +3195,8 @@ int mg_ensure(lsamd_fd_system* s, hipStream_t st) {
 int mg_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const double* b, double* c,
              lsamd_solve_info* inf, hipStream_t st) {
   if (s->op != 0) return fail(LSAMD_ERR_ARG, "multigrid is available for FD systems only");
-  if (int rc = mg_ensure(s, st)) return rc;
   if (int rc = pcg_gram_ensure(s, st)) return rc;
+  if (int rc = mg_ensure(s, st)) return rc;
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : 10 * n;
   const int maxiter = (int)std::min<int64_t>(maxiter64, 2000000000LL);
@@ -3229,6 +3248,8 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   std::vector<std::vector<int2>> all(nl), sm(nl);
   std::vector<std::vector<int>> dense(nl);
   std::vector<BmgSys> hs(nsys);
+  std::vector<int64_t> lnodes(nl, 0);  // smoothed nodes of a level, all systems
+  std::vector<int2> cv;                // blocks of the covered lists of level 0
   for (int i = 0; i < nsys; ++i) {
     lsamd_fd_system* s = ss[i];
     const Mg* m = s->mg;
@@ -3244,6 +3265,8 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
         d.A.gval = m->g0v32;
         d.g0list = m->g0list;
         d.g0n = m->g0list ? m->g0n : 0;
+        d.cov = V.sptr ? V.cov : nullptr;
+        d.ncov = d.cov ? V.ncov : 0;
       }
       d.S = mg_sm(V);
       d.b = V.b;
@@ -3266,6 +3289,10 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
         all[l].push_back(make_int2(i, b));
         if (l < last) sm[l].push_back(make_int2(i, b));
       }
+      if (l < last) lnodes[l] += V.n;
+      if (l == 0 && l < last)
+        for (int64_t b = 0; b < ceil_div(d.ncov * kCovLanes, 256); ++b)
+          cv.push_back(make_int2(i, (int)(-1 - b)));
       if (l == 0) hs[i].b1 = (int)all[0].size();
     }
     BmgSys& y = hs[i];
@@ -3289,6 +3316,18 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
     y.gb0 = y.b0;  // node-block partials (the plane-streaming form resets these)
     y.gb1 = y.b1;
   }
+  // level 0 smooths its covered lists first (their rows are the longer
+  // chains); the coarse levels' blocks hold 256 / G nodes
+  cv.insert(cv.end(), sm[0].begin(), sm[0].end());
+  std::vector<std::vector<int2>> ln(nl);
+  for (int l = 1; l < nl; ++l)
+    for (int i = 0; i < nsys; ++i) {
+      const Mg* m = ss[i]->mg;
+      if (l >= (int)m->lv.size() - 1) continue;
+      int per = 256;
+      mg_lanes(lnodes[l], [&](auto g) { per = 256 / decltype(g)::value; });
+      for (int64_t b = 0; b < ceil_div(m->lv[l].n, per); ++b) ln[l].push_back(make_int2(i, (int)b));
+    }
   // level 0 by the plane-streaming stencil when every system shares the
   // class table (one regulariser) and is large enough for z-chunks of 16 on
   // 32 x 16 tiles, and level 0 is not its coarsest; the work items of every
@@ -3304,14 +3343,15 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   }
   std::vector<int4> ht;
   std::vector<BSys> hb32, hb64;
-  std::vector<int2> hgl;  // blocks of 256 entries of every system's Gram node list
+  std::vector<int2> hgl;  // blocks of every system's Gram node list
   if (tiles0) {
     hb32.resize(nsys);
     hb64.resize(nsys);
     for (int i = 0; i < nsys; ++i) {
       lsamd_fd_system* s = ss[i];
       hs[i].gb0 = (int)hgl.size();
-      for (int64_t b = 0; b < ceil_div(hs[i].g0n, 256); ++b) hgl.push_back(make_int2(i, (int)b));
+      for (int64_t b = 0; b < ceil_div(hs[i].g0n * kG0Lanes, 256); ++b)
+        hgl.push_back(make_int2(i, (int)b));
       hs[i].gb1 = (int)hgl.size();
       hs[i].t0 = (int)ht.size();
       stencil_tiles(i, s->gd, kB0Zc, ht, kB0Tx);
@@ -3332,10 +3372,11 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   size_t bytes = up(nsys * sizeof(BmgSys)) + up(nsys * sizeof(CgCtl)) + up(sizeof(int)) +
                  up(2 * all[0].size() * sizeof(double)) + up(ht.size() * sizeof(int4)) +
                  up(ht.size() * sizeof(double)) + 2 * up(hb32.size() * sizeof(BSys)) +
-                 up(hgl.size() * sizeof(int2));
+                 up(hgl.size() * sizeof(int2)) + up(cv.size() * sizeof(int2)) +
+                 up(hgl.size() * sizeof(double));
   for (int l = 0; l < nl; ++l)
     bytes += up(nsys * sizeof(BmgLevel)) + up(all[l].size() * sizeof(int2)) +
-             up(sm[l].size() * sizeof(int2)) + up(dense[l].size() * sizeof(int));
+             up(sm[l].size() * sizeof(int2)) + up(ln[l].size() * sizeof(int2)) + up(dense[l].size() * sizeof(int));
   unsigned char* base = nullptr;
   if (hipMalloc((void**)&base, bytes) != hipSuccess)
     return fail(LSAMD_ERR_ALLOC, "batched multigrid: hipMalloc failed");
@@ -3361,19 +3402,21 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   BmgSys* dsys = (BmgSys*)take(nsys * sizeof(BmgSys));
   CgCtl* ctl = (CgCtl*)take(nsys * sizeof(CgCtl));
   int* flag = (int*)take(sizeof(int));
-  double* part = (double*)take(2 * all[0].size() * sizeof(double));
+  double* part = (double*)take(std::max(2 * all[0].size(), hgl.size()) * sizeof(double));
+  int2* dcv = (int2*)take(cv.size() * sizeof(int2));
   int4* dtiles = (int4*)take(ht.size() * sizeof(int4));
   double* tpart = (double*)take(ht.size() * sizeof(double));
   BSys* db32 = (BSys*)take(hb32.size() * sizeof(BSys));
   BSys* db64 = (BSys*)take(hb64.size() * sizeof(BSys));
   int2* dgl = (int2*)take(hgl.size() * sizeof(int2));
   std::vector<BmgLevel*> dlv(nl);
-  std::vector<int2*> dall(nl), dsm(nl);
+  std::vector<int2*> dall(nl), dsm(nl), dln(nl);
   std::vector<int*> ddense(nl);
   for (int l = 0; l < nl; ++l) {
     dlv[l] = (BmgLevel*)take(nsys * sizeof(BmgLevel));
     dall[l] = (int2*)take(all[l].size() * sizeof(int2));
     dsm[l] = (int2*)take(sm[l].size() * sizeof(int2));
+    dln[l] = (int2*)take(ln[l].size() * sizeof(int2));
     ddense[l] = (int*)take(dense[l].size() * sizeof(int));
   }
   auto h2d = [&](void* d, const void* h, size_t b) {
@@ -3384,10 +3427,12 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   if (e == hipSuccess) e = h2d(db32, hb32.data(), hb32.size() * sizeof(BSys));
   if (e == hipSuccess) e = h2d(db64, hb64.data(), hb64.size() * sizeof(BSys));
   if (e == hipSuccess) e = h2d(dgl, hgl.data(), hgl.size() * sizeof(int2));
+  if (e == hipSuccess) e = h2d(dcv, cv.data(), cv.size() * sizeof(int2));
   for (int l = 0; l < nl && e == hipSuccess; ++l) {
     e = h2d(dlv[l], hl[l].data(), nsys * sizeof(BmgLevel));
     if (e == hipSuccess) e = h2d(dall[l], all[l].data(), all[l].size() * sizeof(int2));
     if (e == hipSuccess) e = h2d(dsm[l], sm[l].data(), sm[l].size() * sizeof(int2));
+    if (e == hipSuccess) e = h2d(dln[l], ln[l].data(), ln[l].size() * sizeof(int2));
     if (e == hipSuccess) e = h2d(ddense[l], dense[l].data(), dense[l].size() * sizeof(int));
   }
   if (e != hipSuccess) return finish(fail(LSAMD_ERR_HIP, "batched multigrid: upload failed"));
@@ -3405,8 +3450,16 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
   LSAMD_CHECK_LAUNCH("batched multigrid init");
   // one iteration for every system
   auto cheb = [&](int l, int mode, int k, int last, hipStream_t cs) {
-    hipLaunchKernelGGL(k_bmg_cheb, g(sm[l].size()), b256, 0, cs, (const BmgLevel*)dlv[l],
-                       (const int2*)dsm[l], mode, k, last, (const CgCtl*)ctl);
+    if (l == 0)
+      hipLaunchKernelGGL(k_bmg_cheb, g(cv.size()), b256, 0, cs, (const BmgLevel*)dlv[l],
+                         (const int2*)dcv, mode, k, last, (const CgCtl*)ctl);
+    else
+      mg_lanes(lnodes[l], [&](auto gg) {
+        constexpr int G = decltype(gg)::value;
+        hipLaunchKernelGGL(k_bmg_smooth<G>, g(ln[l].size()), b256, 0, cs,
+                           (const BmgLevel*)dlv[l], (const int2*)dln[l], mode, k, last,
+                           (const CgCtl*)ctl);
+      });
   };
   const unsigned nt0 = (unsigned)ht.size();
   auto apply = [&](int l, hipStream_t cs) {
@@ -3420,8 +3473,15 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
                            (const int2*)dgl, (const CgCtl*)ctl);
       return;
     }
-    hipLaunchKernelGGL(k_bmg_apply, g(sm[l].size()), b256, 0, cs, (const BmgLevel*)dlv[l],
-                       (const int2*)dsm[l], (const CgCtl*)ctl);
+    if (l == 0)
+      hipLaunchKernelGGL(k_bmg_apply, g(sm[l].size()), b256, 0, cs, (const BmgLevel*)dlv[l],
+                         (const int2*)dsm[l], (const CgCtl*)ctl);
+    else
+      mg_lanes(lnodes[l], [&](auto gg) {
+        constexpr int G = decltype(gg)::value;
+        hipLaunchKernelGGL(k_bmg_resid<G>, g(ln[l].size()), b256, 0, cs, (const BmgLevel*)dlv[l],
+                           (const int2*)dln[l], (const CgCtl*)ctl);
+      });
   };
   auto smooth = [&](int l, int from_zero, hipStream_t cs) {
     const int dg = l == 0 ? deg0 : deg;
@@ -3438,7 +3498,7 @@ int bmg_solve(lsamd_fd_system* const* ss, int nsys, const lsamd_solve_opts* o,
         apply(l, cs);
         hipLaunchKernelGGL(k_bmg_restrict, g(all[l + 1].size()), b256, 0, cs,
                            (const BmgLevel*)dlv[l], (const BmgLevel*)dlv[l + 1],
-                           (const int2*)dall[l + 1], (const CgCtl*)ctl);
+                           (const int2*)dall[l + 1], l == 0, (const CgCtl*)ctl);
       }
       if (!dense[l].empty())
         hipLaunchKernelGGL(k_bmg_dense, dim3(kMgCoarse * kMgCoarse * kMgCoarse,
@@ -3887,9 +3947,9 @@ int mr_sell_ensure(lsamd_fd_system* s, hipStream_t st) {
     MgLevel& L = m->lv[l];
     // levels with a covered list: the covered rows over list positions;
     // the others: every node's row
-    if (L.sptr && !L.cov)
+    if (L.sptr && !mr_covered(L))
       if (int rc = sell_build(m, L.sptr, L.scol, L.sval, L.sm, nullptr, L.n, &L.ssl, st)) return rc;
-    if (L.sptr && L.cov && L.ncov > 0) {
+    if (L.sptr && mr_covered(L) && L.ncov > 0) {
       if (int rc = sell_build(m, L.sptr, L.scol, L.sval, nullptr, L.cov, L.ncov, &L.csl, st))
         return rc;
       int32_t* pos = nullptr;
@@ -4042,7 +4102,7 @@ void mr_vcycle(lsamd_fd_system* s, MrWork* w, int l, hipStream_t st) {
   }
   const dim3 nb((unsigned)ceil_div(L.n, 256), R);
   const MgSm S = mg_sm(L);
-  const int split = L.cov ? 1 : 0;
+  const int split = mr_covered(L) ? 1 : 0;
   // XCD-contiguous workgroups where measured faster: the sliced smoother
   // and the restriction; the covered-node step and the prolongation keep the
   // hardware order
@@ -4620,7 +4680,7 @@ int time_multi(lsamd_fd_system* s, MrWork* w, int32_t kernel, int32_t iters, dou
   const int* zflag = (const int*)s->tzero;
   const MgLevel& L = s->mg->lv[0];
   const int64_t n = s->n;
-  const int split = L.cov ? 1 : 0;
+  const int split = mr_covered(L) ? 1 : 0;
   // the all-node step (covered nodes read M r from the list) where the
   // level has one, else the split step over the uncovered nodes
   const bool all = split && L.cpos && w->zcov.size() > 0 && w->zcov[0];

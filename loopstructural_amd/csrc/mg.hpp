@@ -356,56 +356,59 @@ __global__ void k_mg_rows(const int64_t* __restrict__ row_ptr, const int32_t* __
   }
 }
 
-// power iteration step: w = M y (y = N v), partial |w|^2 and v.w
+// power iteration step w = M y (y = N v), G threads per node
+template <int G>
 __global__ __launch_bounds__(256) void k_mg_power(const double* __restrict__ y,
                                                   const double* __restrict__ minv,
                                                   const float* __restrict__ sm,
                                                   const int64_t* __restrict__ sptr,
                                                   const int32_t* __restrict__ scol,
-                                                  const double* __restrict__ sval,
-                                                  const double* __restrict__ v,
-                                                  double* __restrict__ w, int64_t n,
+                                                  const double* __restrict__ sval, int64_t n,
+                                                  double* __restrict__ w) {
+  const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t i = th / G;
+  const int l = (int)(th % G);
+  if (i >= n) return;  // whole groups
+  const float t = sm[i];
+  const double own = minv[i] * y[i];
+  double z = 0.0;
+  if (sptr) {
+    const int64_t e1 = sptr[i + 1];
+    for (int64_t e = sptr[i] + l; e < e1; e += 2 * G) {
+      const bool two = e + G < e1;
+      const int64_t f = two ? e + G : e;
+      z += sval[e] * y[scol[e]] + (two ? sval[f] : 0.0) * y[scol[f]];
+    }
+  }
+#pragma unroll
+  for (int o = G / 2; o > 0; o >>= 1) z += __shfl_xor(z, o, 64);
+  if (l == 0) w[i] = t >= 0.f ? own : z;
+}
+
+// partials of |v|^2, then those of |w|^2
+__global__ __launch_bounds__(256) void k_mg_norms(const double* __restrict__ v,
+                                                  const double* __restrict__ w, int64_t n,
                                                   double* __restrict__ part) {
   __shared__ double sh[4];
   double a = 0.0, b = 0.0;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
-    double wv;
-    if (sm[i] >= 0.f) {
-      wv = minv[i] * y[i];
-    } else {
-      wv = 0.0;
-      for (int64_t e = sptr[i]; e < sptr[i + 1]; ++e) wv += sval[e] * y[scol[e]];
-    }
-    w[i] = wv;
-    a += wv * wv;
-    b += v[i] * wv;
+    a += v[i] * v[i];
+    b += w[i] * w[i];
   }
   const double sa = block_sum(a, sh);
   const double sb = block_sum(b, sh);
   if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = sa;
-    part[2 * blockIdx.x + 1] = sb;
+    part[blockIdx.x] = sa;
+    part[gridDim.x + blockIdx.x] = sb;
   }
 }
 
-// one block: scal[0] = |w| (the eigenvalue estimate), scal[1] = 1/|w|
+// one block: scal[0] = |w| / |v| (the eigenvalue estimate)
 __global__ __launch_bounds__(256) void k_mg_norm_fin(const double* __restrict__ part, int np,
                                                      double* __restrict__ scal) {
   __shared__ double sh[4];
-  double a = 0.0;
-  for (int i = threadIdx.x; i < np; i += 256) a += part[2 * i];
-  const double sa = block_sum(a, sh);
-  if (threadIdx.x == 0) {
-    const double wn = sqrt(sa);
-    scal[0] = wn;
-    scal[1] = wn > 0.0 ? 1.0 / wn : 0.0;
-  }
-}
-
-__global__ void k_mg_scale(const double* __restrict__ w, double* __restrict__ v, int64_t n,
-                           const double* __restrict__ scal) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) v[i] = w[i] * scal[1];
+  const double a = pcg_total(part, np, sh), b = pcg_total(part + np, np, sh);
+  if (threadIdx.x == 0) scal[0] = a > 0.0 ? sqrt(b / a) : 0.0;
 }
 
 // deterministic positive start vector of the power iteration
@@ -595,35 +598,38 @@ __global__ __launch_bounds__(256) void k_fcg_upd_fin(const double* __restrict__ 
 // Device view of one coarse level's operator: regulariser (class table, or
 // the exact per-node formula when the table does not apply) + data Gram
 // matrix.
-struct MgDev {
+template <typename T>
+struct MgDevT {
   GridDev g;
   int64_t n;
-  const float* tab;  // FP32 class table, nullptr: per-node formula with w
-  RegW<float> w;
+  const T* tab;  // class table, nullptr: per-node formula with w
+  RegW<T> w;
   const int64_t* gptr;
   const int32_t* gcol;
-  const float* gval;
+  const T* gval;
 };
+using MgDev = MgDevT<float>;
 
-__device__ inline float mg_apply_node(const MgDev& L, const float* __restrict__ x, int64_t id) {
+template <typename T>
+__device__ inline T mg_apply_node(const MgDevT<T>& L, const T* __restrict__ x, int64_t id) {
   int i, j, k;
   mg_ijk(id, L.g.nx, L.g.ny, i, j, k);
-  float acc;
+  T acc;
   if (L.tab) {
     const int nx = L.g.nx, ny = L.g.ny, nz = L.g.nz;
     const int64_t nxy = (int64_t)nx * ny;
-    const float* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
+    const T* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
     acc = c[0] * x[id];
 #pragma unroll
     for (int t = 1; t < kTaps; ++t) {
       const int dx = kBTap[t][0], dy = kBTap[t][1], dz = kBTap[t][2];
       const bool ok = (unsigned)(i + dx) < (unsigned)nx && (unsigned)(j + dy) < (unsigned)ny &&
                       (unsigned)(k + dz) < (unsigned)nz;
-      const float xv = x[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
-      acc += c[t] * (ok ? xv : 0.f);
+      const T xv = x[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
+      acc += c[t] * (ok ? xv : (T)0);
     }
   } else {
-    acc = general_node<float>(x, L.g, L.w, nullptr, i, j, k);
+    acc = general_node<T>(x, L.g, L.w, nullptr, i, j, k);
   }
   if (L.gptr) {
     int64_t e = L.gptr[id];
@@ -663,22 +669,21 @@ __constant__ int kTapPack[32] = {
     0x420, 0x442, 0x402, -1,    -1,    -1,    -1,    -1,    -1,    -1};
 
 // sum of val[e] v[col[e]] over a row's entries, this thread's share
-template <int G>
-__device__ inline float mg_row_share(const int64_t* __restrict__ ptr,
-                                     const int32_t* __restrict__ col,
-                                     const float* __restrict__ val, const float* __restrict__ v,
-                                     int64_t i, int l) {
+template <int G, typename T>
+__device__ inline T mg_row_share(const int64_t* __restrict__ ptr, const int32_t* __restrict__ col,
+                                 const T* __restrict__ val, const T* __restrict__ v, int64_t i,
+                                 int l) {
   const int64_t e1 = ptr[i + 1];
-  float acc = 0.f;
+  T acc = 0;
   for (int64_t e = ptr[i] + l; e < e1; e += 4 * G) {
     int32_t c[4];
-    float a[4];
+    T a[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const bool ok = e + k * G < e1;
       const int64_t at = ok ? e + k * G : e;
       c[k] = col[at];
-      a[k] = ok ? val[at] : 0.f;
+      a[k] = ok ? val[at] : (T)0;
     }
 #pragma unroll
     for (int k = 0; k < 4; ++k) acc += a[k] * v[c[k]];
@@ -686,14 +691,51 @@ __device__ inline float mg_row_share(const int64_t* __restrict__ ptr,
   return acc;
 }
 
-template <int G>
-__device__ inline float mg_lane_sum(float v) {
+template <int G, typename T>
+__device__ inline T mg_lane_sum(T v) {
 #pragma unroll
   for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
 
-// r = b - N x of a level with a class table
+// (N x)[id], summed over the G threads of the node
+template <int G, typename T>
+__device__ inline T mg_product(const MgDevT<T>& L, const T* __restrict__ x, int64_t id, int l) {
+  if (!L.tab) return mg_lane_sum<G>(l == 0 ? mg_apply_node(L, x, id) : (T)0);
+  int i, j, k;
+  mg_ijk(id, L.g.nx, L.g.ny, i, j, k);
+  const int nx = L.g.nx, ny = L.g.ny, nz = L.g.nz;
+  const int64_t nxy = (int64_t)nx * ny;
+  const T* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
+  constexpr int kT = (kTaps + G - 1) / G;
+  T cv[kT], xv[kT];
+#pragma unroll
+  for (int q = 0; q < kT; ++q) {
+    const int t = l + q * G;
+    const int p = kTapPack[t < 32 ? t : 31];
+    const int dx = (p & 15) - 2, dy = ((p >> 4) & 15) - 2, dz = ((p >> 8) & 15) - 2;
+    const bool ok = t < kTaps && (unsigned)(i + dx) < (unsigned)nx &&
+                    (unsigned)(j + dy) < (unsigned)ny && (unsigned)(k + dz) < (unsigned)nz;
+    cv[q] = ok ? c[t] : (T)0;
+    xv[q] = x[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
+  }
+  T acc = L.gptr ? mg_row_share<G>(L.gptr, L.gcol, L.gval, x, id, l) : (T)0;
+#pragma unroll
+  for (int q = 0; q < kT; ++q) acc += cv[q] * xv[q];
+  return mg_lane_sum<G>(acc);
+}
+
+// (M r)[i] of the smoother, summed over the G threads of the node
+template <int G>
+__device__ inline float mg_smoothed(const MgSm& S, const float* __restrict__ r, int64_t i, int l) {
+  const float t = S.sm[i], rv = r[i];
+  float z = 0.f;
+  if (S.sptr) z = mg_row_share<G>(S.sptr, S.scol, S.sval, r, i, l);
+  z = mg_lane_sum<G>(z);
+  return t >= 0.f ? t * rv : z;
+}
+
+// r = b - N x
 template <int G>
 __global__ __launch_bounds__(256) void k_mg_resid(MgDev L, const float* __restrict__ b,
                                                   const float* __restrict__ x,
@@ -703,38 +745,20 @@ __global__ __launch_bounds__(256) void k_mg_resid(MgDev L, const float* __restri
   const int l = (int)(th % G);
   if (id >= L.n) return;  // whole groups
   const int done = ctl->done;
-  int i, j, k;
-  mg_ijk(id, L.g.nx, L.g.ny, i, j, k);
-  const int nx = L.g.nx, ny = L.g.ny, nz = L.g.nz;
-  const int64_t nxy = (int64_t)nx * ny;
-  const float* c = L.tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
   const float bv = b[id];
-  constexpr int kT = (kTaps + G - 1) / G;
-  float cv[kT], xv[kT];
-#pragma unroll
-  for (int q = 0; q < kT; ++q) {
-    const int t = l + q * G;
-    const int p = kTapPack[t < 32 ? t : 31];
-    const int dx = (p & 15) - 2, dy = ((p >> 4) & 15) - 2, dz = ((p >> 8) & 15) - 2;
-    const bool ok = t < kTaps && (unsigned)(i + dx) < (unsigned)nx &&
-                    (unsigned)(j + dy) < (unsigned)ny && (unsigned)(k + dz) < (unsigned)nz;
-    cv[q] = ok ? c[t] : 0.f;
-    xv[q] = x[ok ? id + dx + (int64_t)nx * dy + nxy * dz : id];
-  }
-  float acc = L.gptr ? mg_row_share<G>(L.gptr, L.gcol, L.gval, x, id, l) : 0.f;
-#pragma unroll
-  for (int q = 0; q < kT; ++q) acc += cv[q] * xv[q];
-  acc = mg_lane_sum<G>(acc);
-  if (l == 0 && !done) r[id] = bv - acc;
+  const float v = mg_product<G>(L, x, id, l);
+  if (l == 0 && !done) r[id] = bv - v;
 }
 
-// the same where no class table applies, one node per thread
-__global__ __launch_bounds__(256) void k_mg_resid_node(MgDev L, const float* __restrict__ b,
-                                                       const float* __restrict__ x,
-                                                       float* __restrict__ r, const CgCtl* ctl) {
-  if (ctl->done) return;
-  const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id < L.n) r[id] = b[id] - mg_apply_node(L, x, id);
+// y = N x in FP64 (set-up)
+template <int G>
+__global__ __launch_bounds__(256) void k_mg_apply64(MgDevT<double> L, const double* __restrict__ x,
+                                                    double* __restrict__ y) {
+  const int64_t th = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t id = th / G;
+  if (id >= L.n) return;
+  const double v = mg_product<G>(L, x, id, (int)(th % G));
+  if (th % G == 0) y[id] = v;
 }
 
 // smoothing step from the residual r: dv = c1 d + c2 M r (c1 = 0: d is not
@@ -749,13 +773,8 @@ __global__ __launch_bounds__(256) void k_mg_smooth(const float* __restrict__ r, 
   const int l = (int)(th % G);
   if (i >= n) return;  // whole groups
   const int done = ctl->done;
-  const float t = S.sm[i], rv = r[i];
   const float xv = from_zero ? 0.f : x[i], dv0 = c1 != 0.f ? d[i] : 0.f;
-  float z = 0.f;
-  if (S.sptr) z = mg_row_share<G>(S.sptr, S.scol, S.sval, r, i, l);
-  z = mg_lane_sum<G>(z);
-  if (t >= 0.f) z = t * rv;
-  const float dv = c1 * dv0 + c2 * z;
+  const float dv = c1 * dv0 + c2 * mg_smoothed<G>(S, r, i, l);
   if (l != 0 || done) return;
   if (!last) d[i] = dv;
   x[i] = xv + dv;
