@@ -918,7 +918,7 @@ __global__ void k_fill_one(double* a, float* b, int64_t n) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) {
     a[i] = 1.0;
-    b[i] = 1.0f;
+    if (b) b[i] = 1.0f;
   }
 }
 void launch_eval_entries(const GridDev& g, const double* pts, const double* gv, int64_t n,
@@ -4389,16 +4389,19 @@ int mr_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, int nrhs, const doub
 
 // ------------------------------------------------------------------ LSMR ----
 struct Ls {
-  double *v = nullptr, *h = nullptr, *hbar = nullptr, *x = nullptr, *xs = nullptr, *y = nullptr;
-  double *ureg = nullptr, *urid = nullptr, *ud = nullptr, *tr = nullptr;
-  double *pa = nullptr, *pb = nullptr, *pv = nullptr, *px = nullptr;  // partials
-  int na = 0, nb = 0, nv = 0;
-  LsCtl* ctl = nullptr;
-  LsCtl* host = nullptr;
+  double *v = nullptr, *h = nullptr, *hbar = nullptr, *x = nullptr, *xs = nullptr, *sv = nullptr;
+  double *uw = nullptr, *urid = nullptr, *ud = nullptr, *cw = nullptr;
+  double *pu = nullptr, *pv = nullptr, *px = nullptr;  // partials
+  int nn = 0, nd = 0, nc = 0;  // workgroups: nodes, data rows, nodes with data rows
+  uint64_t* mask = nullptr;    // nodes with data rows, and their count before each word
+  int32_t* base = nullptr;
+  LsCtl* ctl = nullptr;  // two slots
+  LsEst* est = nullptr;  // two slots
+  LsMid* mid = nullptr;
+  LsMid* host = nullptr;
   std::vector<void*> mem;
   hipGraphExec_t graph = nullptr;
   int graph_chunk = 0;
-  const double* graph_scale = nullptr;  // column scaling the graph was captured with
 };
 
 void ls_destroy(Ls* l) {
@@ -4422,79 +4425,81 @@ int ls_alloc(Ls* l, P** p, int64_t count) {
 }
 
 int ls_build(lsamd_fd_system* s, Ls* l) {
-  const int64_t n = s->n, m = std::max<int64_t>(s->nrows, 1);
-  for (double** p : {&l->v, &l->h, &l->hbar, &l->x, &l->xs, &l->y, &l->urid})
+  const int64_t n = s->n, m = std::max<int64_t>(s->nrows, 1), nw = ceil_div(n, 64);
+  for (double** p : {&l->v, &l->h, &l->hbar, &l->x, &l->xs, &l->sv, &l->urid})
     if (int rc = ls_alloc(l, p, n)) return rc;
-  if (int rc = ls_alloc(l, &l->ureg, 6 * n)) return rc;
+  if (int rc = ls_alloc(l, &l->uw, 6 * n)) return rc;
   if (int rc = ls_alloc(l, &l->ud, m)) return rc;
-  if (int rc = ls_alloc(l, &l->tr, m)) return rc;
-  l->na = (int)ceil_div(n, 256);
-  l->nb = (int)ceil_div(m, 256);
-  l->nv = vec_blocks(n);
-  if (int rc = ls_alloc(l, &l->pa, l->na)) return rc;
-  if (int rc = ls_alloc(l, &l->pb, l->nb)) return rc;
-  if (int rc = ls_alloc(l, &l->pv, l->nv)) return rc;
-  if (int rc = ls_alloc(l, &l->px, l->nv)) return rc;
-  if (int rc = ls_alloc(l, &l->ctl, 1)) return rc;
-  if (hipHostMalloc((void**)&l->host, sizeof(LsCtl), hipHostMallocDefault) != hipSuccess)
+  l->nn = (int)ceil_div(n, 256);
+  l->nd = (int)ceil_div(s->nrows, 32);
+  l->nc = (int)ceil_div(s->ndn, 64);
+  if (int rc = ls_alloc(l, &l->cw, s->nnz)) return rc;
+  // the partials and their sum (k_ls_fold)
+  if (int rc = ls_alloc(l, &l->pu, l->nn + l->nd + 1)) return rc;
+  if (int rc = ls_alloc(l, &l->pv, l->nn + l->nc + 1)) return rc;
+  if (int rc = ls_alloc(l, &l->px, l->nn + 1)) return rc;
+  if (int rc = ls_alloc(l, &l->mask, nw)) return rc;
+  if (int rc = ls_alloc(l, &l->base, nw)) return rc;
+  if (int rc = ls_alloc(l, &l->ctl, 2)) return rc;
+  if (int rc = ls_alloc(l, &l->est, 2)) return rc;
+  if (int rc = ls_alloc(l, &l->mid, 1)) return rc;
+  if (hipHostMalloc((void**)&l->host, sizeof(LsMid), hipHostMallocDefault) != hipSuccess)
     return fail(LSAMD_ERR_ALLOC, "hipHostMalloc failed (LSMR)");
-  for (double* p : {l->v, l->h, l->hbar, l->x, l->xs, l->y, l->urid})
-    LSAMD_HIP(legacy_memset(p, 0, n * 8));
-  LSAMD_HIP(legacy_memset(l->ureg, 0, 6 * n * 8));
-  LSAMD_HIP(legacy_memset(l->ud, 0, m * 8));
-  LSAMD_HIP(legacy_memset(l->tr, 0, m * 8));
   return LSAMD_OK;
 }
 
-// u <- A S xs - fwd_coef u ; beta ; v <- S A^T u / beta - beta v ; partials
-// of |v|^2.  init: u = b instead of the product, v = S A^T u / beta.
-// sc: squared column scaling (diag(A^T A)^-1, or ones)
-void ls_bidiag(lsamd_fd_system* s, Ls* l, const double* sc, int init, hipStream_t st) {
-  const int64_t n = s->n;
-  const RegW<double> w = make_regw<double>(s->reg);
-  RowsDev R = rows_dev(s, false);
-  const dim3 nb((unsigned)l->na), b256(256);
-  if (!init)
-    hipLaunchKernelGGL(k_ls_scale, nb, b256, 0, st, (const double*)l->v,
-                       sc, l->xs, n, (const LsCtl*)l->ctl);
-  hipLaunchKernelGGL(k_ls_reg_fwd, nb, b256, 0, st, (const double*)l->xs, s->gd, w,
-                     (const double*)s->scale2, l->ureg, l->urid, n, init, l->pa,
-                     (const LsCtl*)l->ctl);
-  int nbp = 0;
-  if (s->nrows > 0) {
-    nbp = l->nb;
-    hipLaunchKernelGGL(k_ls_data_fwd, dim3((unsigned)l->nb), b256, 0, st, (const double*)l->xs,
-                       R, (const double*)s->w, (const double*)s->b, l->ud, init, l->pb,
-                       (const LsCtl*)l->ctl);
-  }
-  hipLaunchKernelGGL(k_ls_beta, dim3(1), b256, 0, st, (const double*)l->pa, l->na,
-                     (const double*)l->pb, nbp, l->ctl, init);
-  hipLaunchKernelGGL(k_ls_reg_t, nb, b256, 0, st, (const double*)l->ureg, (const double*)l->urid,
-                     s->gd, w, (const double*)s->scale2, l->y, n, (const LsCtl*)l->ctl);
-  if (s->nrows > 0) {
-    hipLaunchKernelGGL(k_ls_data_t, dim3((unsigned)l->nb), b256, 0, st, (const double*)l->ud,
-                       (const double*)s->w, l->tr, s->nrows, (const LsCtl*)l->ctl);
-    hipLaunchKernelGGL((k_rows_scatter<double, double>),
-                       dim3((unsigned)std::max<int64_t>(1, ceil_div(s->ndn, 256))), b256, 0, st, R,
-                       (const double*)l->tr, l->y, 1, (CgCtl*)nullptr, 0, (const double*)nullptr,
-                       0, (const double*)nullptr, 0);
-  }
-  hipLaunchKernelGGL(k_ls_vupd, dim3((unsigned)l->nv), b256, 0, st, (const double*)l->y,
-                     sc, l->v, n, init, l->pv, (const LsCtl*)l->ctl);
-  hipLaunchKernelGGL(k_ls_step, dim3(1), b256, 0, st, (const double*)l->pv, l->nv, l->ctl, init);
-  hipLaunchKernelGGL(k_ls_xupd, dim3((unsigned)l->nv), b256, 0, st, l->v, l->h, l->hbar, l->x, n,
-                     init, l->px, (const LsCtl*)l->ctl);
-  if (!init)
-    hipLaunchKernelGGL(k_ls_test, dim3(1), b256, 0, st, (const double*)l->px, l->nv, l->ctl);
+// the partials' sum, where there are too many for every workgroup to read
+void ls_fold(const double** part, int* n, hipStream_t st) {
+  if (*n <= kLsPart) return;
+  hipLaunchKernelGGL(k_ls_fold, dim3(1), dim3(1024), 0, st, *part, *n, (double*)*part + *n);
+  *part += *n;
+  *n = 1;
 }
 
-__global__ void k_ls_setup(LsCtl* c, double atol, double btol, double ctol, int maxiter) {
-  LsCtl z = {};
+// |x|^2 as it stands after a step (see ls_fold)
+void ls_px(const Ls* l, const double** px, int* nx) {
+  const bool folded = l->nn > kLsPart;
+  *px = l->px + (folded ? l->nn : 0);
+  *nx = folded ? 1 : l->nn;
+}
+
+// One LSMR step from the state in slot `par` to the other one; init: the
+// start from u = b, to slot 0.
+void ls_bidiag(lsamd_fd_system* s, Ls* l, int init, int par, hipStream_t st) {
+  const int64_t n = s->n;
+  const RegW<double> w = make_regw<double>(s->reg);
+  const RowsDev R = rows_dev(s, false);
+  const dim3 nb((unsigned)l->nn), b256(256);
+  const LsCtl* in = l->ctl + (init ? 1 : par);
+  LsCtl* out = l->ctl + (init ? 0 : 1 - par);
+  const double *px, *pu = l->pu, *pv = l->pv;
+  int nx, nu = l->nd + l->nn, nv = l->nc + l->nn;
+  ls_px(l, &px, &nx);
+  hipLaunchKernelGGL(k_ls_fwd, dim3((unsigned)(l->nd + l->nn)), b256, 0, st,
+                     (const double*)l->xs, s->gd, w, (const double*)s->scale2, l->uw, l->urid, n,
+                     R, (const double*)s->w, (const double*)s->b, l->ud, l->nd, init,
+                     l->pu, in, (const LsMid*)l->mid);
+  ls_fold(&pu, &nu, st);
+  hipLaunchKernelGGL(k_ls_bwd, dim3((unsigned)(1 + l->nc + l->nn)), b256, 0, st,
+                     (const double*)l->uw, (const double*)l->urid, s->gd, sqrt(w.ridge), R,
+                     (const double*)l->cw, (const double*)l->ud, (const uint64_t*)l->mask,
+                     (const double*)l->sv, l->v, n, l->nc, init, pu, nu, l->pv, in,
+                     (const LsEst*)l->est + (1 - par), l->est + par, px, nx, l->mid);
+  ls_fold(&pv, &nv, st);
+  hipLaunchKernelGGL(k_ls_rot, nb, b256, 0, st, l->v, l->h, l->hbar, l->x, l->xs,
+                     (const double*)l->sv, n, init, pv, nv, l->px, in, out, l->est, l->mid);
+  px = l->px;
+  nx = l->nn;
+  ls_fold(&px, &nx, st);
+}
+
+__global__ void k_ls_setup(LsMid* m, double atol, double btol, double ctol, int maxiter) {
+  LsMid z = {};
   z.atol = atol;
   z.btol = btol;
   z.ctol = ctol;
   z.maxiter = maxiter;
-  *c = z;
+  *m = z;
 }
 
 }  // namespace
@@ -4514,23 +4519,25 @@ int ls_solve(lsamd_fd_system* s, const lsamd_lsmr_opts* o, double* c, lsamd_lsmr
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : n;
   const int maxiter = (int)std::min<int64_t>(maxiter64, 2000000000LL);
-  const int chunk = o->check_every > 0 ? o->check_every : 64;
+  int chunk = o->check_every > 0 ? o->check_every : 64;
+  chunk += chunk & 1;  // whole pairs: a step's slots are fixed at capture
   const double ctol = o->conlim > 0 ? 1.0 / o->conlim : 0.0;
-  hipLaunchKernelGGL(k_ls_setup, dim3(1), dim3(1), 0, st, l->ctl, o->atol, o->btol, ctol, maxiter);
-  const double* sc = s->minv64;
-  if (!o->scaling) {
-    if (!s->ones64) {
-      if (int rc = dalloc(s, &s->ones64, n)) return rc;
-      if (int rc = dalloc(s, &s->ones32, n)) return rc;
-      hipLaunchKernelGGL(k_fill_one, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st,
-                         s->ones64, s->ones32, n);
-    }
-    sc = s->ones64;
-  }
-  hipLaunchKernelGGL(k_zero_d, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, l->x, n);
-  ls_bidiag(s, l, sc, 1, st);
+  const dim3 nb((unsigned)ceil_div(n, 256)), b256(256);
+  const int64_t nw = ceil_div(n, 64);
+  hipLaunchKernelGGL(k_ls_setup, dim3(1), dim3(1), 0, st, l->mid, o->atol, o->btol, ctol,
+                     maxiter);
+  if (o->scaling)
+    hipLaunchKernelGGL(k_ls_sqrt, nb, b256, 0, st, (const double*)s->minv64, l->sv, n);
+  else
+    hipLaunchKernelGGL(k_fill_one, nb, b256, 0, st, l->sv, (float*)nullptr, n);
+  hipLaunchKernelGGL(k_pcg_gram_mask, dim3((unsigned)ceil_div(nw, 256)), b256, 0, st,
+                     (const int32_t*)s->dnode, s->ndn, nw, l->mask, l->base);
+  if (s->nnz > 0)
+    hipLaunchKernelGGL(k_ls_coef, dim3((unsigned)ceil_div(s->nnz, 256)), b256, 0, st,
+                       rows_dev(s, false), (const double*)s->w, l->cw, s->nnz);
+  ls_bidiag(s, l, 1, 0, st);
   LSAMD_CHECK_LAUNCH("lsmr init");
-  if (l->graph && (l->graph_chunk != chunk || l->graph_scale != sc)) {
+  if (l->graph && l->graph_chunk != chunk) {
     hipGraphExecDestroy(l->graph);
     l->graph = nullptr;
   }
@@ -4540,7 +4547,12 @@ int ls_solve(lsamd_fd_system* s, const lsamd_lsmr_opts* o, double* c, lsamd_lsmr
     LSAMD_HIP(hipStreamCreateWithFlags(&cs, hipStreamNonBlocking));
     hipGraph_t graph;
     LSAMD_HIP(hipStreamBeginCapture(cs, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < chunk; ++i) ls_bidiag(s, l, sc, 0, cs);
+    for (int i = 0; i < chunk; ++i) ls_bidiag(s, l, 0, i & 1, cs);
+    const double* px;
+    int nx;
+    ls_px(l, &px, &nx);
+    hipLaunchKernelGGL(k_ls_check, dim3(1), b256, 0, cs, (const LsCtl*)l->ctl,
+                       (const LsEst*)l->est + 1, l->est, px, nx, l->mid);
     hipError_t e = hipStreamEndCapture(cs, &graph);
     hipStreamDestroy(cs);
     if (e != hipSuccess) return fail(LSAMD_ERR_HIP, "graph capture failed (LSMR)");
@@ -4548,19 +4560,17 @@ int ls_solve(lsamd_fd_system* s, const lsamd_lsmr_opts* o, double* c, lsamd_lsmr
     hipGraphDestroy(graph);
     if (e != hipSuccess) return fail(LSAMD_ERR_HIP, "graph instantiate failed (LSMR)");
     l->graph_chunk = chunk;
-    l->graph_scale = sc;
   }
   for (;;) {
-    LSAMD_HIP(hipMemcpyAsync(l->host, l->ctl, sizeof(LsCtl), hipMemcpyDeviceToHost, st));
+    LSAMD_HIP(hipMemcpyAsync(l->host, l->mid, sizeof(LsMid), hipMemcpyDeviceToHost, st));
     LSAMD_HIP(hipStreamSynchronize(st));
     if (l->host->done) break;
     LSAMD_HIP(hipGraphLaunch(l->graph, st));
   }
-  hipLaunchKernelGGL(k_ls_out, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st,
-                     (const double*)l->x, sc, c, n);
+  hipLaunchKernelGGL(k_ls_out, nb, b256, 0, st, (const double*)l->x, (const double*)l->sv, c, n);
   LSAMD_CHECK_LAUNCH("lsmr out");
   LSAMD_HIP(hipStreamSynchronize(st));
-  const LsCtl* h = l->host;
+  const LsMid* h = l->host;
   inf->iterations = h->itn;
   inf->istop = h->istop;
   inf->normr = h->normr;
