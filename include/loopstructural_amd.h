@@ -277,6 +277,13 @@ int lsamd_fd_system_stencil_info(lsamd_fd_system* s, int32_t precision, int32_t*
  * Values: outside -> NaN, NaN coordinate -> 0.  Gradients: outside -> 0. */
 int lsamd_fd_evaluate(const lsamd_grid* g, const double* c, const double* pts, int64_t n,
                       double* values, double* grads, void* stream);
+/* The same, with scratch memory on the device (32-byte aligned, of the size that
+ * lsamd_fd_evaluate_scratch gives for this grid and n; 0: none is used; NULL:
+ * as lsamd_fd_evaluate).  Large evaluations at scattered points are faster
+ * with it, the results are the same. */
+int lsamd_fd_evaluate_scratch(const lsamd_grid* g, int64_t n, int64_t* bytes);
+int lsamd_fd_evaluate_with(const lsamd_grid* g, const double* c, const double* pts, int64_t n,
+                           double* values, double* grads, void* scratch, void* stream);
 
 /* A7 (use_regularisation_weight_scale): squared distance from every node
  * (np.linspace coordinates) to the nearest of m points (m,3); d2 (nnodes).

@@ -389,6 +389,8 @@ typedef double pair_t __attribute__((ext_vector_type(2), aligned(8)));
 // (1 - y is -(y - 1) exactly, and a product's sign does not change its
 // rounding).  False where a dividend is out of range (the caller takes
 // eval_point); cells past int32 node ids stay with 64-bit offsets.
+// QUAD: c is the corners' copy (k_eval_quad).
+template <bool QUAD>
 __device__ inline bool eval_point_known(const GridDev& g, const EvalGrid& e,
                                         const double* __restrict__ c, double px, double py,
                                         double pz, double* val, double* gr) {
@@ -407,9 +409,26 @@ __device__ inline bool eval_point_known(const GridDev& g, const EvalGrid& e,
   const int cy = cell(dy, g.hy, e.y[1], g.ny);
   const int cz = cell(dz, g.hz, e.y[2], g.nz);
   const int64_t nx = g.nx, nxy = nx * g.ny;
-  const double* c0 = c + cx + nx * cy + nxy * cz;
-  const pair_t c01 = *(const pair_t*)c0, c23 = *(const pair_t*)(c0 + nx);
-  const pair_t c45 = *(const pair_t*)(c0 + nxy), c67 = *(const pair_t*)(c0 + nxy + nx);
+  const int64_t at = cx + nx * cy + nxy * cz;
+  double cv[8];
+  auto ld = [](const double* p, double& a, double& b) {
+    const pair_t v = *(const pair_t*)p;
+    a = v.x;
+    b = v.y;
+  };
+  if constexpr (QUAD) {
+    const double* c0 = c + 4 * at;
+    ld(c0, cv[0], cv[2]);
+    ld(c0 + 2, cv[4], cv[6]);
+    ld(c0 + 4, cv[1], cv[3]);
+    ld(c0 + 6, cv[5], cv[7]);
+  } else {
+    const double* c0 = c + at;
+    ld(c0, cv[0], cv[1]);
+    ld(c0 + nx, cv[2], cv[3]);
+    ld(c0 + nxy, cv[4], cv[5]);
+    ld(c0 + nxy + nx, cv[6], cv[7]);
+  }
   const double ax = px - (g.ox + g.hx * (double)cx), ay = py - (g.oy + g.hy * (double)cy);
   const double az = pz - (g.oz + g.hz * (double)cz);
   ok = ok && div_known_dividend(ax) && div_known_dividend(ay) && div_known_dividend(az);
@@ -424,7 +443,6 @@ __device__ inline bool eval_point_known(const GridDev& g, const EvalGrid& e,
   for (const double d : {yz00, yz10, yz01, yz11, xz00, xz10, xz01, xz11, xy00, xy10, xy01, xy11})
     ok = ok && div_known_dividend(d);
   if (!ok) return false;
-  const double cv[8] = {c01.x, c01.y, c23.x, c23.y, c45.x, c45.y, c67.x, c67.y};
   const double w[8] = {xy00 * z1, xy10 * z1, xy01 * z1, xy11 * z1,
                        xy00 * z,  xy10 * z,  xy01 * z,  xy11 * z};
   double a[8];
@@ -450,14 +468,58 @@ __device__ inline bool eval_point_known(const GridDev& g, const EvalGrid& e,
   return true;
 }
 
+// Scattered points read four pieces of c each, from lines that no neighbour
+// shares: past the L2 that is what an evaluation waits for.  The table holds
+// for each node the four values c(i, j..j+1, k..k+1) side by side, so that a
+// point's eight corners are 64 bytes in one place: 1e7 random points on 128^3
+// nodes 598 -> 306 us, of which 25 us make the table.
+// Points in some order share their lines and would only pay for the table: 252
+// pairs of neighbours in four places of the list are looked at, and the
+// table is filled (ws[0] = 1) where fewer than half of them are within two
+// cells of each other.
+constexpr int kQuadHead = 16;      // doubles before the table
+constexpr int kQuadBlocks = 1024;  // every workgroup looks at the points: few
+__global__ __launch_bounds__(256) void k_eval_quad(GridDev g, EvalGrid e,
+                                                   const double* __restrict__ c,
+                                                   const double* __restrict__ pts, int64_t n,
+                                                   double* __restrict__ ws) {
+  __shared__ int sh[4];
+  const int t = threadIdx.x, wave = t >> 6, lane = t & 63;
+  const int64_t s = (n - 64) / 4 * wave + lane;  // n >= 64
+  float q[3];
+  const double o[3] = {g.ox, g.oy, g.oz};
+  int near = lane < 63;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    q[a] = (float)((pts[3 * s + a] - o[a]) * e.y[a]);
+    near = near && fabsf(q[a] - __shfl_down(q[a], 1, 64)) <= 2.f;
+  }
+  const int cnt = __popcll(__ballot(near));
+  if (lane == 0) sh[wave] = cnt;
+  __syncthreads();
+  const bool fill = sh[0] + sh[1] + sh[2] + sh[3] < 126;
+  if (blockIdx.x == 0 && t == 0) ws[0] = fill ? 1.0 : 0.0;
+  if (!fill) return;
+  const int64_t nx = g.nx, nxy = nx * g.ny, nn = nxy * g.nz;
+  typedef double quad_t __attribute__((ext_vector_type(4)));
+  for (int64_t i = (int64_t)blockIdx.x * 256 + t; i < nn; i += (int64_t)gridDim.x * 256) {
+    // past the last row or plane: any value, no cell has its corners there
+    const int64_t a = i + nx < nn ? i + nx : i, b = i + nxy < nn ? i + nxy : i;
+    const int64_t d = i + nx + nxy < nn ? i + nx + nxy : i;
+    *(quad_t*)(ws + kQuadHead + 4 * i) = quad_t{c[i], c[a], c[b], c[d]};
+  }
+}
+
 // Values and gradients at n points.  A workgroup's points come in, and its
 // gradients leave, through LDS in whole lines (a thread's own three doubles
 // lie 24 bytes from its neighbour's); they are streamed past the caches, whose
 // room belongs to c.  KNOWN: uniform grid with steps that div_known takes.
+// QUAD: corners from the table of k_eval_quad, where that has been filled.
 constexpr int kEvalBlock = 256;
-template <bool KNOWN>
+template <bool KNOWN, bool QUAD = false>
 __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
                                                          const double* __restrict__ c,
+                                                         const double* __restrict__ ws,
                                                          const double* __restrict__ pts,
                                                          int64_t n, double* __restrict__ vals,
                                                          double* __restrict__ grads) {
@@ -465,6 +527,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
   const int t = threadIdx.x;
   const int64_t b = (int64_t)blockIdx.x * kEvalBlock;
   const int m = (int)(n - b < kEvalBlock ? n - b : kEvalBlock);
+  const bool quad = QUAD && ws[0] != 0.0;
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (t + k * kEvalBlock < 3 * m)
@@ -473,8 +536,11 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
   double val = 0.0, gr[3] = {0.0, 0.0, 0.0};
   if (t < m) {
     const double px = sh[3 * t], py = sh[3 * t + 1], pz = sh[3 * t + 2];
-    if (!KNOWN || !eval_point_known(g, e, c, px, py, pz, &val, gr))
-      eval_point(g, c, px, py, pz, &val, gr);
+    bool ok = false;
+    if constexpr (KNOWN)
+      ok = quad ? eval_point_known<true>(g, e, ws + kQuadHead, px, py, pz, &val, gr)
+                : eval_point_known<false>(g, e, c, px, py, pz, &val, gr);
+    if (!ok) eval_point(g, c, px, py, pz, &val, gr);
     if (vals) __builtin_nontemporal_store(val, vals + b + t);
   }
   if (!grads) return;
@@ -613,22 +679,58 @@ extern "C" int lsamd_fd_build_rows(const lsamd_grid* g, int32_t kind, double* pt
   return LSAMD_OK;
 }
 
-extern "C" int lsamd_fd_evaluate(const lsamd_grid* g, const double* c, const double* pts,
-                                 int64_t n, double* values, double* grads, void* stream) {
+// Where the table of k_eval_quad is worth a look at the points.  Scattered
+// points without -> with it, us: 1e6 on 80^3 nodes (c fits an L2) 32 -> 42,
+// on 128^3 64 -> 51; 5e6 on 128^3 301 -> 163; 8e6 on 200^3 628 -> 339.  Points in order
+// pay 3 us for the look: of 18 us at 1e6, of 72 us at 5e6, nothing that
+// shows at 1e7.  So: c well past an L2, and points enough that 3 us don't count.
+constexpr int64_t kQuadNodesMin = 1 << 20, kQuadPointsMin = 1 << 22;
+static bool eval_quad_takes(const lsamd_grid* g, int64_t n) {
+  const int64_t nn = (int64_t)g->nnodes[0] * g->nnodes[1] * g->nnodes[2];
+  return nn >= kQuadNodesMin && n >= kQuadPointsMin && n >= nn && !g->axis_nodes[0] &&
+         div_known_divisor(g->step[0]) && div_known_divisor(g->step[1]) &&
+         div_known_divisor(g->step[2]);
+}
+
+extern "C" int lsamd_fd_evaluate_scratch(const lsamd_grid* g, int64_t n, int64_t* bytes) {
+  if (int rc = check_grid(g)) return rc;
+  if (!bytes) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate_scratch: NULL output");
+  const int64_t nn = (int64_t)g->nnodes[0] * g->nnodes[1] * g->nnodes[2];
+  *bytes = eval_quad_takes(g, n) ? (kQuadHead + 4 * nn) * 8 : 0;
+  return LSAMD_OK;
+}
+
+extern "C" int lsamd_fd_evaluate_with(const lsamd_grid* g, const double* c, const double* pts,
+                                      int64_t n, double* values, double* grads, void* scratch,
+                                      void* stream) {
   if (int rc = injected("evaluate")) return rc;
   if (int rc = check_grid(g)) return rc;
   if (n < 0) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate: n < 0");
   if (n == 0) return LSAMD_OK;
   if (!c || !pts) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate: NULL input");
+  if ((uintptr_t)scratch % 32) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate: scratch alignment");
   const dim3 nb((unsigned)ceil_div(n, kEvalBlock)), bs(kEvalBlock);
   const EvalGrid e = to_eval(*g);
-  if (!g->axis_nodes[0] && div_known_divisor(g->step[0]) && div_known_divisor(g->step[1]) &&
-      div_known_divisor(g->step[2]))
-    hipLaunchKernelGGL(k_evaluate<true>, nb, bs, 0, (hipStream_t)stream, to_dev(*g), e, c, pts, n,
+  const hipStream_t st = (hipStream_t)stream;
+  double* ws = (double*)scratch;
+  if (ws && eval_quad_takes(g, n)) {
+    hipLaunchKernelGGL(k_eval_quad, dim3(kQuadBlocks), dim3(256), 0, st, to_dev(*g), e, c, pts, n,
+                       ws);
+    hipLaunchKernelGGL((k_evaluate<true, true>), nb, bs, 0, st, to_dev(*g), e, c, ws, pts, n,
                        values, grads);
-  else
-    hipLaunchKernelGGL(k_evaluate<false>, nb, bs, 0, (hipStream_t)stream, to_dev(*g), e, c, pts,
-                       n, values, grads);
+  } else if (!g->axis_nodes[0] && div_known_divisor(g->step[0]) &&
+             div_known_divisor(g->step[1]) && div_known_divisor(g->step[2])) {
+    hipLaunchKernelGGL(k_evaluate<true>, nb, bs, 0, st, to_dev(*g), e, c, nullptr, pts, n, values,
+                       grads);
+  } else {
+    hipLaunchKernelGGL(k_evaluate<false>, nb, bs, 0, st, to_dev(*g), e, c, nullptr, pts, n,
+                       values, grads);
+  }
   LSAMD_CHECK_LAUNCH("k_evaluate");
   return LSAMD_OK;
+}
+
+extern "C" int lsamd_fd_evaluate(const lsamd_grid* g, const double* c, const double* pts,
+                                 int64_t n, double* values, double* grads, void* stream) {
+  return lsamd_fd_evaluate_with(g, c, pts, n, values, grads, nullptr, stream);
 }

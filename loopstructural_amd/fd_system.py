@@ -323,14 +323,31 @@ def build_rows(grid: _lib.Grid, kind: int, pts: torch.Tensor, weight_col: int, w
     return fixed_width_rows(cols, coef, b, w, norm, dof)
 
 
+_SCRATCH_POINTS = 1 << 22  # fewer points never use scratch memory
+
+
+def _evaluate_scratch(grid, n, dev):
+    """Scratch memory that an evaluation of n points would use, or None (also
+    where there is no room for it: it only saves time)."""
+    size = C.c_int64(0)
+    _lib.call("lsamd_fd_evaluate_scratch", C.byref(grid), n, C.byref(size))
+    if not size.value:
+        return None
+    try:
+        return torch.empty(size.value // 8, dtype=F64, device=dev)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def evaluate(grid: _lib.Grid, c: torch.Tensor, pts: torch.Tensor, values=True, gradients=False):
     pts = pts.to(_lib.device(), F64).contiguous()
     c = c.to(pts.device, F64).contiguous()
     n = pts.shape[0]
     v = torch.empty(n, dtype=F64, device=pts.device) if values else None
     g = torch.empty((n, 3), dtype=F64, device=pts.device) if gradients else None
-    _lib.call("lsamd_fd_evaluate", C.byref(grid), _lib.ptr(c), _lib.ptr(pts), n, _lib.ptr(v),
-              _lib.ptr(g), _lib.stream())
+    scratch = _evaluate_scratch(grid, n, pts.device) if n >= _SCRATCH_POINTS else None
+    _lib.call("lsamd_fd_evaluate_with", C.byref(grid), _lib.ptr(c), _lib.ptr(pts), n, _lib.ptr(v),
+              _lib.ptr(g), _lib.ptr(scratch), _lib.stream())
     return v, g
 
 

@@ -87,3 +87,55 @@ def test_p1_bit_exact(gi):
         # roundings of the largest
         scale = np.abs(c).max() / (np.array(h))
         assert np.all(np.nan_to_num(np.abs(g - r) / scale) <= 1e-14)
+
+
+@pytest.mark.parametrize("nn,n,kind", [
+    ((128, 128, 64), 1 << 22, "random"),     # the smallest grid and list with a table
+    ((131, 97, 83), (1 << 22) + 37, "random"),
+    ((131, 97, 83), (1 << 22) + 37, "ordered"),
+    ((131, 97, 83), (1 << 22) + 37, "mixed"),
+    ((128, 128, 63), 1 << 22, "random"),     # one plane less: none
+])
+def test_fd_corner_table_changes_nothing(nn, n, kind):
+    """Evaluation with scratch memory against the one without, bit for bit,
+    and a piece of it against the oracle."""
+    import ctypes as C
+
+    from loopstructural_amd import _lib
+    from loopstructural_amd import fd_system as fs
+
+    o, h = (10.0, -3.0, 0.5), (0.25, 0.5, 0.125)
+    cells = np.array(nn) - 1
+    rng = np.random.default_rng(n % 1000)
+    pts = np.array(o) + rng.uniform(-0.01, 1.01, (n, 3)) * cells * h
+    if kind != "random":
+        pts = pts[np.argsort(pts[:, 2], kind="stable")]
+        pts[:, 0] = o[0] + np.linspace(0.1, 0.9, n) * cells[0] * h[0]
+        pts[:, 1] = o[1] + 0.3 * cells[1] * h[1]
+    if kind == "mixed":
+        pts[n // 2:] = np.array(o) + rng.random((n - n // 2, 3)) * cells * h
+    pts[::100003] = np.nan
+    pts[7::100003] = np.array(o) + cells * h
+    c = rng.standard_normal(int(np.prod(nn)))
+    grid = _grid(o, cells, h)
+    size = C.c_int64(0)
+    _lib.call("lsamd_fd_evaluate_scratch", C.byref(grid), n, C.byref(size))
+    assert size.value == (0 if nn[2] == 63 else 8 * (16 + 4 * c.size))
+    dc, dp = torch.from_numpy(c).cuda(), torch.from_numpy(pts).cuda()
+    v, g = fs.evaluate(grid, dc, dp, True, True)
+    v0, g0 = torch.empty_like(v), torch.empty_like(g)
+    _lib.call("lsamd_fd_evaluate", C.byref(grid), _lib.ptr(dc), _lib.ptr(dp), n, _lib.ptr(v0),
+              _lib.ptr(g0), _lib.stream())
+    assert torch.equal(v.view(torch.int64), v0.view(torch.int64))
+    assert torch.equal(g.view(torch.int64), g0.view(torch.int64))
+    part = slice(0, 5000)
+    og = ofd.Grid(o, tuple(int(x) for x in cells), h)
+    with np.errstate(all="ignore"):
+        assert np.array_equal(v[part].cpu().numpy(), ofd.evaluate_value(og, c, pts[part]),
+                              equal_nan=True)
+        assert np.array_equal(g[part].cpu().numpy(), ofd.evaluate_gradient(og, c, pts[part]),
+                              equal_nan=True)
+    only, _ = fs.evaluate(grid, dc, dp, True, False)
+    assert torch.equal(only.view(torch.int64), v0.view(torch.int64))
+    _, only = fs.evaluate(grid, dc, dp, False, True)
+    assert torch.equal(only.view(torch.int64), g0.view(torch.int64))
