@@ -2945,13 +2945,26 @@ int mg_build_rows(lsamd_fd_system* s, Mg* m, hipStream_t st) {
     // regulariser-only diagonal of the coarse system, then its Gram diagonal
     launch_reg_diag(cs, st);
     if (nr > 0) {
-      hipLaunchKernelGGL(k_mg_rows, dim3((unsigned)ceil_div(nr, 128)), dim3(128), 0, st, prow,
-                         pcols, pcoef, nr, gf, gcd, 1, 0, cnt, (int32_t*)nullptr,
-                         (double*)nullptr);
+      const dim3 gb((unsigned)ceil_div(nr, kMgRowThreads)), tb(kMgRowThreads);
+      hipLaunchKernelGGL(k_mg_rows_box<true>, gb, tb, 0, st, prow, pcols, pcoef, nr, gf, gcd, 0,
+                         cnt, (int32_t*)nullptr, (double*)nullptr);
       LSAMD_HIP(hipMemcpyAsync(hc.data(), cnt, nr * 4, hipMemcpyDeviceToHost, st));
       LSAMD_HIP(hipStreamSynchronize(st));
-      int wc = 1;
-      for (int64_t r = 0; r < nr; ++r) wc = std::max(wc, (int)hc[r]);
+      auto widest = [&]() {
+        int w = 1;
+        for (int64_t r = 0; r < nr; ++r) w = std::max(w, (int)hc[r]);
+        return w;
+      };
+      int wc = widest();
+      const bool boxes = wc < kMgRowFar;
+      if (!boxes) {
+        hipLaunchKernelGGL(k_mg_rows, dim3((unsigned)ceil_div(nr, 128)), dim3(128), 0, st, prow,
+                           pcols, pcoef, nr, gf, gcd, 1, 0, cnt, (int32_t*)nullptr,
+                           (double*)nullptr);
+        LSAMD_HIP(hipMemcpyAsync(hc.data(), cnt, nr * 4, hipMemcpyDeviceToHost, st));
+        LSAMD_HIP(hipStreamSynchronize(st));
+        wc = widest();
+      }
       if (wc > 64) return fail(LSAMD_ERR_ARG, "multigrid: a data row spans too many cells");
       int32_t* ccols = nullptr;
       double* ccoef = nullptr;
@@ -2961,8 +2974,12 @@ int mg_build_rows(lsamd_fd_system* s, Mg* m, hipStream_t st) {
       if (int rc = mg_dalloc(m, &rptr, nr + 1)) return rc;
       hipLaunchKernelGGL(k_iota_rows, dim3((unsigned)ceil_div(nr + 1, 256)), dim3(256), 0, st,
                          rptr, nr + 1, (int64_t)wc);
-      hipLaunchKernelGGL(k_mg_rows, dim3((unsigned)ceil_div(nr, 128)), dim3(128), 0, st, prow,
-                         pcols, pcoef, nr, gf, gcd, 0, wc, (int32_t*)nullptr, ccols, ccoef);
+      if (boxes)
+        hipLaunchKernelGGL(k_mg_rows_box<false>, gb, tb, 0, st, prow, pcols, pcoef, nr, gf, gcd,
+                           wc, (int32_t*)nullptr, ccols, ccoef);
+      else
+        hipLaunchKernelGGL(k_mg_rows, dim3((unsigned)ceil_div(nr, 128)), dim3(128), 0, st, prow,
+                           pcols, pcoef, nr, gf, gcd, 0, wc, (int32_t*)nullptr, ccols, ccoef);
       LSAMD_CHECK_LAUNCH("multigrid rows");
       mg_give(m, own_row);
       mg_give(m, own_cols);

@@ -40,3 +40,32 @@ def test_iterations_and_minimiser(nodes, n_values, n_normals, most):
     _, info = s.solve(rtol=1e-10, multigrid=True)
     assert info["iterations"] <= most
     s.close()
+
+
+# extents of a row's columns in fine nodes: on the coarse grid boxes of at most
+# 4 nodes (slots) or more (the general form, which takes up to 64 coarse columns)
+@pytest.mark.parametrize("extent,entries", [(1, 8), (2, 5), (4, 12), (5, 12), (6, 10), (7, 6),
+                                            (30, 3), (5, 1)])
+def test_rows_of_any_extent_reach_the_minimiser(extent, entries):
+    from loopstructural_amd import _lib
+    from loopstructural_amd import fd_system as fs
+
+    nodes = np.array((34, 33, 41))
+    rng = np.random.default_rng(100 * extent + entries)
+    nrows, dev = 301, _lib.device()
+    lo = rng.integers(0, nodes - extent, (nrows, 1, 3))
+    c = lo + rng.integers(0, extent + 1, (nrows, entries, 3))
+    cols = c[..., 0] + nodes[0] * (c[..., 1] + nodes[1] * c[..., 2])
+    s = fs.FdSystem(_lib.make_grid((0, 0, 0), tuple(1 / (nodes - 1)), nodes),
+                    fs.reg_struct(W, tuple(int(n) for n in nodes), 1e-8))
+    coef = rng.uniform(0.2, 1.0, (nrows, entries)) / entries
+    s.set_rows(fs.FdRows(
+        torch.arange(nrows + 1, device=dev) * entries,
+        torch.from_numpy(cols.reshape(-1).astype(np.int32)).to(dev),
+        torch.from_numpy(coef.reshape(-1)).to(dev), torch.from_numpy(rng.normal(size=nrows)).to(dev),
+        torch.ones(nrows, dtype=torch.float64, device=dev), None, s.n))
+    x, info = s.solve(rtol=1e-11, multigrid=True)
+    assert info["converged"] and info["iterations"] <= 120
+    y, _ = s.solve(rtol=1e-13, precision="fp64")
+    assert float(torch.linalg.vector_norm(x - y) / torch.linalg.vector_norm(y)) < 1e-7
+    s.close()
