@@ -4495,7 +4495,7 @@ void ls_bidiag(lsamd_fd_system* s, Ls* l, int init, int par, hipStream_t st) {
   hipLaunchKernelGGL(k_ls_fwd, dim3((unsigned)(l->nd + l->nn)), b256, 0, st,
                      (const double*)l->xs, s->gd, w, (const double*)s->scale2, l->uw, l->urid, n,
                      R, (const double*)s->w, (const double*)s->b, l->ud, l->nd, init,
-                     l->pu, in, (const LsMid*)l->mid);
+                     l->pu, in, l->mid);
   ls_fold(&pu, &nu, st);
   hipLaunchKernelGGL(k_ls_bwd, dim3((unsigned)(1 + l->nc + l->nn)), b256, 0, st,
                      (const double*)l->uw, (const double*)l->urid, s->gd, sqrt(w.ridge), R,

@@ -19,7 +19,10 @@
 // Reductions are summed by every workgroup for itself (in the same order);
 // one records the scalars.  State alternates between two slots, so that no
 // launch writes what it reads, and the estimates of a step can be made again
-// at the end of a chunk.  The regulariser's part of u is kept as
+// at the end of a chunk.  For the same reason the end of a solve, recorded by
+// k_ls_bwd, stops k_ls_rot at once and k_ls_bwd only from the next k_ls_fwd on
+// (`halt`): had k_ls_bwd looked at `done` itself, the wavefronts of a
+// workgroup could have parted before a barrier.  The regulariser's part of u is kept as
 // uw = sqrt(W) u: its recurrence needs W itself, and the transposed product
 // neither weights nor roots at the 21 neighbours it gathers.
 // Eleven launches took 45 us per iteration at 26^3 nodes and 1000 rows, 55 us
@@ -47,6 +50,7 @@ struct LsMid {
   double normx, normr, normar, normA, condA;
   int skipv;  // beta == 0: v and alpha kept (as scipy's lsmr)
   int maxiter, itn, istop, done;
+  int halt;  // done as k_ls_fwd found it, for k_ls_bwd
 };
 
 // (c, s, r) with c a + s b = r, -s a + c b = 0 (stable); no jumps
@@ -154,10 +158,11 @@ __global__ __launch_bounds__(256) void k_ls_fwd(const double* __restrict__ xs, G
                                                 const double* __restrict__ b,
                                                 double* __restrict__ ud, int ndb, int init,
                                                 double* __restrict__ part, const LsCtl* c,
-                                                const LsMid* m) {
+                                                LsMid* m) {
   __shared__ double sh[4];
   double acc = 0.0;
   const int done = init ? 0 : m->done;
+  if (blockIdx.x == 0 && threadIdx.x == 0) m->halt = done;
   const double a = init ? 0.0 : c->fwd_coef;
   if ((int)blockIdx.x < ndb) {
     const double* coef = (const double*)R.coef;
@@ -270,7 +275,7 @@ __global__ __launch_bounds__(256) void k_ls_bwd(
     double* __restrict__ part, const LsCtl* c, const LsEst* ein, LsEst* eout,
     const double* __restrict__ px, int nx, LsMid* m) {
   __shared__ double sh[4];
-  const int done = init ? 0 : m->done;
+  const int done = init ? 0 : m->halt;
   if (blockIdx.x == 0) {
     if (init || c->itn == 0) return;
     const double x2 = pcg_total(px, nx, sh);
