@@ -62,8 +62,9 @@ class InterpolatorType(Enum):
 
 class _Lazy:
     """A ``constraints`` entry computed when it is read; ``keep``: once, and
-    then the stored array.  ``uniform``: (value, count) of an entry that holds
-    one value, for readers that need no array."""
+    then the stored array.  ``uniform``: a function that gives (value, count)
+    while the entry holds one value, for readers that need no array, and None
+    while it does not."""
 
     def __init__(self, fn, keep=False, uniform=None):
         self.fn, self.keep, self.uniform = fn, keep, uniform
@@ -1127,9 +1128,10 @@ class DiscreteInterpolator(GeologicalInterpolator):
             m = dict.__getitem__(con, "matrix")
             rows[fam] += int(m.shape[0])
             w = dict.__getitem__(con, "w")
-            if isinstance(w, _Lazy) and w.uniform is not None:
-                if w.uniform[1]:
-                    wts[fam].append(w.uniform)
+            same = w.uniform() if isinstance(w, _Lazy) and w.uniform else None
+            if same is not None:
+                if same[1]:
+                    wts[fam].append(same)
                 continue
             w = con["w"]
             if w is not None:
@@ -1481,7 +1483,9 @@ class FiniteDifferenceInterpolator(DiscreteInterpolator):
                 w = self.regularisation_scale[fam.centres()] * fam.weight
             return w
 
-        uniform = None if self.use_regularisation_weight_scale else (fam.weight, fam.nrows)
+        def uniform():
+            return None if self.use_regularisation_weight_scale else (fam.weight, fam.nrows)
+
         self.constraints[fam.name] = _Constraint(matrix=fam, b=np.zeros(fam.nrows),
                                                  w=_Lazy(weights, uniform=uniform))
 
@@ -1657,7 +1661,7 @@ class P1Interpolator(DiscreteInterpolator):
             # the solver needs the weight alone: 2e7 copies of it (128^3 cells)
             # took 30 ms of a 160 ms solve
             self.constraints[name] = _Constraint(matrix=fam, b=np.zeros(P), w=_Lazy(
-                lambda: np.full(P, float(w)), keep=True, uniform=(float(w), P)))
+                lambda: np.full(P, float(w)), keep=True, uniform=lambda: (float(w), P)))
         self.up_to_date = False
 
     def get_regularisation_sample_points(self):
