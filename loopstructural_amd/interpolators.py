@@ -94,10 +94,32 @@ class _Constraint(dict):
 
     def raw(self, key):
         """The stored object (device block, stencil family) behind ``key``."""
-        return dict.__getitem__(self, key)
+        return dict.__getitem__(self._kept(key), key)
 
     def get(self, key, default=None):
         return self[key] if key in self else default
+
+    def _kept(self, *keys):
+        """This dict, after its entries (or ``keys`` of them) that are computed
+        once and then stored have been: callers who go past ``__getitem__``
+        find the arrays."""
+        for key in keys or list(self):
+            v = dict.get(self, key)
+            if isinstance(v, _Lazy) and v.keep:
+                self[key]
+        return self
+
+    def items(self):
+        return dict.items(self._kept())
+
+    def values(self):
+        return dict.values(self._kept())
+
+    def copy(self):
+        return dict.copy(self._kept())
+
+    def pop(self, key, *default):
+        return dict.pop(self._kept(key), key, *default)
 
 
 def _weight_statistics(parts):

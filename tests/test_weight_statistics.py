@@ -1,4 +1,4 @@
-"""Weight statistics of the setup report from uniform parts."""
+"""Weights of uniform families: statistics of the setup report, stored entries."""
 import numpy as np
 import pytest
 import torch
@@ -32,3 +32,18 @@ def test_report_follows_the_weights_in_force():
         assert (fam.effective_weight_min, fam.effective_weight_max) == (w.min(), w.max())
         assert fam.effective_weight_mean == pytest.approx(w.mean(), rel=1e-14)
     assert w.max() > w.min()
+
+
+@pytest.mark.parametrize("read", [
+    lambda c: dict(c.items())["w"], lambda c: list(c.values())[list(c).index("w")],
+    lambda c: dict.__getitem__(c.copy(), "w"), lambda c: c.pop("w"), lambda c: c.raw("w"),
+    lambda c: c["w"]])
+def test_edge_jump_weights_are_an_array(read):
+    """However the entry is read, and once it has been, the same array."""
+    mesh = L.TetMesh(origin=np.zeros(3), nsteps=np.array([3, 3, 3]), step_vector=np.ones(3))
+    interp = L.P1Interpolator(mesh)
+    interp.minimise_edge_jumps(0.3)
+    con = interp.constraints["edge jump"]
+    w = read(con)
+    assert isinstance(w, np.ndarray) and w.shape == con["b"].shape and (w == 0.3).all()
+    assert "w" not in con or con["w"] is w
