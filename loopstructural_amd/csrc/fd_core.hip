@@ -5582,8 +5582,6 @@ int lsamd_batch_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const doubl
       inf[i].threshold = s->bctl_host[i].thr;
     }
   } else if (o->precision == LSAMD_FP32) {
-    if (int rc = pcg_gram_ensure(s, st)) return rc;
-    if (int rc = pcg_buffer(s, &s->pcg_b32)) return rc;
     const double inner = o->inner_rtol > 0 ? o->inner_rtol : 1e-4;
     const int64_t max_outer = o->max_outer > 0 ? o->max_outer : 50;
     hipLaunchKernelGGL(k_zero_d, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st, c, n);
