@@ -1194,7 +1194,7 @@ struct lsamd_fd_system {
   float* minv32 = nullptr;
   // work
   // Jacobi PCG (pcg.hpp): the data term by node (gram_state: 0 not built for
-  // these rows, 1 built, 2 its rows are too long), the direction's second
+  // these rows, 1 built, 2 row form), the direction's second
   // buffer per precision, the partials of r.z and of the data term
   int gram_state = 0, gram_width = 0;
   int32_t *gram_col = nullptr, *gram_base = nullptr;
@@ -1292,6 +1292,12 @@ int rbuf(lsamd_fd_system* s, int slot, P** p, int64_t count) {
   }
   *p = (P*)e.first;
   return LSAMD_OK;
+}
+
+void rbuf_free(lsamd_fd_system* s, int slot) {
+  if (s->rpool.empty()) return;
+  dfree(s, s->rpool[slot].first);
+  s->rpool[slot] = {nullptr, 0};
 }
 
 RowsDev rows_dev(const lsamd_fd_system* s, bool fp32) {
@@ -1666,7 +1672,8 @@ int launch_apply(lsamd_fd_system* s, const T* x, T* y, T* t, CgCtl* ctl, hipStre
 
 // Data term by node of the current rows, built on the first Jacobi solve
 // after they changed (gram_state).  Rows that couple a node with more than
-// kGramCap others, or more than kGramNodesMax data nodes, keep the row form.
+// kGramCap others, or more than kGramNodesMax data nodes, keep the row form;
+// so do rows whose node rows there is no memory for, as these only save time.
 
 int pcg_gram_ensure(lsamd_fd_system* s, hipStream_t st) {
   if (s->gram_state || s->nrows == 0) return LSAMD_OK;
@@ -1675,14 +1682,19 @@ int pcg_gram_ensure(lsamd_fd_system* s, hipStream_t st) {
   if (nd > kGramNodesMax) return LSAMD_OK;
   int* over = nullptr;
   double* gq = nullptr;
-  if (int rc = rbuf(s, kRsGramCol, &s->gram_col, nd * kGramCap)) return rc;
-  if (int rc = rbuf(s, kRsGramV64, &s->gram_v64, nd * kGramCap)) return rc;
-  if (int rc = rbuf(s, kRsGramV32, &s->gram_v32, nd * kGramCap)) return rc;
-  if (int rc = rbuf(s, kRsGramMask, &s->gram_mask, nw)) return rc;
-  if (int rc = rbuf(s, kRsGramBase, &s->gram_base, nw)) return rc;
-  if (int rc = rbuf(s, kRsGramQ, &gq, nd)) return rc;
-  if (int rc = rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB))) return rc;
-  if (int rc = rbuf(s, kRsGramOver, &over, 2)) return rc;
+  if (injected("node_rows") || rbuf(s, kRsGramCol, &s->gram_col, nd * kGramCap) ||
+      rbuf(s, kRsGramV64, &s->gram_v64, nd * kGramCap) ||
+      rbuf(s, kRsGramV32, &s->gram_v32, nd * kGramCap) ||
+      rbuf(s, kRsGramMask, &s->gram_mask, nw) || rbuf(s, kRsGramBase, &s->gram_base, nw) ||
+      rbuf(s, kRsGramQ, &gq, nd) ||
+      rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB)) ||
+      rbuf(s, kRsGramOver, &over, 2)) {
+    for (int k : {kRsGramCol, kRsGramV64, kRsGramV32, kRsGramMask, kRsGramBase, kRsGramQ,
+                  kRsGramPart, kRsGramOver})
+      rbuf_free(s, k);
+    (void)hipGetLastError();  // the failed allocation's, which the next launch would report
+    return LSAMD_OK;
+  }
   s->gram_q = gq;
   // rows of half the width first where one row set's columns suggest it
   // (four-node rows); a longer one costs a second pass

@@ -55,3 +55,33 @@ def test_batch_solves_take_none():
         taken, _ = _taken(lambda: bs.solve(rtol=1e-3, maxiter=8, precision="fp32"))
     assert taken <= SLACK, taken
     bs.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_solve_without_room_for_them(monkeypatch, precision):
+    """The allocation fails on one handle and not on another: both solve, to
+    the same field, and nothing stays behind; the next row set tries again."""
+    from loopstructural_amd import fd_system as fs
+
+    g, reg, n = _grid()
+    kw = {"rtol": 1e-9, "precision": precision}
+    fields = []
+    for fail in (True, False):
+        s = fs.FdSystem(g, reg)
+        s.set_rows(_single_node_rows(n, 10))
+        s.solve(**kw)
+        s.set_rows(_single_node_rows(n, 100_000))
+        if fail:
+            monkeypatch.setenv("LSAMD_FAULT_INJECT", "node_rows")
+        taken, (c, info) = _taken(lambda: s.solve(**kw))
+        monkeypatch.delenv("LSAMD_FAULT_INJECT", raising=False)
+        assert info["converged"]
+        fields.append(c)
+        assert (taken <= SLACK) == fail, (fail, taken)
+        if fail:
+            s.set_rows(_single_node_rows(n, 99_000))
+            taken, (_, info) = _taken(lambda: s.solve(**kw))
+            assert info["converged"] and taken > SLACK
+        s.close()
+    err = float((fields[0] - fields[1]).norm() / fields[1].norm())
+    assert err <= 1e-6, err
