@@ -1193,10 +1193,10 @@ struct lsamd_fd_system {
   double* minv64 = nullptr;
   float* minv32 = nullptr;
   // work
-  // Jacobi PCG (pcg.hpp): the data term by node (gram_state: 0 not built for
-  // these rows, 1 built, 2 row form), the direction's second
+  // Jacobi PCG (pcg.hpp): the data term by node (gram_state, FP64 and FP32: 0
+  // not built for these rows, 1 built, 2 row form), the direction's second
   // buffer per precision, the partials of r.z and of the data term
-  int gram_state = 0, gram_width = 0;
+  int gram_state[2] = {0, 0}, gram_width = 0;
   int32_t *gram_col = nullptr, *gram_base = nullptr;
   double* gram_v64 = nullptr;
   float* gram_v32 = nullptr;
@@ -1670,40 +1670,53 @@ int launch_apply(lsamd_fd_system* s, const T* x, T* y, T* t, CgCtl* ctl, hipStre
   return LSAMD_OK;
 }
 
-// Data term by node of the current rows, built on the first Jacobi solve
-// after they changed (gram_state).  Rows that couple a node with more than
-// kGramCap others, or more than kGramNodesMax data nodes, keep the row form;
-// so do rows whose node rows there is no memory for, as these only save time.
-
-int pcg_gram_ensure(lsamd_fd_system* s, hipStream_t st) {
-  if (s->gram_state || s->nrows == 0) return LSAMD_OK;
-  s->gram_state = 2;
+// Data term by node of the current rows, in FP64 (w64), FP32 (w32) or both,
+// built on the first solve that asks for it after they changed (gram_state).
+// Rows that couple a node with more than kGramCap others, or more than
+// kGramNodesMax data nodes, keep the row form; so do rows whose node rows there
+// is no memory for, as these only save time.
+int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, hipStream_t st) {
+  int* state = s->gram_state;
+  w64 = w64 && !state[0];
+  w32 = w32 && !state[1];
+  if (!(w64 || w32) || s->nrows == 0) return LSAMD_OK;
+  // what the other precision found for these rows: its columns serve both
+  const int other = w64 ? state[1] : state[0];
+  const bool add = !(w64 && w32) && other == 1;
+  if (w64) state[0] = 2;
+  if (w32) state[1] = 2;
   const int64_t nd = s->ndn, nw = ceil_div(s->n, 64);
-  if (nd > kGramNodesMax) return LSAMD_OK;
-  int* over = nullptr;
-  double* gq = nullptr;
-  if (injected("node_rows") || rbuf(s, kRsGramCol, &s->gram_col, nd * kGramCap) ||
-      rbuf(s, kRsGramV64, &s->gram_v64, nd * kGramCap) ||
-      rbuf(s, kRsGramV32, &s->gram_v32, nd * kGramCap) ||
-      rbuf(s, kRsGramMask, &s->gram_mask, nw) || rbuf(s, kRsGramBase, &s->gram_base, nw) ||
-      rbuf(s, kRsGramQ, &gq, nd) ||
-      rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB)) ||
-      rbuf(s, kRsGramOver, &over, 2)) {
-    for (int k : {kRsGramCol, kRsGramV64, kRsGramV32, kRsGramMask, kRsGramBase, kRsGramQ,
-                  kRsGramPart, kRsGramOver})
-      rbuf_free(s, k);
-    (void)hipGetLastError();  // the failed allocation's, which the next launch would report
-    return LSAMD_OK;
-  }
-  s->gram_q = gq;
+  if (nd > kGramNodesMax || (!(w64 && w32) && other == 2)) return LSAMD_OK;
   // rows of half the width first where one row set's columns suggest it
   // (four-node rows); a longer one costs a second pass
-  int width = s->nnz <= 5 * s->nrows ? kGramCap / 2 : kGramCap;
+  int width = add ? s->gram_width : s->nnz <= 5 * s->nrows ? kGramCap / 2 : kGramCap;
+  int* over = nullptr;
+  double* gq = nullptr;
   for (;;) {
+    if (injected("node_rows") || (w64 && rbuf(s, kRsGramV64, &s->gram_v64, nd * width)) ||
+        (w32 && rbuf(s, kRsGramV32, &s->gram_v32, nd * width)) ||
+        rbuf(s, kRsGramCol, &s->gram_col, nd * width) ||
+        rbuf(s, kRsGramMask, &s->gram_mask, nw) || rbuf(s, kRsGramBase, &s->gram_base, nw) ||
+        rbuf(s, kRsGramQ, &gq, nd) ||
+        rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB)) ||
+        rbuf(s, kRsGramOver, &over, 2)) {
+      if (w64) rbuf_free(s, kRsGramV64);
+      if (w32) rbuf_free(s, kRsGramV32);
+      if (!add)
+        for (int k : {kRsGramCol, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart, kRsGramOver})
+          rbuf_free(s, k);
+      (void)hipGetLastError();  // the failed allocation's, which the next launch would report
+      return LSAMD_OK;
+    }
+    s->gram_q = gq;
     LSAMD_HIP(hipMemsetAsync(over, 0, 2 * sizeof(int), st));
     hipLaunchKernelGGL(k_pcg_gram_build, dim3((unsigned)ceil_div(nd, 64)), dim3(64), 0, st,
                        rows_dev(s, false), (const double*)s->coef64, (const double*)s->w2_64,
-                       width, s->gram_col, s->gram_v64, s->gram_v32, over);
+                       width, add ? (int32_t*)nullptr : s->gram_col,
+                       w64 ? s->gram_v64 : (double*)nullptr, w32 ? s->gram_v32 : (float*)nullptr,
+                       over);
+    LSAMD_CHECK_LAUNCH("data term by node");
+    if (add) break;
     hipLaunchKernelGGL(k_pcg_gram_mask, dim3((unsigned)ceil_div(nw, 256)), dim3(256), 0, st,
                        (const int32_t*)s->dnode, nd, nw, s->gram_mask, s->gram_base);
     LSAMD_CHECK_LAUNCH("data term by node");
@@ -1715,14 +1728,15 @@ int pcg_gram_ensure(lsamd_fd_system* s, hipStream_t st) {
     width = kGramCap;
   }
   s->gram_width = width;
-  s->gram_state = 1;
+  if (w64) state[0] = 1;
+  if (w32) state[1] = 1;
   return LSAMD_OK;
 }
 
 GramDev gram_dev(const lsamd_fd_system* s, bool f32) {
   GramDev G;
   memset(&G, 0, sizeof(G));
-  if (s->gram_state != 1) return G;
+  if (s->gram_state[f32] != 1) return G;
   G.ndn = s->ndn;
   G.node = s->dnode;
   G.col = s->gram_col;
@@ -1787,7 +1801,7 @@ int launch_iteration(lsamd_fd_system* s, int par, T* x, T* r, T* pa, T* pb, T* q
     nrow = ng;
   }
   const double* part_g = s->pcg_pg;
-  if (s->nrows > 0 && s->gram_state != 1) {
+  if (s->nrows > 0 && s->gram_state[f32] != 1) {
     const RowsDev R = rows_dev(s, f32);
     nrow = (int)ceil_div(s->nrows, 256);
     part_g = s->part_rows;
@@ -2261,7 +2275,7 @@ MgSm mg_sm(const MgLevel& L) {
   return S;
 }
 
-// y += the data term of x by node, one launch (level 0; gram_state == 1);
+// y += the data term of x by node, one launch (level 0, where it is built);
 // partials of x.Gx to part where given
 template <typename T>
 void launch_gram_add(const lsamd_fd_system* s, const T* x, T* y, double* part, const CgCtl* ctl,
@@ -2281,7 +2295,7 @@ void mg_level_apply(const MgLevel& L, const float* x, float* y, const CgCtl* ctl
   if (L.owned) {
     hipLaunchKernelGGL(k_mg_apply, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st,
                        mg_dev(L), x, y, ctl);
-  } else if (L.sys->gram_state == 1) {
+  } else if (L.sys->gram_state[1] == 1) {
     launch_stencil<float>(L.sys, x, y, ctl, st, L.sys->zc[1]);
     launch_gram_add<float>(L.sys, x, y, nullptr, ctl, st);
   } else {
@@ -2324,7 +2338,7 @@ int mg_level_apply64(const MgLevel& L, const double* x, double* y, hipStream_t s
       hipLaunchKernelGGL(k_mg_apply64<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0, st,
                          mg_dev<double>(L), x, y);
     });
-  } else if (s->gram_state == 1) {
+  } else if (s->gram_state[0] == 1) {
     launch_stencil<double>(s, x, y, s->ctl_apply, st, s->zc[0]);
     launch_gram_add<double>(s, x, y, nullptr, s->ctl_apply, st);
   } else {
@@ -3130,9 +3144,9 @@ int launch_fcg_iteration(lsamd_fd_system* s, hipStream_t st) {
                      (const double*)s->pcg_pr, vb, s->ctl);
   int64_t nq = -1;
   int ng = 0;
-  if (s->gram_state == 1 || s->nrows == 0) {
+  if (s->gram_state[0] == 1 || s->nrows == 0) {
     nq = launch_stencil<double>(s, (const double*)s->p64, s->q64, s->ctl, st, s->zc[0]);
-    if (s->gram_state == 1) {
+    if (s->gram_state[0] == 1) {
       launch_gram_add<double>(s, (const double*)s->p64, s->q64, s->pcg_pg, s->ctl, st);
       ng = (int)ceil_div(s->ndn * kGramLanes, 256);
     }
@@ -3224,7 +3238,7 @@ int mg_ensure(lsamd_fd_system* s, hipStream_t st) {
 int mg_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const double* b, double* c,
              lsamd_solve_info* inf, hipStream_t st) {
   if (s->op != 0) return fail(LSAMD_ERR_ARG, "multigrid is available for FD systems only");
-  if (int rc = pcg_gram_ensure(s, st)) return rc;
+  if (int rc = pcg_gram_ensure(s, true, true, st)) return rc;
   if (int rc = mg_ensure(s, st)) return rc;
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : 10 * n;
@@ -4920,7 +4934,7 @@ int lsamd_fd_system_set_rows(lsamd_fd_system* s, int64_t nrows, int64_t nnz,
   s->t64 = nullptr;
   s->t32 = nullptr;
   s->part_rows = nullptr;
-  s->gram_state = 0;
+  s->gram_state[0] = s->gram_state[1] = 0;
   LSAMD_HIP(hipMemsetAsync(s->ctl, 0, sizeof(CgCtl), st));
   LSAMD_HIP(hipMemsetAsync(s->ctl_apply, 0, sizeof(CgCtl), st));
   s->nrows = nrows;
@@ -5130,7 +5144,7 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
       if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
     if (int rc = launch_init<double>(s, b, minv64, s->x64, s->r64, o->rtol, o->atol, maxiter, st))
       return rc;
-    if (int rc = pcg_gram_ensure(s, st)) return rc;
+    if (int rc = pcg_gram_ensure(s, true, false, st)) return rc;
     if (int rc = pcg_buffer(s, &s->pcg_b64)) return rc;
     if (int rc = run_pcg<double>(s, chunk, s->x64, s->r64, s->p64, s->pcg_b64, s->q64, s->t64,
                                  minv64, st))
@@ -5149,7 +5163,7 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
       if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
       if (int rc = ensure_tuned<float>(s, s->p32, s->q32, st)) return rc;
     }
-    if (int rc = pcg_gram_ensure(s, st)) return rc;
+    if (int rc = pcg_gram_ensure(s, false, true, st)) return rc;
     if (int rc = pcg_buffer(s, &s->pcg_b32)) return rc;
     const double inner = o->inner_rtol > 0 ? o->inner_rtol : 1e-4;
     const int64_t max_outer = o->max_outer > 0 ? o->max_outer : 50;

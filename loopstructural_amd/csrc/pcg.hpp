@@ -24,7 +24,9 @@ namespace lsamd {
 
 constexpr int kGramCap = 32;       // most entries of a node's Gram row (27 for rows of one cell)
 constexpr int kGramLanes = 8;      // threads per row, two or four entries each
-constexpr int64_t kGramNodesMax = 500000;  // 192 MB of rows; larger data terms keep the row form
+// larger data terms keep the row form: the rows of this many nodes take 192 MB
+// in FP64, 128 MB in FP32 and 256 MB in both
+constexpr int64_t kGramNodesMax = 500000;
 constexpr int kPcgBlocks = 2048;   // partials of the vector kernels
 constexpr int kPcgPartMax = 2048;  // operator partials that every workgroup sums itself
 
@@ -49,8 +51,9 @@ struct GramDev {
 };
 
 // one thread per data node: its distinct columns in order of appearance and
-// the sums of w^2 a_i a_j, in rows of kGramCap; over[0] when a row needs more,
-// over[1] when one needs more than half
+// the sums of w^2 a_i a_j, in rows of `width` (col, v64 and v32: those given);
+// over[0] when a row needs more than kGramCap, over[1] when one needs more than
+// half of that
 __global__ __launch_bounds__(64) void k_pcg_gram_build(RowsDev R, const double* __restrict__ coef,
                                                        const double* __restrict__ w2, int width,
                                                        int32_t* __restrict__ col,
@@ -85,9 +88,9 @@ __global__ __launch_bounds__(64) void k_pcg_gram_build(RowsDev R, const double* 
   const int32_t self = R.dnode[d];
   for (int k = 0; k < width; ++k) {
     const double v = k < m ? lv[k][t] : 0.0;
-    col[d * width + k] = k < m ? lc[k][t] : self;
-    v64[d * width + k] = v;
-    v32[d * width + k] = (float)v;
+    if (col) col[d * width + k] = k < m ? lc[k][t] : self;
+    if (v64) v64[d * width + k] = v;
+    if (v32) v32[d * width + k] = (float)v;
   }
 }
 

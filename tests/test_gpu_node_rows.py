@@ -85,3 +85,34 @@ def test_solve_without_room_for_them(monkeypatch, precision):
         s.close()
     err = float((fields[0] - fields[1]).norm() / fields[1].norm())
     assert err <= 1e-6, err
+
+
+def test_memory_is_that_of_the_width_and_the_precision():
+    """Rows of 16 entries; FP64, then FP32 beside it, then the other way round
+    on a second handle; the fields agree with a multigrid solve (which builds
+    both in one pass)."""
+    from loopstructural_amd import fd_system as fs
+
+    g, reg, n = _grid()
+    count = 170_000
+    col, v64, v32 = (1.25 * 16 * k * count for k in (4, 8, 4))
+    per_node = 1.25 * 8 * count + n  # the product's compact result, partials, masks
+    fields = []
+    for order in (("fp64", "fp32"), ("fp32", "fp64"), ("mg",)):
+        s = fs.FdSystem(g, reg)
+        run = {p: (lambda p=p: s.solve(rtol=1e-9, precision=p)) for p in ("fp64", "fp32")}
+        run["mg"] = lambda: s.solve(rtol=1e-9, multigrid=True)
+        s.set_rows(_single_node_rows(n, 10))
+        for p in order:
+            run[p]()
+        s.set_rows(_single_node_rows(n, count))
+        for first, p in zip((True, False), order):
+            taken, (c, info) = _taken(run[p])
+            assert info["converged"]
+            fields.append(c)
+            if p != "mg":
+                room = (v32 if p == "fp32" else v64) + (col + per_node if first else 0)
+                assert taken <= room + SLACK, (order, p, taken, room)
+        s.close()
+    for c in fields[:-1]:
+        assert float((c - fields[-1]).norm() / fields[-1].norm()) <= 1e-6
