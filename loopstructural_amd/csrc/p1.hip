@@ -363,7 +363,8 @@ __global__ void k_p1_build_rows(P1Mesh m, int kind, const double* __restrict__ p
 // values cv.  Along each axis the gradient is the difference over the edge at
 // the apex of a corner tet, half the difference of two corner pairs of the
 // centre tet, over the cell's width (the entries of the element gradient are
-// 0, +-1 and +-1/2 over it).
+// 0, +-1 and +-1/2 over it).  A corner with the entry 0 still makes the
+// component NaN where its value is not finite, as in the sum over all four.
 __device__ inline void p1_field(const P1Mesh& m, const TetLoc& L, const double* __restrict__ c,
                                 double* val, double* gr) {
   const int odd = (L.cell[0] + L.cell[1] + L.cell[2]) & 1;
@@ -386,7 +387,10 @@ __device__ inline void p1_field(const P1Mesh& m, const TetLoc& L, const double* 
     const int nb = cr[0] ^ (1 << a);  // the apex's neighbour along the axis
     const double other = cr[1] == nb ? cv[1] : (cr[2] == nb ? cv[2] : cv[3]);
     const double edge = (cr[0] >> a) & 1 ? cv[0] - other : other - cv[0];
-    gr[a] = (L.loc == 0 ? mid[a] : edge) /
+    double off = 0.0;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) off += cr[k] == nb ? 0.0 : 0.0 * cv[k];
+    gr[a] = (L.loc == 0 ? mid[a] : edge + off) /
             (node_pos(m, a, L.cell[a] + 1) - node_pos(m, a, L.cell[a]));
   }
 }

@@ -139,3 +139,29 @@ def test_fd_corner_table_changes_nothing(nn, n, kind):
     assert torch.equal(only.view(torch.int64), v0.view(torch.int64))
     _, only = fs.evaluate(grid, dc, dp, False, True)
     assert torch.equal(only.view(torch.int64), g0.view(torch.int64))
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("support", ["fd", "p1"])
+def test_coefficients_that_are_not_finite(support, bad):
+    """A NaN or infinite coefficient reaches every value and every gradient
+    component that the sum over the cell's or the tet's corners gives it, and
+    no other point."""
+    from loopstructural_amd import fd_system as fs
+
+    o, cells, h = GRIDS[0]
+    og = ofd.Grid(o, cells, h) if support == "fd" else op1.TetMesh(o, cells, h)
+    pts = np.array(o) + np.random.default_rng(5).uniform(0, 1, (3000, 3)) * np.array(cells) * h
+    c = np.random.default_rng(6).standard_normal(og.n_nodes)
+    c[::17] = bad
+    with np.errstate(all="ignore"):
+        if support == "fd":
+            rv, rg = ofd.evaluate_value(og, c, pts), ofd.evaluate_gradient(og, c, pts)
+        else:
+            rv, rg = og.evaluate_value(pts, c), og.evaluate_gradient(pts, c)
+    f = fs.evaluate if support == "fd" else fs.p1_evaluate
+    v, g = f(_grid(o, cells, h), torch.from_numpy(c), torch.from_numpy(pts), True, True)
+    for got, want in ((v.cpu().numpy(), rv), (g.cpu().numpy(), rg)):
+        assert 0 < np.isfinite(want).sum() < want.size
+        for kind in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(kind(got), kind(want)), kind
