@@ -266,10 +266,11 @@ int lsamd_fd_system_time_multi(lsamd_fd_system* s, int32_t kernel, int32_t iters
  * 64 x 8 tiles, 1008 / 1016 / 1032 for those z-chunks with planes copied
  * straight into LDS, or 2008 / 2016 / 2032 for register-staged planes on
  * 32 x 16 tiles (0 = exact per-node kernel: an axis has < 7 nodes or a
- * per-node weight scale is set; also 0 while nothing has timed the forms: a
- * Jacobi solve of a grid of up to 768 tiles of 16 x 8 x 4 nodes does not), and the
+ * per-node weight scale is set; also 0 before the first apply/solve), and the
  * timed forms in that order (8, 16, 32, 1008, 1016, 1032, 2008, 2016, 2032)
- * in microseconds (tune_us[9], nullable, -1 = skipped). */
+ * in microseconds (tune_us[9], nullable, -1 = skipped).  Where only Jacobi solves
+ * of a small grid (up to 768 tiles of 16 x 8 x 4 nodes) have run, which take
+ * none of these forms, the first call times them, on the null stream. */
 int lsamd_fd_system_stencil_info(lsamd_fd_system* s, int32_t precision, int32_t* zc,
                                  float* tune_us);
 

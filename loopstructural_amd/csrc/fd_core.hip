@@ -1172,6 +1172,9 @@ struct lsamd_fd_system {
   hipGraphExec_t bgraph[2] = {nullptr, nullptr};
   int bgraph_chunk[2] = {0, 0};
   int zc[2] = {0, 0};          // tuned z-chunk per precision (0: not tuned yet)
+  // solved by k_pcg_tile, which takes none of the forms: they are timed when
+  // they are asked for (lsamd_fd_system_stencil_info)
+  bool untimed[2] = {false, false};
   float tune_us[2][9] = {{0}};  // timings of the stencil forms kStCand
   // data rows
   int64_t nrows = 0, nnz = 0, ndn = 0;
@@ -1593,6 +1596,17 @@ int tune_p1(lsamd_fd_system* s, T* x, T* y, hipStream_t st) {
   return LSAMD_OK;
 }
 
+// the form that LSAMD_STENCIL_ZC names, if this system can take it
+template <typename T>
+void pin_stencil(lsamd_fd_system* s) {
+  const char* e = getenv("LSAMD_STENCIL_ZC");
+  const int pi = sizeof(T) == 4 ? 1 : 0, v = e ? atoi(e) : 0;
+  for (int c = 0; c < kNStCand; ++c)
+    if (s->regular && !s->zc[pi] && v == kStCand[c] &&
+        (v < kDmaZc || v > kTile32 || dma_fits(s->gd, sizeof(T))))
+      s->zc[pi] = v;
+}
+
 // Autotuner: time each stencil form (z-chunk 8/16/32 with register-staged
 // planes, 8/16 with LDS-DMA staged planes; HIP events) and keep the fastest.
 // LSAMD_STENCIL_ZC in the environment pins the choice (a kStCand value).
@@ -1605,14 +1619,8 @@ int ensure_tuned(lsamd_fd_system* s, T* x, T* y, hipStream_t st) {
     s->zc[pi] = 1;
     return LSAMD_OK;
   }
-  if (const char* e = getenv("LSAMD_STENCIL_ZC")) {
-    const int v = atoi(e);
-    for (int c = 0; c < kNStCand; ++c)
-      if (v == kStCand[c] && (v < kDmaZc || v > kTile32 || dma_fits(s->gd, sizeof(T)))) {
-        s->zc[pi] = v;
-        return LSAMD_OK;
-      }
-  }
+  pin_stencil<T>(s);
+  if (s->zc[pi]) return LSAMD_OK;
   hipEvent_t e0, e1;
   LSAMD_HIP(hipEventCreate(&e0));
   LSAMD_HIP(hipEventCreate(&e1));
@@ -5138,6 +5146,14 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
   // the tile form takes no timed stencil (the FP64 residuals of the mixed
   // solve, a handful, take the form of a small grid)
   const bool timed = pcg_tiles(s) == 0;
+  if (!timed) {
+    pin_stencil<double>(s);
+    s->untimed[0] = true;
+    if (o->precision == LSAMD_FP32) {
+      pin_stencil<float>(s);
+      s->untimed[1] = true;
+    }
+  }
   if (o->precision == LSAMD_FP64) {
     if (int rc = ensure_work(s, false)) return rc;
     if (timed)
@@ -5395,6 +5411,13 @@ int lsamd_fd_system_stencil_info(lsamd_fd_system* s, int32_t precision, int32_t*
                                  float* tune_us) {
   if (!s || !zc) return fail(LSAMD_ERR_ARG, "stencil_info: NULL argument");
   const int pi = precision == LSAMD_FP32 ? 1 : 0;
+  if (s->untimed[pi] && !s->zc[pi]) {
+    std::lock_guard<std::recursive_mutex> lock(g_legacy_mu);
+    if (int rc = pi ? ensure_tuned<float>(s, s->p32, s->q32, nullptr)
+                    : ensure_tuned<double>(s, s->p64, s->q64, nullptr))
+      return rc;
+    LSAMD_HIP(hipStreamSynchronize(nullptr));
+  }
   *zc = s->regular ? s->zc[pi] : 0;
   if (tune_us)
     for (int c = 0; c < kNStCand; ++c) tune_us[c] = s->tune_us[pi][c];

@@ -55,3 +55,37 @@ def test_stencil_forms_bit_identical(nn):
         want = N @ x64.cpu().numpy()
         got = _apply(nn, 1016, x64).cpu().numpy()
         assert np.max(np.abs(got - want)) <= 1e-13 * np.max(np.abs(want))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("nn", [(9, 11, 13), (40, 33, 28)])
+def test_info_after_a_solve_of_a_small_grid(monkeypatch, nn, precision):
+    """A Jacobi solve of a small grid takes none of the forms; the report on
+    them is there all the same, timed or pinned, and the operator's bits and
+    the next solve are not touched by it."""
+    from loopstructural_amd import _lib
+    from loopstructural_amd import fd_system as fs
+
+    n = int(np.prod(nn))
+    gen = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.rand(n, dtype=torch.float64, device="cuda", generator=gen) - 0.5
+    want = None
+    for pin in (16, None):
+        if pin:
+            monkeypatch.setenv("LSAMD_STENCIL_ZC", str(pin))
+        s = fs.FdSystem(_lib.make_grid((0, 0, 0), (0.1, 0.1, 0.1), nn),
+                        fs.reg_struct(W, nn, 1e-1))
+        assert s.stencil_info(precision)["zc"] == 0
+        kw = {"rtol": 1e-9, "rhs": x, "precision": precision}
+        c, _ = s.solve(**kw)
+        monkeypatch.delenv("LSAMD_STENCIL_ZC", raising=False)
+        info = s.stencil_info(precision)
+        us = info["candidates_us"]
+        if pin:
+            assert info["zc"] == pin
+        else:
+            assert info["zc"] in FORMS and us[info["zc"]] == min(t for t in us.values() if t > 0)
+        want = s.apply(x) if want is None else want
+        assert torch.equal(s.apply(x), want)
+        assert torch.equal(s.solve(**kw)[0], c)
+        s.close()
