@@ -1678,12 +1678,28 @@ int launch_apply(lsamd_fd_system* s, const T* x, T* y, T* t, CgCtl* ctl, hipStre
   return LSAMD_OK;
 }
 
+// Most data nodes whose term goes by node.  A node's row is some 27 entries, each
+// a gather (three in the PCG direction), where a data point's row is 8: the
+// node form saves launches and, where points share their nodes, work, but at
+// scattered points costs more from some tens of thousands of nodes on.  us per
+// Jacobi iteration in FP64, by node against by row, values at random unless
+// noted: 128^3 nodes 23879 data nodes 56.2, 63.4; 62923 65.2, 64.5; 153814
+// 82.3, 66.8; 363894 119.6, 71.5; 150000 points on 63875 nodes 65.3, 94.6; 93 x
+// 77 x 61 59284 33.5, 34.7; 133160 46.1, 36.9; 150000 points on 405665 87.0,
+// 65.1; 64^3 56415 26.8, 28.8; 118694 39.1, 29.8; 150000 points on 257878 62.9,
+// 53.1; P1 on 129^3 31644 69.1, 72.7; 77861 78.0, 73.9.  (Rows for 363894
+// nodes also take 3 ms to build.)
+int64_t pcg_node_limit(const lsamd_fd_system* s) {
+  return std::min<int64_t>(kGramNodesMax, 50000 + s->nnz / 6);
+}
+
 // Data term by node of the current rows, in FP64 (w64), FP32 (w32) or both,
 // built on the first solve that asks for it after they changed (gram_state).
-// Rows that couple a node with more than kGramCap others, or more than
-// kGramNodesMax data nodes, keep the row form; so do rows whose node rows there
-// is no memory for, as these only save time.
-int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, hipStream_t st) {
+// More data nodes than `most` (pcg_node_limit, mg_node_limit) keep the row form,
+// and so do rows that couple a node with more than kGramCap others, and those
+// whose node rows there is no memory for, as these only save time.
+int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, int64_t most, hipStream_t st) {
+  if (s->ndn > most) return LSAMD_OK;
   int* state = s->gram_state;
   w64 = w64 && !state[0];
   w32 = w32 && !state[1];
@@ -1694,7 +1710,7 @@ int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, hipStream_t st) {
   if (w64) state[0] = 2;
   if (w32) state[1] = 2;
   const int64_t nd = s->ndn, nw = ceil_div(s->n, 64);
-  if (nd > kGramNodesMax || (!(w64 && w32) && other == 2)) return LSAMD_OK;
+  if (!(w64 && w32) && other == 2) return LSAMD_OK;
   // rows of half the width first where one row set's columns suggest it
   // (four-node rows); a longer one costs a second pass
   int width = add ? s->gram_width : s->nnz <= 5 * s->nrows ? kGramCap / 2 : kGramCap;
@@ -1741,10 +1757,10 @@ int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, hipStream_t st) {
   return LSAMD_OK;
 }
 
-GramDev gram_dev(const lsamd_fd_system* s, bool f32) {
+GramDev gram_dev(const lsamd_fd_system* s, bool f32, int64_t most) {
   GramDev G;
   memset(&G, 0, sizeof(G));
-  if (s->gram_state[f32] != 1) return G;
+  if (s->gram_state[f32] != 1 || s->ndn > most) return G;
   G.ndn = s->ndn;
   G.node = s->dnode;
   G.col = s->gram_col;
@@ -1776,7 +1792,7 @@ int launch_iteration(lsamd_fd_system* s, int par, T* x, T* r, T* pa, T* pb, T* q
                      const T* minv, CgCtl* ctl, hipStream_t st) {
   const bool f32 = sizeof(T) == 4;
   const int vb = pcg_blocks(s->n, sizeof(T));
-  const GramDev G = gram_dev(s, f32);
+  const GramDev G = gram_dev(s, f32, pcg_node_limit(s));
   T* gq = (T*)s->gram_q;
   const bool half = s->gram_width == kGramCap / 2;
   const T* po = par ? pb : pa;
@@ -1809,7 +1825,7 @@ int launch_iteration(lsamd_fd_system* s, int par, T* x, T* r, T* pa, T* pb, T* q
     nrow = ng;
   }
   const double* part_g = s->pcg_pg;
-  if (s->nrows > 0 && s->gram_state[f32] != 1) {
+  if (s->nrows > 0 && G.ndn == 0) {
     const RowsDev R = rows_dev(s, f32);
     nrow = (int)ceil_div(s->nrows, 256);
     part_g = s->part_rows;
@@ -2283,12 +2299,25 @@ MgSm mg_sm(const MgLevel& L) {
   return S;
 }
 
+// As pcg_node_limit, for the multigrid solve, whose product gathers one vector.
+// ms per solve, by node against by row: 64^3 nodes 56415 data nodes 14.3, 15.6;
+// 118694 21.1, 21.4; 97 x 89 x 81 60951 22.2, 23.3; 142641 24.7, 24.5; 324970
+// 44.1, 39.9; 128^3 62923 25.8, 26.9; 153814 30.5, 29.1; 396586 40.1, 36.3;
+// 150000 points on 63875 102, 134; 200^3 150000 points on 228129 548, 585.
+int64_t mg_node_limit(const lsamd_fd_system* s) {
+  return std::min<int64_t>(kGramNodesMax, 110000 + s->nnz / 5);
+}
+// the multigrid solve's data term in a precision is applied by node
+bool mg_by_node(const lsamd_fd_system* s, bool f32) {
+  return s->gram_state[f32] == 1 && s->ndn <= mg_node_limit(s);
+}
+
 // y += the data term of x by node, one launch (level 0, where it is built);
 // partials of x.Gx to part where given
 template <typename T>
 void launch_gram_add(const lsamd_fd_system* s, const T* x, T* y, double* part, const CgCtl* ctl,
                      hipStream_t st) {
-  const GramDev G = gram_dev(s, sizeof(T) == 4);
+  const GramDev G = gram_dev(s, sizeof(T) == 4, mg_node_limit(s));
   const dim3 nb((unsigned)ceil_div(G.ndn * kGramLanes, 256));
   if (s->gram_width == kGramCap / 2)
     hipLaunchKernelGGL((k_gram_add<T, kGramCap / 2>), nb, dim3(256), 0, st, G, x, y, part, ctl);
@@ -2303,7 +2332,7 @@ void mg_level_apply(const MgLevel& L, const float* x, float* y, const CgCtl* ctl
   if (L.owned) {
     hipLaunchKernelGGL(k_mg_apply, dim3((unsigned)ceil_div(L.n, 256)), dim3(256), 0, st,
                        mg_dev(L), x, y, ctl);
-  } else if (L.sys->gram_state[1] == 1) {
+  } else if (mg_by_node(L.sys, true)) {
     launch_stencil<float>(L.sys, x, y, ctl, st, L.sys->zc[1]);
     launch_gram_add<float>(L.sys, x, y, nullptr, ctl, st);
   } else {
@@ -2346,7 +2375,7 @@ int mg_level_apply64(const MgLevel& L, const double* x, double* y, hipStream_t s
       hipLaunchKernelGGL(k_mg_apply64<G>, dim3((unsigned)ceil_div(L.n * G, 256)), dim3(256), 0, st,
                          mg_dev<double>(L), x, y);
     });
-  } else if (s->gram_state[0] == 1) {
+  } else if (mg_by_node(s, false)) {
     launch_stencil<double>(s, x, y, s->ctl_apply, st, s->zc[0]);
     launch_gram_add<double>(s, x, y, nullptr, s->ctl_apply, st);
   } else {
@@ -3152,9 +3181,10 @@ int launch_fcg_iteration(lsamd_fd_system* s, hipStream_t st) {
                      (const double*)s->pcg_pr, vb, s->ctl);
   int64_t nq = -1;
   int ng = 0;
-  if (s->gram_state[0] == 1 || s->nrows == 0) {
+  const bool node = mg_by_node(s, false);
+  if (node || s->nrows == 0) {
     nq = launch_stencil<double>(s, (const double*)s->p64, s->q64, s->ctl, st, s->zc[0]);
-    if (s->gram_state[0] == 1) {
+    if (node) {
       launch_gram_add<double>(s, (const double*)s->p64, s->q64, s->pcg_pg, s->ctl, st);
       ng = (int)ceil_div(s->ndn * kGramLanes, 256);
     }
@@ -3246,7 +3276,7 @@ int mg_ensure(lsamd_fd_system* s, hipStream_t st) {
 int mg_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const double* b, double* c,
              lsamd_solve_info* inf, hipStream_t st) {
   if (s->op != 0) return fail(LSAMD_ERR_ARG, "multigrid is available for FD systems only");
-  if (int rc = pcg_gram_ensure(s, true, true, st)) return rc;
+  if (int rc = pcg_gram_ensure(s, true, true, mg_node_limit(s), st)) return rc;
   if (int rc = mg_ensure(s, st)) return rc;
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : 10 * n;
@@ -5164,7 +5194,7 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
       if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
     if (int rc = launch_init<double>(s, b, minv64, s->x64, s->r64, o->rtol, o->atol, maxiter, st))
       return rc;
-    if (int rc = pcg_gram_ensure(s, true, false, st)) return rc;
+    if (int rc = pcg_gram_ensure(s, true, false, pcg_node_limit(s), st)) return rc;
     if (int rc = pcg_buffer(s, &s->pcg_b64)) return rc;
     if (int rc = run_pcg<double>(s, chunk, s->x64, s->r64, s->p64, s->pcg_b64, s->q64, s->t64,
                                  minv64, st))
@@ -5183,7 +5213,7 @@ int lsamd_fd_system_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const d
       if (int rc = ensure_tuned<double>(s, s->p64, s->q64, st)) return rc;
       if (int rc = ensure_tuned<float>(s, s->p32, s->q32, st)) return rc;
     }
-    if (int rc = pcg_gram_ensure(s, false, true, st)) return rc;
+    if (int rc = pcg_gram_ensure(s, false, true, pcg_node_limit(s), st)) return rc;
     if (int rc = pcg_buffer(s, &s->pcg_b32)) return rc;
     const double inner = o->inner_rtol > 0 ? o->inner_rtol : 1e-4;
     const int64_t max_outer = o->max_outer > 0 ? o->max_outer : 50;

@@ -24,8 +24,8 @@ namespace lsamd {
 
 constexpr int kGramCap = 32;       // most entries of a node's Gram row (27 for rows of one cell)
 constexpr int kGramLanes = 8;      // threads per row, two or four entries each
-// larger data terms keep the row form: the rows of this many nodes take 192 MB
-// in FP64, 128 MB in FP32 and 256 MB in both
+// more data nodes keep the row form in any case: the node rows of this many take
+// 192 MB in FP64, 128 MB in FP32 and 256 MB in both
 constexpr int64_t kGramNodesMax = 500000;
 constexpr int kPcgBlocks = 2048;   // partials of the vector kernels
 constexpr int kPcgPartMax = 2048;  // operator partials that every workgroup sums itself

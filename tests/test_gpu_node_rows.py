@@ -70,7 +70,7 @@ def test_solve_without_room_for_them(monkeypatch, precision):
         s = fs.FdSystem(g, reg)
         s.set_rows(_single_node_rows(n, 10))
         s.solve(**kw)
-        s.set_rows(_single_node_rows(n, 100_000))
+        s.set_rows(_single_node_rows(n, 60_000))
         if fail:
             monkeypatch.setenv("LSAMD_FAULT_INJECT", "node_rows")
         taken, (c, info) = _taken(lambda: s.solve(**kw))
@@ -79,7 +79,7 @@ def test_solve_without_room_for_them(monkeypatch, precision):
         fields.append(c)
         assert (taken <= SLACK) == fail, (fail, taken)
         if fail:
-            s.set_rows(_single_node_rows(n, 99_000))
+            s.set_rows(_single_node_rows(n, 59_000))
             taken, (_, info) = _taken(lambda: s.solve(**kw))
             assert info["converged"] and taken > SLACK
         s.close()
@@ -94,7 +94,7 @@ def test_memory_is_that_of_the_width_and_the_precision():
     from loopstructural_amd import fd_system as fs
 
     g, reg, n = _grid()
-    count = 170_000
+    count = 60_000
     col, v64, v32 = (1.25 * 16 * k * count for k in (4, 8, 4))
     per_node = 1.25 * 8 * count + n  # the product's compact result, partials, masks
     fields = []
@@ -116,3 +116,36 @@ def test_memory_is_that_of_the_width_and_the_precision():
         s.close()
     for c in fields[:-1]:
         assert float((c - fields[-1]).norm() / fields[-1].norm()) <= 1e-6
+
+
+@pytest.mark.parametrize("multigrid,count", [(False, 60_000), (False, 60_001), (True, 137_500),
+                                             (True, 137_501)])
+def test_many_data_nodes_take_the_row_form(monkeypatch, multigrid, count):
+    """At and past the limits (50000 + entries / 6 data nodes in the Jacobi
+    solve, 110000 + entries / 5 in multigrid): node rows on one side only, and
+    the iterates of the row form either way.  Nine steps; their rounding differs
+    by the order of the sums: FP64 (2^-53, a few hundred of them) in the Jacobi
+    solve; in multigrid also in the FP32 V-cycle, whose every output may differ by
+    some 2^-24 = 6e-8 of itself, and an iterate by no more than that share of
+    its size for each of the nine directions."""
+    from loopstructural_amd import fd_system as fs
+
+    g, reg, n = _grid()
+    s = fs.FdSystem(g, reg)
+    kw = {"rtol": 0.0, "maxiter": 9, "multigrid": multigrid}
+    s.set_rows(_single_node_rows(n, 10))
+    s.solve(**kw)
+    rows = _single_node_rows(n, count)
+    if multigrid:  # the hierarchy's memory apart
+        s.set_rows(rows)
+        monkeypatch.setenv("LSAMD_FAULT_INJECT", "node_rows")
+        s.solve(**kw)
+        monkeypatch.delenv("LSAMD_FAULT_INJECT")
+    s.set_rows(rows)
+    taken, (c, _) = _taken(lambda: s.solve(**kw))
+    assert (taken > SLACK) == (count % 10 == 0), taken
+    monkeypatch.setenv("LSAMD_FAULT_INJECT", "node_rows")
+    s.set_rows(rows)
+    want, _ = s.solve(**kw)
+    assert float((c - want).norm() / want.norm()) <= (9 * 6e-8 if multigrid else 1e-11)
+    s.close()
