@@ -98,7 +98,8 @@ typedef struct lsamd_solve_opts {
                            multigrid preconditioned flexible CG (FD systems
                            only; FP32 V-cycle with an additive-Schwarz
                            Chebyshev smoother, FP64 outer iteration, the same
-                           Jacobi-scaled stopping test; precision, inner_rtol
+                           Jacobi-scaled stopping test, which has to hold in two
+                           iterations running; precision, inner_rtol
                            and max_outer unused; check_every capped at 8.
                            Environment: LSAMD_MG_SMOOTHER=jacobi for point
                            Jacobi, LSAMD_MG_DEGREE=1..8 for the Chebyshev
