@@ -4474,8 +4474,7 @@ struct Ls {
   double *uw = nullptr, *urid = nullptr, *ud = nullptr, *cw = nullptr;
   double *pu = nullptr, *pv = nullptr, *px = nullptr;  // partials
   int nn = 0, nd = 0, nc = 0;  // workgroups: nodes, data rows, nodes with data rows
-  uint64_t* mask = nullptr;    // nodes with data rows, and their count before each word
-  int32_t* base = nullptr;
+  uint64_t* mask = nullptr;    // nodes with data rows
   LsCtl* ctl = nullptr;  // two slots
   LsEst* est = nullptr;  // two slots
   LsMid* mid = nullptr;
@@ -4520,7 +4519,6 @@ int ls_build(lsamd_fd_system* s, Ls* l) {
   if (int rc = ls_alloc(l, &l->pv, l->nn + l->nc + 1)) return rc;
   if (int rc = ls_alloc(l, &l->px, l->nn + 1)) return rc;
   if (int rc = ls_alloc(l, &l->mask, nw)) return rc;
-  if (int rc = ls_alloc(l, &l->base, nw)) return rc;
   if (int rc = ls_alloc(l, &l->ctl, 2)) return rc;
   if (int rc = ls_alloc(l, &l->est, 2)) return rc;
   if (int rc = ls_alloc(l, &l->mid, 1)) return rc;
@@ -4613,7 +4611,7 @@ int ls_solve(lsamd_fd_system* s, const lsamd_lsmr_opts* o, double* c, lsamd_lsmr
   else
     hipLaunchKernelGGL(k_fill_one, nb, b256, 0, st, l->sv, (float*)nullptr, n);
   hipLaunchKernelGGL(k_pcg_gram_mask, dim3((unsigned)ceil_div(nw, 256)), b256, 0, st,
-                     (const int32_t*)s->dnode, s->ndn, nw, l->mask, l->base);
+                     (const int32_t*)s->dnode, s->ndn, nw, l->mask, (int32_t*)nullptr);
   if (s->nnz > 0)
     hipLaunchKernelGGL(k_ls_coef, dim3((unsigned)ceil_div(s->nnz, 256)), b256, 0, st,
                        rows_dev(s, false), (const double*)s->w, l->cw, s->nnz);

@@ -679,11 +679,16 @@ extern "C" int lsamd_fd_build_rows(const lsamd_grid* g, int32_t kind, double* pt
   return LSAMD_OK;
 }
 
-// Where the table of k_eval_quad is worth a look at the points.  Scattered
-// points without -> with it, us: 1e6 on 80^3 nodes (c fits an L2) 32 -> 42,
-// on 128^3 64 -> 51; 5e6 on 128^3 301 -> 163; 8e6 on 200^3 628 -> 339.  Points in order
-// pay 3 us for the look: of 18 us at 1e6, of 72 us at 5e6, nothing that
-// shows at 1e7.  So: c well past an L2, and points enough that 3 us don't count.
+// Where the table of k_eval_quad is worth a look at the points: c well past an
+// L2 (scattered points on 80^3 nodes, 1e6 of them: 32 us without, 42 with the
+// table), no more nodes than points (200^3 nodes, scattered: 1e6 points 82, 131;
+// 2e6 160, 168; 3e6 238, 196), and so many points that the look, 2.2 us, is
+// little beside them.  The last is a trade: scattered points would gain from
+// 1e6 on, points in order pay the look and gain nothing.  us without and with
+// the table, scattered / in order, on 128^3 nodes: 1e6 64, 51 / 33.8, 35.9 (6%);
+// 2e6 123, 79 / 52.7, 54.9 (4%); 3e6 183, 107 / 69.5, 71.8 (3%); 4e6 242, 136 /
+// 87.0, 89.1 (2.4%).  (The package's _SCRATCH_POINTS saves fewer points than
+// this the call that asks.)
 constexpr int64_t kQuadNodesMin = 1 << 20, kQuadPointsMin = 1 << 22;
 static bool eval_quad_takes(const lsamd_grid* g, int64_t n) {
   const int64_t nn = (int64_t)g->nnodes[0] * g->nnodes[1] * g->nnodes[2];

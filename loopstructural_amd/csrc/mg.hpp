@@ -19,6 +19,10 @@
 // (5000 values, 1000 normals) 97 outer iterations against 63, at 97^3 107
 // against 65, 72 x 69 x 109 with 367 values 85 against 62, 24 x 24 x 36 80
 // against 63, over 48 systems of 32^3..96^3 at most 139 against 101.
+// The ridge is no difference and is not scaled by this rule: it stays halved per
+// level, where P^T P would multiply it by 8.  As it is (64^3 nodes, iterations
+// with both halved, and now): 1e-8 78, 62; 0.01 103, 66; 0.05 113, 88; 0.2 28,
+// 33; 1.0 25, 26.
 // The coarsest level (<= 5 nodes per axis) is solved with a dense inverse.
 // Smoother: Chebyshev polynomial (degree 2 on the fine level, 3 on the
 // coarse ones) in M N on
@@ -838,9 +842,12 @@ __global__ __launch_bounds__(256) void k_mg_smooth(const float* __restrict__ r, 
   x[i] = xv + dv;
 }
 
-constexpr int64_t kSplitMin = 1 << 20;  // levels this large smooth covered nodes apart
-// levels this large keep the compact list of their covered nodes (the
-// multi-rhs smoother splits them, the single-system one from kSplitMin)
+// coarse levels this large keep the product N x in q, as level 0 does, and
+// smooth their covered nodes apart; the smaller ones keep the residual
+constexpr int64_t kSplitMin = 1 << 20;
+// coarse levels this large have a compact list of their covered nodes (level 0
+// always has); the multi-rhs smoother splits the levels of this size, level 0
+// among them, and the single-system and batched ones level 0 at any size
 constexpr int64_t kCovListMin = 1 << 17;
 
 // ------------------------------------------------ Schwarz smoother blocks ----

@@ -94,7 +94,7 @@ __global__ __launch_bounds__(64) void k_pcg_gram_build(RowsDev R, const double* 
   }
 }
 
-// mask and base of the words of 64 nodes (node ids ascending)
+// mask and (where given) base of the words of 64 nodes (node ids ascending)
 __global__ void k_pcg_gram_mask(const int32_t* __restrict__ node, int64_t ndn, int64_t nw,
                                 uint64_t* __restrict__ mask, int32_t* __restrict__ base) {
   const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -107,7 +107,7 @@ __global__ void k_pcg_gram_mask(const int32_t* __restrict__ node, int64_t ndn, i
     else
       hi = mid;
   }
-  base[w] = (int32_t)lo;
+  if (base) base[w] = (int32_t)lo;
   uint64_t b = 0;
   for (; lo < ndn && node[lo] < 64 * w + 64; ++lo) b |= 1ull << (node[lo] - 64 * w);
   mask[w] = b;

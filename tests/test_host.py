@@ -241,3 +241,12 @@ def test_factory_builds_support_from_bounding_box(kind, cls):
                                                   buffer=0.1)
     assert np.allclose(it2.support.maximum - it2.support.origin, 1.2 * (box.maximum - box.origin))
     assert it2.bounding_box is box
+
+
+def test_evaluation_asks_for_scratch_memory_where_some_is_used():
+    """_SCRATCH_POINTS is where the library's own rule begins."""
+    g = _lib.make_grid((0, 0, 0), (1, 1, 1), (128, 128, 64))
+    size = ctypes.c_int64(-1)
+    for n, some in ((fs._SCRATCH_POINTS - 1, False), (fs._SCRATCH_POINTS, True)):
+        _lib.call("lsamd_fd_evaluate_scratch", ctypes.byref(g), n, ctypes.byref(size))
+        assert (size.value > 0) == some, (n, size.value)
