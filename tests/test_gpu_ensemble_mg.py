@@ -94,3 +94,34 @@ def test_batched_multigrid_matches_minimiser(nodes, count):
         assert torch.equal(a, b)
     assert [i["iterations"] for i in infos] == [i["iterations"] for i in infos2]
     bm.close()
+
+
+def test_batched_multigrid_on_large_levels():
+    """Six systems of 64 to 72 nodes per axis, whose first coarse levels hold
+    more than 131072 nodes together (one thread per node there), against the
+    single-system solve.  Both stop at 1e-12 of the right-hand side, where
+    their fields are some 1e-10 from the minimiser."""
+    from loopstructural_amd import _lib, synthetic
+    from loopstructural_amd import fd_system as fs
+
+    ens = synthetic.ensemble(6, 5, nodes=(64, 72), n_values=(800, 1500), n_normals=(100, 200))
+    assert sum(((e[0] + 1) // 2) ** 3 for e in ens) > 131072
+    grids, blocks = [], []
+    for nn, v, m in ens:
+        grids.append(_lib.make_grid((0, 0, 0), (1.0 / (nn - 1),) * 3, (nn,) * 3))
+        blocks.append(_rows(grids[-1], v, m, nn ** 3))
+    reg = fs.reg_struct(W, (64, 64, 64), 1e-8)
+    bm = fs.BatchedMultigrid(grids, reg, workers=4)
+    bm.prepare(blocks)
+    c, infos = bm.solve(blocks, rtol=1e-12)
+    for s, g in enumerate(grids):
+        one = fs.FdSystem(g, reg)
+        one.set_rows(blocks[s])
+        want, info = one.solve(rtol=1e-12, multigrid=True)
+        err = float((c[s] - want).norm() / want.norm())
+        print(f"batched multigrid, {ens[s][0]}^3: {infos[s]['iterations']} iterations, "
+              f"single {info['iterations']}, {err:.1e}", flush=True)
+        assert infos[s]["converged"] and info["converged"] and err <= 1e-8
+        assert infos[s]["iterations"] <= 1.3 * info["iterations"] + 8
+        one.close()
+    bm.close()
