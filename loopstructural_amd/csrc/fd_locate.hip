@@ -512,11 +512,12 @@ __global__ __launch_bounds__(256) void k_eval_quad(GridDev g, EvalGrid e,
 
 // Values and gradients at n points.  A workgroup's points come in, and its
 // gradients leave, through LDS in whole lines (a thread's own three doubles
-// lie 24 bytes from its neighbour's); they are streamed past the caches, whose
-// room belongs to c.  KNOWN: uniform grid with steps that div_known takes.
-// QUAD: corners from the table of k_eval_quad, where that has been filled.
+// lie 24 bytes from its neighbour's).  KNOWN: uniform grid with steps that
+// div_known takes.  QUAD: corners from the table of k_eval_quad, where that has
+// been filled.  STREAM: points and results pass the caches by, whose room belongs
+// to c (see eval_streams).
 constexpr int kEvalBlock = 256;
-template <bool KNOWN, bool QUAD = false>
+template <bool KNOWN, bool QUAD, bool STREAM>
 __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
                                                          const double* __restrict__ c,
                                                          const double* __restrict__ ws,
@@ -528,10 +529,18 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
   const int64_t b = (int64_t)blockIdx.x * kEvalBlock;
   const int m = (int)(n - b < kEvalBlock ? n - b : kEvalBlock);
   const bool quad = QUAD && ws[0] != 0.0;
+  auto put = [](double v, double* p) {
+    if constexpr (STREAM)
+      __builtin_nontemporal_store(v, p);
+    else
+      *p = v;
+  };
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (t + k * kEvalBlock < 3 * m)
-      sh[t + k * kEvalBlock] = __builtin_nontemporal_load(pts + 3 * b + t + k * kEvalBlock);
+      sh[t + k * kEvalBlock] = STREAM
+                                   ? __builtin_nontemporal_load(pts + 3 * b + t + k * kEvalBlock)
+                                   : pts[3 * b + t + k * kEvalBlock];
   __syncthreads();
   double val = 0.0, gr[3] = {0.0, 0.0, 0.0};
   if (t < m) {
@@ -541,7 +550,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
       ok = quad ? eval_point_known<true>(g, e, ws + kQuadHead, px, py, pz, &val, gr)
                 : eval_point_known<false>(g, e, c, px, py, pz, &val, gr);
     if (!ok) eval_point(g, c, px, py, pz, &val, gr);
-    if (vals) __builtin_nontemporal_store(val, vals + b + t);
+    if (vals) put(val, vals + b + t);
   }
   if (!grads) return;
   // a thread overwrites only the three entries that it alone has read
@@ -554,7 +563,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (t + k * kEvalBlock < 3 * m)
-      __builtin_nontemporal_store(sh[t + k * kEvalBlock], grads + 3 * b + t + k * kEvalBlock);
+      put(sh[t + k * kEvalBlock], grads + 3 * b + t + k * kEvalBlock);
 }
 
 // numpy's pairwise summation of a contiguous run of n <= 128 doubles
@@ -697,6 +706,17 @@ static bool eval_quad_takes(const lsamd_grid* g, int64_t n) {
          div_known_divisor(g->step[2]);
 }
 
+// Points and results of an evaluation stay in the 256 MiB last-level cache for
+// the call before or after it, where they fit; where they don't, they only push c
+// out.  us of repeated calls with values and gradients, streamed past the caches
+// against kept: 4e6 points (224 MB) in order on 128^3 nodes 87.1, 73.4, on 70 x
+// 61 x 66 61.9, 49.8; scattered on 32^3 89.8, 74.2, on 128^3 244, 249; 6e6 (336
+// MB) in order on 128^3 124.7, 136.7, scattered 192, 204; 9e6 on 32^3 scattered
+// 198, 210.
+static bool eval_streams(int64_t n, const double* values, const double* grads) {
+  return n * (24 + (values ? 8 : 0) + (grads ? 24 : 0)) > (int64_t)256 << 20;
+}
+
 extern "C" int lsamd_fd_evaluate_scratch(const lsamd_grid* g, int64_t n, int64_t* bytes) {
   if (int rc = check_grid(g)) return rc;
   if (!bytes) return fail(LSAMD_ERR_ARG, "lsamd_fd_evaluate_scratch: NULL output");
@@ -718,18 +738,21 @@ extern "C" int lsamd_fd_evaluate_with(const lsamd_grid* g, const double* c, cons
   const EvalGrid e = to_eval(*g);
   const hipStream_t st = (hipStream_t)stream;
   double* ws = (double*)scratch;
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, nb, bs, 0, st, to_dev(*g), e, c, (const double*)ws, pts, n, values,
+                       grads);
+  };
+  const bool known = !g->axis_nodes[0] && div_known_divisor(g->step[0]) &&
+                     div_known_divisor(g->step[1]) && div_known_divisor(g->step[2]);
+  const bool stream_by = eval_streams(n, values, grads);
   if (ws && eval_quad_takes(g, n)) {
     hipLaunchKernelGGL(k_eval_quad, dim3(kQuadBlocks), dim3(256), 0, st, to_dev(*g), e, c, pts, n,
                        ws);
-    hipLaunchKernelGGL((k_evaluate<true, true>), nb, bs, 0, st, to_dev(*g), e, c, ws, pts, n,
-                       values, grads);
-  } else if (!g->axis_nodes[0] && div_known_divisor(g->step[0]) &&
-             div_known_divisor(g->step[1]) && div_known_divisor(g->step[2])) {
-    hipLaunchKernelGGL(k_evaluate<true>, nb, bs, 0, st, to_dev(*g), e, c, nullptr, pts, n, values,
-                       grads);
+    launch(stream_by ? k_evaluate<true, true, true> : k_evaluate<true, true, false>);
+  } else if (known) {
+    launch(stream_by ? k_evaluate<true, false, true> : k_evaluate<true, false, false>);
   } else {
-    hipLaunchKernelGGL(k_evaluate<false>, nb, bs, 0, st, to_dev(*g), e, c, nullptr, pts, n,
-                       values, grads);
+    launch(stream_by ? k_evaluate<false, false, true> : k_evaluate<false, false, false>);
   }
   LSAMD_CHECK_LAUNCH("k_evaluate");
   return LSAMD_OK;
