@@ -514,8 +514,7 @@ __global__ __launch_bounds__(256) void k_eval_quad(GridDev g, EvalGrid e,
 // gradients leave, through LDS in whole lines (a thread's own three doubles
 // lie 24 bytes from its neighbour's).  KNOWN: uniform grid with steps that
 // div_known takes.  QUAD: corners from the table of k_eval_quad, where that has
-// been filled.  STREAM: points and results pass the caches by, whose room belongs
-// to c (see eval_streams).
+// been filled.  STREAM: points are read past the caches (see eval_streams).
 constexpr int kEvalBlock = 256;
 template <bool KNOWN, bool QUAD, bool STREAM>
 __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
@@ -529,18 +528,10 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
   const int64_t b = (int64_t)blockIdx.x * kEvalBlock;
   const int m = (int)(n - b < kEvalBlock ? n - b : kEvalBlock);
   const bool quad = QUAD && ws[0] != 0.0;
-  auto put = [](double v, double* p) {
-    if constexpr (STREAM)
-      __builtin_nontemporal_store(v, p);
-    else
-      *p = v;
-  };
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (t + k * kEvalBlock < 3 * m)
-      sh[t + k * kEvalBlock] = STREAM
-                                   ? __builtin_nontemporal_load(pts + 3 * b + t + k * kEvalBlock)
-                                   : pts[3 * b + t + k * kEvalBlock];
+      sh[t + k * kEvalBlock] = eval_ld<STREAM>(pts + 3 * b + t + k * kEvalBlock);
   __syncthreads();
   double val = 0.0, gr[3] = {0.0, 0.0, 0.0};
   if (t < m) {
@@ -550,7 +541,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
       ok = quad ? eval_point_known<true>(g, e, ws + kQuadHead, px, py, pz, &val, gr)
                 : eval_point_known<false>(g, e, c, px, py, pz, &val, gr);
     if (!ok) eval_point(g, c, px, py, pz, &val, gr);
-    if (vals) put(val, vals + b + t);
+    if (vals) __builtin_nontemporal_store(val, vals + b + t);
   }
   if (!grads) return;
   // a thread overwrites only the three entries that it alone has read
@@ -563,7 +554,7 @@ __global__ __launch_bounds__(kEvalBlock) void k_evaluate(GridDev g, EvalGrid e,
 #pragma unroll
   for (int k = 0; k < 3; ++k)
     if (t + k * kEvalBlock < 3 * m)
-      put(sh[t + k * kEvalBlock], grads + 3 * b + t + k * kEvalBlock);
+      __builtin_nontemporal_store(sh[t + k * kEvalBlock], grads + 3 * b + t + k * kEvalBlock);
 }
 
 // numpy's pairwise summation of a contiguous run of n <= 128 doubles
@@ -693,28 +684,17 @@ extern "C" int lsamd_fd_build_rows(const lsamd_grid* g, int32_t kind, double* pt
 // table), no more nodes than points (200^3 nodes, scattered: 1e6 points 82, 131;
 // 2e6 160, 168; 3e6 238, 196), and so many points that the look, 2.2 us, is
 // little beside them.  The last is a trade: scattered points would gain from
-// 1e6 on, points in order pay the look and gain nothing.  us without and with
-// the table, scattered / in order, on 128^3 nodes: 1e6 64, 51 / 33.8, 35.9 (6%);
-// 2e6 123, 79 / 52.7, 54.9 (4%); 3e6 183, 107 / 69.5, 71.8 (3%); 4e6 242, 136 /
-// 87.0, 89.1 (2.4%).  (The package's _SCRATCH_POINTS saves fewer points than
-// this the call that asks.)
+// 1e6 on, points in order pay the look and gain nothing.  On 128^3 nodes,
+// scattered without and with the table, and in order: 1e6 64, 51 and 32 us; 2e6
+// 123, 79 and 45; 3e6 183, 107 and 57; 4e6 242, 136 and 70, where the look is 3%.
+// (The package's _SCRATCH_POINTS saves fewer points than this the call that
+// asks.)
 constexpr int64_t kQuadNodesMin = 1 << 20, kQuadPointsMin = 1 << 22;
 static bool eval_quad_takes(const lsamd_grid* g, int64_t n) {
   const int64_t nn = (int64_t)g->nnodes[0] * g->nnodes[1] * g->nnodes[2];
   return nn >= kQuadNodesMin && n >= kQuadPointsMin && n >= nn && !g->axis_nodes[0] &&
          div_known_divisor(g->step[0]) && div_known_divisor(g->step[1]) &&
          div_known_divisor(g->step[2]);
-}
-
-// Points and results of an evaluation stay in the 256 MiB last-level cache for
-// the call before or after it, where they fit; where they don't, they only push c
-// out.  us of repeated calls with values and gradients, streamed past the caches
-// against kept: 4e6 points (224 MB) in order on 128^3 nodes 87.1, 73.4, on 70 x
-// 61 x 66 61.9, 49.8; scattered on 32^3 89.8, 74.2, on 128^3 244, 249; 6e6 (336
-// MB) in order on 128^3 124.7, 136.7, scattered 192, 204; 9e6 on 32^3 scattered
-// 198, 210.
-static bool eval_streams(int64_t n, const double* values, const double* grads) {
-  return n * (24 + (values ? 8 : 0) + (grads ? 24 : 0)) > (int64_t)256 << 20;
 }
 
 extern "C" int lsamd_fd_evaluate_scratch(const lsamd_grid* g, int64_t n, int64_t* bytes) {
@@ -744,15 +724,15 @@ extern "C" int lsamd_fd_evaluate_with(const lsamd_grid* g, const double* c, cons
   };
   const bool known = !g->axis_nodes[0] && div_known_divisor(g->step[0]) &&
                      div_known_divisor(g->step[1]) && div_known_divisor(g->step[2]);
-  const bool stream_by = eval_streams(n, values, grads);
+  const bool past = eval_streams(n, values, grads);
   if (ws && eval_quad_takes(g, n)) {
     hipLaunchKernelGGL(k_eval_quad, dim3(kQuadBlocks), dim3(256), 0, st, to_dev(*g), e, c, pts, n,
                        ws);
-    launch(stream_by ? k_evaluate<true, true, true> : k_evaluate<true, true, false>);
+    launch(past ? k_evaluate<true, true, true> : k_evaluate<true, true, false>);
   } else if (known) {
-    launch(stream_by ? k_evaluate<true, false, true> : k_evaluate<true, false, false>);
+    launch(past ? k_evaluate<true, false, true> : k_evaluate<true, false, false>);
   } else {
-    launch(stream_by ? k_evaluate<false, false, true> : k_evaluate<false, false, false>);
+    launch(past ? k_evaluate<false, false, true> : k_evaluate<false, false, false>);
   }
   LSAMD_CHECK_LAUNCH("k_evaluate");
   return LSAMD_OK;

@@ -136,4 +136,23 @@ __device__ inline double reduce_partials(const double* part, int n, double* sh) 
   return block_sum(v, sh);
 }
 
+// An evaluation writes its results past the caches, whose room belongs to c, and
+// reads its points past them only where points and results are more than the 256
+// MiB last-level cache holds: the points of a smaller call are often still there,
+// from the call that made them or from an evaluation before.  us of repeated
+// calls with values and gradients, points read past the caches against kept: 4e6
+// points in order on 128^3 nodes 87.6, 71.3, on 70 x 61 x 66 62.0, 48.8, P1 on
+// 128^3 91.2, 80.1; scattered on 32^3 89.8, 73.4, P1 91.7, 79.0, on 128^3 241,
+// 244.  Beyond the line, up to the 1.1e7 points whose coordinates alone fit,
+// points in order would gain too (1e7 on 128^3: 187, 143), but scattered ones
+// lose (305, 314).
+inline bool eval_streams(int64_t n, const double* values, const double* grads) {
+  return n * (24 + (values ? 8 : 0) + (grads ? 24 : 0)) > (int64_t)256 << 20;
+}
+template <bool STREAM>
+__device__ inline double eval_ld(const double* p) {
+  if constexpr (STREAM) return __builtin_nontemporal_load(p);
+  return *p;
+}
+
 }  // namespace lsamd

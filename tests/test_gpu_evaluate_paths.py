@@ -167,10 +167,11 @@ def test_coefficients_that_are_not_finite(support, bad):
             assert np.array_equal(kind(got), kind(want)), kind
 
 
+@pytest.mark.parametrize("support", ["fd", "p1"])
 @pytest.mark.parametrize("gi", [0, 4])
-def test_streamed_and_cached_results_are_the_same(gi):
+def test_streamed_and_cached_results_are_the_same(gi, support):
     """One call past the last-level cache (256 MiB of points and results), whose
-    points and results pass it by, against calls that fit; steps that are known
+    points are read past it, against calls that fit; steps that are known
     divisors and one that is none."""
     from loopstructural_amd import fd_system as fs
 
@@ -182,9 +183,10 @@ def test_streamed_and_cached_results_are_the_same(gi):
                                                       generator=gen) * box * 1.01
     c = torch.rand(int(np.prod(np.array(cells) + 1)), dtype=fs.F64, device="cuda", generator=gen)
     grid = _grid(o, cells, h)
-    v, g = fs.evaluate(grid, c, pts, True, True)
+    f = fs.evaluate if support == "fd" else fs.p1_evaluate
+    v, g = f(grid, c, pts, True, True)
     assert 0 < int(torch.isnan(v).sum()) < n
     for part in (slice(0, n // 2), slice(n // 2, n - 1), slice(n - 1, n)):
-        v1, g1 = fs.evaluate(grid, c, pts[part], True, True)
+        v1, g1 = f(grid, c, pts[part], True, True)
         assert torch.equal(v[part].view(torch.int64), v1.view(torch.int64))
         assert torch.equal(g[part].view(torch.int64), g1.view(torch.int64))
