@@ -1277,7 +1277,7 @@ enum RowSlot {
   kRsRowPtr, kRsCols, kRsCoef64, kRsCoef32, kRsB, kRsW, kRsW2_64, kRsW2_32, kRsT64, kRsT32,
   kRsPartRows, kRsURows, kRsBad, kRsErow, kRsKeys, kRsVals, kRsSegEntry, kRsSegRow, kRsUniq,
   kRsCounts, kRsNrun, kRsTmp, kRsOff32, kRsSegPtr, kRsDnode, kRsAdjoint, kRsGramCol,
-  kRsGramV64, kRsGramV32, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart, kRsGramOver, kRsSlots
+  kRsGramV64, kRsGramV32, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart, kRsSlots
 };
 
 template <typename P>
@@ -1688,8 +1688,11 @@ int launch_apply(lsamd_fd_system* s, const T* x, T* y, T* t, CgCtl* ctl, hipStre
 // 77 x 61 59284 33.5, 34.7; 133160 46.1, 36.9; 150000 points on 405665 87.0,
 // 65.1; 64^3 56415 26.8, 28.8; 118694 39.1, 29.8; 150000 points on 257878 62.9,
 // 53.1; P1 on 129^3 31644 69.1, 72.7; 77861 78.0, 73.9.  (Rows for 363894
-// nodes also take 3 ms to build.)
+// nodes also take 3 ms to build.)  A P1 regulariser with weights of its own comes
+// as nine rows per node; by node these cost more to build (1.2 ms) than they
+// gain: a solve on 17^3 nodes 15.4 ms, by row 14.0, on 33^3 55.9, 53.9.
 int64_t pcg_node_limit(const lsamd_fd_system* s) {
+  if (s->op == 1 && s->nrows >= 4 * s->n) return 0;
   return std::min<int64_t>(kGramNodesMax, 50000 + s->nnz / 6);
 }
 
@@ -1714,7 +1717,7 @@ int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, int64_t most, hipStr
   // rows of half the width first where one row set's columns suggest it
   // (four-node rows); a longer one costs a second pass
   int width = add ? s->gram_width : s->nnz <= 5 * s->nrows ? kGramCap / 2 : kGramCap;
-  int* over = nullptr;
+  int* over = (int*)s->part;  // not in use between solves
   double* gq = nullptr;
   for (;;) {
     if (injected("node_rows") || (w64 && rbuf(s, kRsGramV64, &s->gram_v64, nd * width)) ||
@@ -1722,12 +1725,11 @@ int pcg_gram_ensure(lsamd_fd_system* s, bool w64, bool w32, int64_t most, hipStr
         rbuf(s, kRsGramCol, &s->gram_col, nd * width) ||
         rbuf(s, kRsGramMask, &s->gram_mask, nw) || rbuf(s, kRsGramBase, &s->gram_base, nw) ||
         rbuf(s, kRsGramQ, &gq, nd) ||
-        rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB)) ||
-        rbuf(s, kRsGramOver, &over, 2)) {
+        rbuf(s, kRsGramPart, &s->pcg_pg, ceil_div(nd * kGramLanes, VB))) {
       if (w64) rbuf_free(s, kRsGramV64);
       if (w32) rbuf_free(s, kRsGramV32);
       if (!add)
-        for (int k : {kRsGramCol, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart, kRsGramOver})
+        for (int k : {kRsGramCol, kRsGramMask, kRsGramBase, kRsGramQ, kRsGramPart})
           rbuf_free(s, k);
       (void)hipGetLastError();  // the failed allocation's, which the next launch would report
       return LSAMD_OK;

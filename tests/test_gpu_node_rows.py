@@ -149,3 +149,37 @@ def test_many_data_nodes_take_the_row_form(monkeypatch, multigrid, count):
     want, _ = s.solve(**kw)
     assert float((c - want).norm() / want.norm()) <= (9 * 6e-8 if multigrid else 1e-11)
     s.close()
+
+
+def test_rows_of_a_weighted_p1_regulariser_take_none():
+    """Nine rows per node, as a P1 regulariser with weights of its own gives:
+    no memory for node rows; a quarter of the rows has them.  The iterates of
+    the row form either way (FP64, a few hundred terms per sum)."""
+    from loopstructural_amd import _lib
+    from loopstructural_amd import fd_system as fs
+
+    nn = (30, 28, 26)
+    n, dev = int(np.prod(nn)), torch.device("cuda")
+    g = _lib.make_grid((0, 0, 0), tuple(1.0 / (k - 1) for k in nn), nn)
+    gen = torch.Generator(device=dev).manual_seed(1)
+    corner = torch.tensor([i + nn[0] * (j + nn[1] * k) for k in (0, 1) for j in (0, 1)
+                           for i in (0, 1)], device=dev)
+    for m, some in ((9 * n, False), (9 * n // 4, True)):
+        at = torch.arange(m, device=dev) % n
+        one = torch.ones(m, dtype=fs.F64, device=dev)
+        rows = fs.FdRows(torch.arange(m + 1, device=dev) * 8,
+                         (at[:, None] + corner).clamp(max=n - 1).reshape(-1).to(torch.int32),
+                         torch.rand(8 * m, dtype=fs.F64, device=dev, generator=gen) - 0.4,
+                         torch.cos(one.cumsum(0)), one, one.clone(), n)
+        s = fs.P1System(g, 0.1, 1e-2)
+        s.set_rows(_single_node_rows(n, 10))
+        s.solve(rtol=0.0, maxiter=6)
+        s.set_rows(rows)
+        taken, (c, _) = _taken(lambda: s.solve(rtol=0.0, maxiter=6))
+        assert (taken > 5 << 20) == some, taken  # 22e3 x 32 entries x 12 bytes: 8 MiB
+        with pytest.MonkeyPatch.context() as mp:
+            mp.setenv("LSAMD_FAULT_INJECT", "node_rows")
+            s.set_rows(rows)
+            want, _ = s.solve(rtol=0.0, maxiter=6)
+        assert float((c - want).norm() / want.norm()) <= 1e-11
+        s.close()
