@@ -3283,7 +3283,8 @@ int mg_solve(lsamd_fd_system* s, const lsamd_solve_opts* o, const double* b, dou
   const int64_t n = s->n;
   const int64_t maxiter64 = o->maxiter > 0 ? o->maxiter : 10 * n;
   const int maxiter = (int)std::min<int64_t>(maxiter64, 2000000000LL);
-  const int chunk = std::max(1, std::min(o->check_every > 0 ? o->check_every : 8, 8));
+  // no more iterations a launch than may run (as in the Jacobi solve)
+  const int chunk = std::min({o->check_every > 0 ? o->check_every : 8, 8, maxiter});
   if (int rc = launch_init<double>(s, b, s->minv64, s->x64, s->r64, o->rtol, o->atol, maxiter, st))
     return rc;
   hipLaunchKernelGGL(k_mg_to_f32, dim3((unsigned)ceil_div(n, 256)), dim3(256), 0, st,
