@@ -112,49 +112,6 @@ __global__ __launch_bounds__(NT) void k_b_tiles(const T* __restrict__ xg, T* __r
   if (threadIdx.x == 0) part[blockIdx.x] = bs;
 }
 
-// y = R x (+ ridge) for every node of every active system, one node per
-// thread (reference form of k_b_tiles); per-block partials of x.y.
-template <typename T>
-__global__ __launch_bounds__(256) void k_b_stencil(const T* __restrict__ x, T* __restrict__ y,
-                                                   const BSys* __restrict__ sys,
-                                                   const int* __restrict__ blk_sys,
-                                                   const T* __restrict__ tab,
-                                                   double* __restrict__ part,
-                                                   const CgCtl* __restrict__ ctl) {
-  __shared__ double sh[4];
-  const int s = blk_sys[blockIdx.x];
-  if (ctl[s].done) return;
-  const BSys S = sys[s];
-  const int64_t start = (int64_t)(blockIdx.x - S.b0) * kBNodes;
-  const int64_t end = start + kBNodes < S.n ? start + kBNodes : S.n;
-  const int nx = S.g.nx, ny = S.g.ny, nz = S.g.nz;
-  const int64_t nxy = (int64_t)nx * ny;
-  const T* xs = x + S.off;
-  double dot = 0.0;
-  for (int64_t id = start + threadIdx.x; id < end; id += 256) {
-    const int k = (int)(id / nxy);
-    const int64_t rr = id - (int64_t)k * nxy;
-    const int j = (int)(rr / nx);
-    const int i = (int)(rr - (int64_t)j * nx);
-    const T* c = tab + ((cls7(k, nz) * 7 + cls7(j, ny)) * 7 + cls7(i, nx)) * kTaps;
-    const T xc = xs[id];
-    T acc = c[0] * xc;
-#pragma unroll
-    for (int q = 1; q < kTaps; ++q) {
-      const int dx = kBTap[q][0], dy = kBTap[q][1], dz = kBTap[q][2];
-      const bool ok = (unsigned)(i + dx) < (unsigned)nx && (unsigned)(j + dy) < (unsigned)ny &&
-                      (unsigned)(k + dz) < (unsigned)nz;
-      const int64_t o = ok ? id + dx + (int64_t)nx * dy + nxy * dz : id;
-      const T xv = xs[o];
-      acc += c[q] * (ok ? xv : (T)0);
-    }
-    y[S.off + id] = acc;
-    dot += (double)xc * (double)acc;
-  }
-  const double bs = block_sum(dot, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = bs;
-}
-
 __global__ void k_b_diag(const BSys* __restrict__ sys, const int* __restrict__ blk_sys,
                          const double* __restrict__ tab, double* __restrict__ diag) {
   const int s = blk_sys[blockIdx.x];
