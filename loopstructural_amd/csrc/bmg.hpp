@@ -454,8 +454,8 @@ __global__ __launch_bounds__(256) void k_bmg_upd_fin(const BmgSys* __restrict__ 
     c.iter = it;
     c.res2 = tot;
     const int conv = sqrt(tot) < c.thr;
+    c.done = (conv && c.converged) || it >= c.maxiter;  // as k_fcg_upd_fin
     c.converged = conv;
-    c.done = conv || it >= c.maxiter;
   }
 }
 

@@ -40,3 +40,28 @@ def test_residual_and_error_at_the_stop():
         errors.append(float((c - want).norm() / want.norm()))
     assert np.exp(np.mean(np.log(errors))) <= 9.4e-9, errors
     s.close()
+
+
+def test_batched_systems_stop_by_the_same_rule():
+    """The last of the systems to stop has met the test one iteration before."""
+    from loopstructural_amd import _lib, synthetic
+    from loopstructural_amd import fd_system as fs
+
+    grids, blocks = [], []
+    for nodes, seed in ((20, 1), (24, 2), (31, 3)):
+        g = _lib.make_grid((0, 0, 0), (1.0 / (nodes - 1),) * 3, (nodes,) * 3)
+        p = torch.from_numpy(synthetic.constraints(300, 10, seed)[0]).cuda()
+        grids.append(g)
+        blocks.append(fs.concat_rows([fs.build_rows(g, _lib.ROWS_VALUE, p, 4, 1.0, nodes ** 3)],
+                                     nodes ** 3))
+    bm = fs.BatchedMultigrid(grids, fs.reg_struct(W, (20, 20, 20), 1e-8), workers=2)
+    bm.prepare(blocks)
+    _, infos = bm.solve(blocks, rtol=1e-10)
+    last = max(range(3), key=lambda s: infos[s]["iterations"])
+    it = infos[last]["iterations"]
+    for maxiter, met in ((it - 1, True), (it - 2, False)):
+        _, early = bm.solve(blocks, rtol=1e-10, maxiter=maxiter)
+        assert early[last]["converged"] == met
+        assert (early[last]["residual"] < early[last]["threshold"]) == met
+    assert all(i["converged"] and i["residual"] < i["threshold"] for i in infos)
+    bm.close()
