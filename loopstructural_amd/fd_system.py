@@ -193,8 +193,8 @@ class FdSystem:
         """PCG on N c = rhs.  jacobi: the reference's column scaling as the
         preconditioner (False: plain CG).  multigrid: geometric-multigrid
         preconditioned flexible CG (FP32 V-cycle, FP64 outer iteration; FD
-        systems only); same stopping test, same minimiser, far fewer
-        iterations."""
+        systems only); same stopping test, held in two iterations running,
+        same minimiser, far fewer iterations."""
         o = _lib.SolveOpts()
         o.rtol = float(rtol)
         o.atol = float(atol)

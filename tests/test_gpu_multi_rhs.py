@@ -92,7 +92,7 @@ def test_multi_rhs_at_128_cubed():
     single-system multigrid solve of each (1e-9); the multi-rhs solve takes
     at most one captured chunk of 8 iterations more (its outer iteration
     keeps direction and residual in FP32, the residual replaced every 8
-    iterations; its coarse levels smooth with degree 6 against 4)."""
+    iterations; its coarse levels smooth with degree 4 against 3)."""
     s, rhs, reals, g, n = _setup(127, 4)
     print("multi-rhs at 128^3: solving 4 lanes", flush=True)
     c, infos = s.solve_multi(rhs, rtol=1e-12)
